@@ -16,6 +16,7 @@
 // previous X.  The preconditioner only steers the Krylov iterations: the
 // solve still stops on the true FP64 residual.
 #include "coarse.hpp"
+#include "win.hpp"
 
 #include <rocblas/rocblas.h>
 
@@ -45,9 +46,8 @@ __device__ inline int agg_of(uint32_t key, const AggGrid& g) {
   return cx / kAgg + g.AX * (cy / kAgg + g.AY * (cz / kAgg));
 }
 
-// Column indices of the four entries of quad q of row i (kFmtRun8: run bases
-// from the row's cell key and run lengths, as in the matvec decoder; entries
-// past cnt get the row's own index and a zero coefficient from the caller).
+// Run bases of row i (kFmtRun8) from its cell key and run lengths, as in the
+// matvec decoder.
 struct RunDecode {
   int B[9], E[8];
 };
@@ -97,7 +97,6 @@ __global__ __launch_bounds__(256) void k_coarse_rows(PpeOp o, AggGrid g, double*
     for (int q = 0; q < nq; q++) {
       const size_t qi = (size_t)q * n + (size_t)i;
       double c[4];
-      uint32_t hb[4] = {0u, 0u, 0u, 0u};  // mixed: hi words, kFmtRun8 offset in the low byte
       if (CM == 2) {
         const double2 a = reinterpret_cast<const double2*>(o.c64)[2 * qi];
         const double2 b = reinterpret_cast<const double2*>(o.c64)[2 * qi + 1];
@@ -105,20 +104,19 @@ __global__ __launch_bounds__(256) void k_coarse_rows(PpeOp o, AggGrid g, double*
       } else {
         const uint4 a = reinterpret_cast<const uint4*>(o.hi)[qi];
         const float4 b = reinterpret_cast<const float4*>(o.lo)[qi];
-        hb[0] = a.x; hb[1] = a.y; hb[2] = a.z; hb[3] = a.w;
-        c[0] = (double)hi_val(hb[0]) + (double)b.x; c[1] = (double)hi_val(hb[1]) + (double)b.y;
-        c[2] = (double)hi_val(hb[2]) + (double)b.z; c[3] = (double)hi_val(hb[3]) + (double)b.w;
+        c[0] = (double)hi_val(a.x) + (double)b.x; c[1] = (double)hi_val(a.y) + (double)b.y;
+        c[2] = (double)hi_val(a.z) + (double)b.z; c[3] = (double)hi_val(a.w) + (double)b.w;
       }
       int j[4];
       if (FMT == kFmtRun8) {
-        const uint32_t w = CM == 2 ? o.idx[qi] : 0u;
+        const uint32_t w = o.idx[qi];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           const int k = 4 * q + u;
           int base = d.B[0];
 #pragma unroll
           for (int r = 0; r < 8; r++) base = k >= d.E[r] ? d.B[r + 1] : base;
-          const uint32_t off = CM == 2 ? (w >> (8 * u)) & 255u : hb[u] & 255u;
+          const uint32_t off = (w >> (8 * u)) & 255u;
           j[u] = k < cnt ? base + (int)off : i;
         }
       } else {
@@ -142,6 +140,63 @@ __global__ __launch_bounds__(256) void k_coarse_rows(PpeOp o, AggGrid g, double*
   }
 #pragma unroll
   for (int t = 0; t < 8; t++) slots[(size_t)t * n + i] = acc[t];
+}
+
+// Pass 1 of the window format (kFmtWin): the tile's cells are staged in LDS as
+// in the matvec, each slot holding the parities of its cell's aggregate
+// coordinates.  Aggregates that couple differ by at most one per axis, so the
+// exclusive or with the row's own parities is the slot sum's index: one byte
+// from LDS per entry in place of a key gather and three divisions.
+__device__ inline uint8_t agg_parity(int x, int y, int z) {
+  return (uint8_t)(((x / kAgg) & 1) | (((y / kAgg) & 1) << 1) | (((z / kAgg) & 1) << 2));
+}
+__global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, double* __restrict__ slots) {
+  __shared__ WinStage<uint8_t> S;
+  const int n = o.n;
+  const int b = (gridDim.x & 7) ? (int)blockIdx.x : (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3));
+  const int i0 = b * kWinThreads, i1 = min(i0 + kWinThreads, n);
+  for (int s0 = i0; s0 < i1;) {
+    int e0;
+    const int m = win_stage(
+        o, s0, i1, S, &e0, [](int x, int y, int z, int) { return (int)agg_parity(x, y, z); },
+        [](int par, int) { return (uint8_t)par; });
+    const int i = s0 + (int)threadIdx.x;
+    s0 = m;
+    if (i >= m) continue;
+    double acc[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) acc[t] = 0.0;
+    if (o.row[i]) {
+      const uint32_t key = o.keys[i];
+      int cx, cy, cz;
+      cell_xyz(key, o.NI, o.NJ, cx, cy, cz);
+      const uint8_t own = agg_parity(cx, cy, cz);
+      const uint8_t* win = S.x + S.p.pre[9 * (win_ekey(o, key) - e0)];
+      acc[0] = o.diag[i];
+      const int meta = o.ccnt[i];
+      const int nq = ((meta & 0xFFFF) + 3) >> 2, anc = (meta >> 16) << 23;
+      const uint4* hp = reinterpret_cast<const uint4*>(o.hi) + i;
+      const float4* lp = reinterpret_cast<const float4*>(o.lo) + i;
+      uint4 w = nq > 0 ? hp[0] : make_uint4(0u, 0u, 0u, 0u);
+      float4 l = nq > 0 ? lp[0] : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int q = 0; q < nq; q++) {
+        const uint32_t c[4] = {w.x, w.y, w.z, w.w};
+        const float lv[4] = {l.x, l.y, l.z, l.w};
+        const size_t qn = (size_t)min(q + 1, nq - 1) * n;
+        w = hp[qn];
+        l = lp[qn];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int sl = (int)(win[c[u] & (uint32_t)kWinMax] ^ own);
+          const double a = (double)win_val(c[u], anc) + (double)lv[u];  // 0 for padding entries
+#pragma unroll
+          for (int t = 0; t < 8; t++) acc[t] -= sl == t ? a : 0.0;
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 8; t++) slots[(size_t)t * n + i] = acc[t];
+  }
 }
 
 // Pass 2, one wave per aggregate I: for each of its cells (fixed order) the
@@ -445,9 +500,10 @@ static int coarse_rows(hipStream_t s, CoarseWork& c, const PpeWork& w) {
   const PpeOp o = ppe_op(w);
   const AggGrid g = agg_grid(c);
   const int gr = grid_xcd(w.n);
-  if (w.fmt == kFmtRun8) {
-    if (w.mixed) k_coarse_rows<kFmtRun8, 1><<<gr, 256, 0, s>>>(o, g, c.slots);
-    else k_coarse_rows<kFmtRun8, 2><<<gr, 256, 0, s>>>(o, g, c.slots);
+  if (w.fmt == kFmtWin) {
+    k_coarse_rows_win<<<gr, kWinThreads, 0, s>>>(o, c.slots);
+  } else if (w.fmt == kFmtRun8) {
+    k_coarse_rows<kFmtRun8, 2><<<gr, 256, 0, s>>>(o, g, c.slots);
   } else {
     if (w.mixed) k_coarse_rows<kFmtIdx32, 1><<<gr, 256, 0, s>>>(o, g, c.slots);
     else k_coarse_rows<kFmtIdx32, 2><<<gr, 256, 0, s>>>(o, g, c.slots);

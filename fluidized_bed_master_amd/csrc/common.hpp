@@ -144,12 +144,13 @@ struct alignas(32) Rec32 {
   float aux;
 };
 // PPE assembly (mixed path): V = m/rho, eps, eps rho and p in FP64 with the
-// FP32 velocity; flags = p_type (low 16 bits) | i_type << 16 | row << 24.
+// FP32 velocity; flags = the cell's coordinates (ten bits per axis) | PPE row
+// << 30 | counted by the pair sums << 31.
 struct alignas(64) RecAsm {
   float4 p;  // pos4
   double vol, por, porrho, pres;
   float ux, uy, uz;
-  int flags;
+  uint32_t flags;
 };
 
 // Advection's neighbour records on the mixed path, after pk = {x, y, z, m}:

@@ -14,12 +14,14 @@
 // buffers -- keep their lagged pressures, as in the reference).
 //
 // Operator storage (PpeOp): only row columns are kept, compacted per row,
-// slot-quad major.  Columns are u8 offsets inside the 9 x-runs of the
-// 27-cell stencil (kFmtRun8) or u32 indices (kFmtIdx32).
-//   FP64 path : a_ij as double                        (8 B + 1 B per entry)
-//   mixed path: hi = fl32(a), lo = fl32(a - hi)
-//               inner FP32 iterations read hi only    (4 B + 1 B per entry)
-//               FP64 residuals read hi + lo (48-bit a)
+// slot-quad major.
+//   FP64 path : a_ij as double and a u8 offset inside the 9 x-runs of the
+//               27-cell stencil (kFmtRun8)            (8 B + 1 B per entry)
+//   mixed path: hi = a at a 16-bit significand with an 11-bit slot in the
+//               row's 27-cell window in the same word (kFmtWin), lo = fl32(a - hi)
+//               inner FP32 iterations read hi only    (4 B per entry)
+//               FP64 residuals read hi + lo (40-bit a)
+// or u32 column indices beside the coefficients (kFmtIdx32).
 //
 // Solver: BiCGStab (van der Vorst 1992) with Jacobi right preconditioning.
 // The mixed path runs the recurrences on FP32 vectors with the hi operator
@@ -34,6 +36,7 @@
 #include "nbr.hpp"
 
 #include "coarse.hpp"
+#include "win.hpp"
 
 #include <cstring>
 #include <type_traits>
@@ -135,38 +138,29 @@ __device__ void sum_partials(const double* partials, int G, double (&tot)[NV]) {
 
 // ----- row sums over the compact operator ----------------------------------
 // CM: 0 = hi (FP32 accumulation), 1 = hi + lo (FP64), 2 = FP64 coefficients.
-// For CM 0 and 1, b holds the raw hi words: their low byte is the kFmtRun8
-// column offset.
 template <int CM>
 struct CoefQuad;
 template <>
 struct CoefQuad<0> {
   float c[4];
-  uint32_t b[4];
   __device__ void load(const PpeOp& o, size_t qi) {
     const uint4 a = reinterpret_cast<const uint4*>(o.hi)[qi];
-    b[0] = a.x; b[1] = a.y; b[2] = a.z; b[3] = a.w;
-#pragma unroll
-    for (int u = 0; u < 4; u++) c[u] = hi_val(b[u]);
+    c[0] = hi_val(a.x); c[1] = hi_val(a.y); c[2] = hi_val(a.z); c[3] = hi_val(a.w);
   }
 };
 template <>
 struct CoefQuad<1> {
   double c[4];
-  uint32_t b[4];
   __device__ void load(const PpeOp& o, size_t qi) {
     const uint4 a = reinterpret_cast<const uint4*>(o.hi)[qi];
     const float4 l = reinterpret_cast<const float4*>(o.lo)[qi];
-    b[0] = a.x; b[1] = a.y; b[2] = a.z; b[3] = a.w;
-    const float lv[4] = {l.x, l.y, l.z, l.w};
-#pragma unroll
-    for (int u = 0; u < 4; u++) c[u] = (double)hi_val(b[u]) + (double)lv[u];
+    c[0] = (double)hi_val(a.x) + (double)l.x; c[1] = (double)hi_val(a.y) + (double)l.y;
+    c[2] = (double)hi_val(a.z) + (double)l.z; c[3] = (double)hi_val(a.w) + (double)l.w;
   }
 };
 template <>
 struct CoefQuad<2> {
   double c[4];
-  uint32_t b[4];  // unused: the FP64 path keeps its offsets in idx
   __device__ void load(const PpeOp& o, size_t qi) {
     double2 a = reinterpret_cast<const double2*>(o.c64)[2 * qi];
     double2 e = reinterpret_cast<const double2*>(o.c64)[2 * qi + 1];
@@ -217,10 +211,8 @@ __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restric
       if (r < 8) E[r] = acc;
     }
     const int self = STAGED ? i + adj[4] : i;
-    // mixed operator: the offsets ride in the coefficient words; FP64: idx
-    constexpr bool PK = CM < 2;
     const size_t q1 = (size_t)min(1, last) * n + i;
-    uint32_t wn0 = PK ? 0u : o.idx[i], wn1 = PK ? 0u : o.idx[q1];
+    uint32_t wn0 = o.idx[i], wn1 = o.idx[q1];
     CoefQuad<CM> cn0, cn1;
     cn0.load(o, (size_t)i);
     cn1.load(o, q1);
@@ -234,9 +226,7 @@ __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restric
         int base = B[0];
 #pragma unroll
         for (int r = 0; r < 8; r++) base = k >= E[r] ? B[r + 1] : base;
-        uint32_t off;
-        if constexpr (PK) off = (u < 4 ? c0.b[u & 3] : c1.b[u & 3]) & 255u;
-        else off = ((u < 4 ? w0 : w1) >> (8 * (u & 3))) & 255u;
+        const uint32_t off = ((u < 4 ? w0 : w1) >> (8 * (u & 3))) & 255u;
         j[u] = k < cnt ? base + (int)off : self;
       }
       XT xv[8];
@@ -244,10 +234,8 @@ __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restric
       for (int u = 0; u < 8; u++) xv[u] = x[j[u]];
       const size_t qa = (size_t)min(q + 2, last) * n + i;
       const size_t qb = (size_t)min(q + 3, last) * n + i;
-      if constexpr (!PK) {
-        wn0 = o.idx[qa];
-        wn1 = o.idx[qb];
-      }
+      wn0 = o.idx[qa];
+      wn1 = o.idx[qb];
       cn0.load(o, qa);
       cn1.load(o, qb);
 #pragma unroll
@@ -286,7 +274,7 @@ __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restric
 
 // ----- assembly ---------------------------------------------------------------
 struct AsmOut {
-  int n, NI, NJ, NK;
+  int n, NI, NJ, NK, pmask, ncell;
   const uint32_t* keys;
   const uint32_t* cell_off;
   const int* row;
@@ -300,6 +288,38 @@ struct AsmOut {
   unsigned* flags;
 };
 
+// Window slots of one row's neighbours (kFmtWin) from the tile's plan: D of the
+// cell at (dx, dy, dz) of the row's cell maps a particle index to its staged
+// slot, and base is the window's first slot.
+struct WinSlots {
+  const int* D;  // plan entry of the row's cell (x - 1, y - 1, z - 1)
+  int base, total;
+  int cx, cy, cz;
+};
+// -1, 0 or 1 from a cell coordinate difference known modulo 1024 (the records
+// keep ten bits): the images across a period of N cells are N - 1 away
+__device__ inline int win_step(int d, bool periodic, int N) {
+  d &= 1023;
+  if (d == 0) return 0;
+  if (d == 1) return 1;
+  if (d == 1023) return -1;
+  if (periodic && d == ((N - 1) & 1023)) return -1;
+  return 1;
+}
+__device__ inline uint32_t cell_bits(int cx, int cy, int cz) {
+  return (uint32_t)(cx & 1023) | (uint32_t)(cy & 1023) << 10 | (uint32_t)(cz & 1023) << 20;
+}
+__device__ inline uint32_t cell_bits_of(const AsmOut& o, uint32_t key) {
+  const int cx = (int)(key % (uint32_t)o.NI), t = (int)(key / (uint32_t)o.NI);
+  return cell_bits(cx, t % o.NJ, t / o.NJ);
+}
+__device__ inline int win_slot(const AsmOut& o, const WinSlots& w, uint32_t cell, int j) {
+  const int dx = win_step((int)(cell & 1023u) - w.cx, o.pmask & 1, o.NI);
+  const int dy = win_step((int)((cell >> 10) & 1023u) - w.cy, o.pmask & 2, o.NJ);
+  const int dz = win_step((int)((cell >> 20) & 1023u) - w.cz, o.pmask & 4, o.NK);
+  return j + w.D[9 * (dx + 1) + 3 * (dz + 1) + dy + 1] - w.base;
+}
+
 __device__ inline int pick9(const int (&a)[9], int r) {
   int v = a[0];
 #pragma unroll
@@ -307,17 +327,68 @@ __device__ inline int pick9(const int (&a)[9], int r) {
   return v;
 }
 
-__global__ void k_rowmask(DevParams P, int n, const int* ptype, const int* btype, const int* itype, const int* surf,
-                          double* pres, int* row) {
-  int i = particle_index();
-  if (i >= n) return;
-  int t = ptype[i];
-  const bool fluid = itype[i] <= 2 && !(P.open_boundary > 0 && btype[i] > 0) && t < 1000 && t > 0;
-  const bool dirichlet = fluid && P.free_surface > 0 && surf[i] != 0;
-  // a free-surface particle is a known value p_ref, not an unknown
-  if (dirichlet) pres[i] = P.p_ref;
-  bool on = fluid && !dirichlet;
-  row[i] = on ? 1 : 0;
+// The row mask and the Dirichlet pressures.  peak (mixed path): per block the
+// largest |eps rho| and |m / rho| of its particles, from which the assembly
+// bounds a row's coefficients.
+__global__ __launch_bounds__(kBlock) void k_rowmask(DevParams P, int n, const int* ptype, const int* btype,
+                                                    const int* itype, const int* surf, const double* m,
+                                                    const double* rho, const double* por, double* pres, int* row,
+                                                    float2* peak) {
+  __shared__ float2 red[kBlock / 64];
+  float pr = 0.f, vol = 0.f;
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    const int t = ptype[i];
+    const bool fluid = itype[i] <= 2 && !(P.open_boundary > 0 && btype[i] > 0) && t < 1000 && t > 0;
+    const bool dirichlet = fluid && P.free_surface > 0 && surf[i] != 0;
+    // a free-surface particle is a known value p_ref, not an unknown
+    if (dirichlet) pres[i] = P.p_ref;
+    row[i] = fluid && !dirichlet ? 1 : 0;
+    if (peak) {
+      pr = fmaxf(pr, (float)fabs(por[i] * rho[i]));
+      vol = fmaxf(vol, (float)fabs(m[i] / rho[i]));
+    }
+  }
+  if (!peak) return;
+  for (int off = 32; off > 0; off >>= 1) {
+    pr = fmaxf(pr, __shfl_xor(pr, off));
+    vol = fmaxf(vol, __shfl_xor(vol, off));
+  }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(pr, vol);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kBlock / 64; w++) {
+      pr = fmaxf(pr, red[w].x);
+      vol = fmaxf(vol, red[w].y);
+    }
+    peak[blockIdx.x] = make_float2(pr, vol);
+  }
+}
+
+// one block: clears the assembly's flags and leaves the two peaks (FP32 bits)
+// behind them.  (An atomic maximum from each wave of k_rowmask in place of the
+// partials took 141 us at 1.16 M particles.)
+__global__ __launch_bounds__(kBlock) void k_asm_begin(const float2* peak, int G, unsigned* flags) {
+  __shared__ float2 red[kBlock / 64];
+  float pr = 0.f, vol = 0.f;
+  for (int b = threadIdx.x; b < G; b += kBlock) {
+    pr = fmaxf(pr, peak[b].x);
+    vol = fmaxf(vol, peak[b].y);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    pr = fmaxf(pr, __shfl_xor(pr, off));
+    vol = fmaxf(vol, __shfl_xor(vol, off));
+  }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(pr, vol);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kBlock / 64; w++) {
+      pr = fmaxf(pr, red[w].x);
+      vol = fmaxf(vol, red[w].y);
+    }
+    flags[0] = flags[1] = 0u;
+    flags[2] = __float_as_uint(pr);
+    flags[3] = __float_as_uint(vol);
+  }
 }
 
 __global__ void k_cell_offsets(int n, const uint32_t* __restrict__ keys, int nc, uint32_t* __restrict__ off) {
@@ -334,7 +405,8 @@ __global__ void k_cell_offsets(int n, const uint32_t* __restrict__ keys, int nc,
 
 // The assembly's 64 B neighbour records (mixed path), after the row mask
 // and the Dirichlet pressures are set
-__global__ void k_pack_asm(SphView<float> v, const int* __restrict__ row) {
+__global__ void k_pack_asm(SphView<float> v, const int* __restrict__ row, const uint32_t* __restrict__ keys, int NI,
+                           int NJ) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= v.n) return;
   RecAsm r;
@@ -347,15 +419,18 @@ __global__ void k_pack_asm(SphView<float> v, const int* __restrict__ row) {
   r.ux = v.ux[i];
   r.uy = v.uy[i];
   r.uz = v.uz[i];
-  const int pt = min(max(v.ptype[i], -32768), 32767);
-  r.flags = (pt & 0xFFFF) | ((v.itype[i] & 0xFF) << 16) | ((row[i] ? 1 : 0) << 24);
+  // the cell's ten bits per axis, the PPE row mark and whether the pair sums
+  // count the particle (p_type < 1000, i_type != 4)
+  const uint32_t key = keys[i];
+  const int cx = (int)(key % (uint32_t)NI), t = (int)(key / (uint32_t)NI);
+  r.flags = cell_bits(cx, t % NJ, t / NJ) | (row[i] ? 1u << 30 : 0u) |
+            (v.ptype[i] < 1000 && v.itype[i] != 4 ? 1u << 31 : 0u);
   v.ra[i] = r;
 }
 
 template <typename R, int FMT, int MIXED>
-__global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, AsmOut o) {
-  int i = particle_index();
-  if (i >= v.n) return;
+__device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R>& v, const AsmOut& o, int i,
+                                             const WinSlots& ww) {
   const int n = v.n;
   const size_t nn = (size_t)n;
   const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
@@ -397,6 +472,27 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
   const float4 pi4 = REL ? v.pos4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   const double uxi = v.ux[i], uyi = v.uy[i], uzi = v.uz[i];
   const double rhoi = v.rho[i], pori = v.por[i], irhoi = 1.0 / rhoi;
+  int anchor = 0;
+  if (FMT == kFmtWin) {
+    // a bound of the row's coefficients: the largest eps_j rho_j and V_j of any
+    // particle, and |Cm| |W'(r) / r| at r -> 0
+    const double r0 = 0.01 * hd;
+    double cmn = 1.0;
+    if (P.kgc > 0) {
+      double c2 = 0;
+#pragma unroll
+      for (int c = 0; c < 6; c++) {
+        const double e = v.cm[(size_t)c * n + i];
+        c2 += ((c == 0 || c == 3 || c == 5) ? 1.0 : 2.0) * e * e;
+      }
+      cmn = sqrt(c2);
+    }
+    const double bound = (fabs(pori * rhoi) + (double)__uint_as_float(o.flags[2])) *
+                         (double)__uint_as_float(o.flags[3]) * fabs(irhoi) * cmn *
+                         fabs(knl_dw_ih<double>(P.kernel_type, A, hd, ihd, r0)) / r0;
+    const int top = (int)((__float_as_uint((float)bound) >> 23) & 255u);
+    anchor = min(max(top + 1 - 31, 1), 223);
+  }
   double bx = 0, by = 0, bz = 0, Aij = 0, AP = 0, lag = 0;
   double dcomp = 0;  // sum over stored columns of a - hi16(a) (mixed)
   int kc = 0, run = 0;
@@ -438,7 +534,8 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
     GT x, y, z;  // x_i - x_j
     double vol, por, porrho, pres;  // V_j = m_j / rho_j, eps_j, eps_j rho_j, p_j
     R ux, uy, uz;
-    int pt, it, row;
+    bool use, row;  // p_type < 1000 and i_type != 4; a PPE row
+    int slot;       // kFmtWin: its slot in the row's window
   };
   const int last4 = (cnt - 1) & ~3;
   uint4 en4 = cnt > 0 ? *(const uint4*)(v.nbr + nbr_slot(0, i, (int)n)) : make_uint4(0u, 0u, 0u, 0u);
@@ -457,13 +554,15 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
         nb[u].x = d.x; nb[u].y = d.y; nb[u].z = d.z;
         nb[u].vol = ra.vol; nb[u].por = ra.por; nb[u].porrho = ra.porrho; nb[u].pres = ra.pres;
         nb[u].ux = ra.ux; nb[u].uy = ra.uy; nb[u].uz = ra.uz;
-        nb[u].pt = (int)(int16_t)(ra.flags & 0xFFFF); nb[u].it = (ra.flags >> 16) & 0xFF; nb[u].row = ra.flags >> 24;
+        nb[u].use = (ra.flags >> 31) != 0; nb[u].row = ((ra.flags >> 30) & 1u) != 0;
+        nb[u].slot = FMT == kFmtWin ? win_slot(o, ww, ra.flags, j) : 0;
       } else {
         pdiff(v, xi, yi, zi, j, nb[u].x, nb[u].y, nb[u].z);
         const double mj = v.m[j], rhoj = v.rho[j], porj = v.por[j];
         nb[u].vol = mj / rhoj; nb[u].por = porj; nb[u].porrho = porj * rhoj; nb[u].pres = v.pres[j];
         nb[u].ux = v.ux[j]; nb[u].uy = v.uy[j]; nb[u].uz = v.uz[j];
-        nb[u].pt = v.ptype[j]; nb[u].it = v.itype[j]; nb[u].row = o.row[j];
+        nb[u].use = v.ptype[j] < 1000 && v.itype[j] != 4; nb[u].row = o.row[j] != 0;
+        nb[u].slot = FMT == kFmtWin ? win_slot(o, ww, cell_bits_of(o, o.keys[j]), j) : 0;
       }
     }
     en4 = *(const uint4*)(v.nbr + nbr_slot(min(k0 + 4, last4), i, (int)n));
@@ -474,7 +573,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
     const int j = (int)(e & ~kNbrFlag);
     const AsmNb& nq = nb[ub];
     if (e & kNbrFlag) continue;
-    if (!(nq.pt < 1000 && nq.it != 4)) continue;
+    if (!nq.use) continue;
     double dx = nq.x, dy = nq.y, dz = nq.z;
     double r = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
     // two reciprocals per pair (1/r, V_j = m_j / rho_j) in place of the
@@ -519,11 +618,16 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
         }
       }
     }
-    if (MIXED) {
+    if (FMT == kFmtWin) {
+      const uint32_t w = win_word(a, anchor, (uint32_t)nq.slot & (uint32_t)kWinMax);
+      const double hv = (double)win_val(w, anchor << 23);
+      dcomp += a - hv;
+      push_quad(0u, w, (float)(a - hv), a);
+    } else if (MIXED) {
       const uint32_t hb = hi16_bits(a);
       const double hv = (double)hi_val(hb);
       dcomp += a - hv;
-      push_quad((uint32_t)j, hb | off8, (float)(a - hv), a);
+      push_quad((uint32_t)j, hb, (float)(a - hv), a);
     } else {
       push_quad((uint32_t)j, 0u, 0.f, a);
     }
@@ -534,12 +638,24 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
   // pad the last quad so whole-quad loads read defined values
   if (kc & 3) {
     const int q = kc >> 2;
-    for (int u = kc & 3; u < 4; u++) push_quad((uint32_t)i, 0u, 0.f, 0.0);
+    if (FMT == kFmtWin) {
+      // the least value of the row's range on the row's own column, taken up
+      // by the diagonal like a rounding: the row sums need no masks
+      const uint32_t self = (uint32_t)(i + ww.D[13] - ww.base) & (uint32_t)kWinMax;
+      const uint32_t w = win_word(0.0, anchor, self);
+      const float t = win_val(w, anchor << 23);
+      for (int u = kc & 3; u < 4; u++) {
+        dcomp -= (double)t;
+        push_quad(0u, w, -t, 0.0);
+      }
+    } else {
+      for (int u = kc & 3; u < 4; u++) push_quad((uint32_t)i, 0u, 0.f, 0.0);
+    }
     store_quad(q);
     if (FMT == kFmtRun8 && !MIXED) o.idx[(size_t)q * nn + i] = word;
   }
   if (bad) atomicOr(o.flags, bad);
-  o.ccnt[i] = kc;
+  o.ccnt[i] = FMT == kFmtWin ? kc | (anchor << 16) : kc;
   o.runc[i] = rcw;
   const double tdt = P.dt_sph;
   const double bi = P.rho_fluid * (bx + by + bz + 2 * (double)v.dpor[i] - (double)v.dpor_prev[i]) / tdt;
@@ -551,6 +667,48 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
   if (MIXED) o.dgi[i] = (float)(Aij - dcomp);
   o.dinv[i] = Aij != 0 ? 1.0 / Aij : 0.0;
   o.rhs[i] = bi + lag;
+}
+
+// kFmtWin: the block plans its tile as the operator passes will (win_plan) and
+// takes each neighbour's window slot from the plan.  (A walk over the row's 27
+// cells through the cell table in place of the plan took 3.3 ms at 1.16 M
+// particles, nearly three times the rest of the assembly.)
+template <typename R, int FMT, int MIXED>
+__global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, AsmOut o) {
+  if constexpr (FMT != kFmtWin) {
+    const int i = particle_index();
+    if (i < v.n) assemble_row<R, FMT, MIXED>(P, v, o, i, WinSlots{});
+  } else {
+    static_assert(kBlock == kWinThreads, "a tile is a block");
+    __shared__ WinPlan S;
+    const int i0 = particle_index() - (int)threadIdx.x, i1 = min(i0 + kBlock, v.n);
+    for (int s0 = i0; s0 < i1;) {
+      int e0, cells;
+      const int m = win_plan(o, s0, i1, S, &e0, &cells, [](int, int, int, int first) { return first; });
+      if ((int)threadIdx.x < cells) S.start[threadIdx.x] = S.pre[threadIdx.x] - S.start[threadIdx.x];
+      __syncthreads();
+      const int i = s0 + (int)threadIdx.x;
+      s0 = m;
+      if (i >= m) continue;
+      WinSlots w{};
+      if (cells > 0) {
+        const uint32_t key = o.keys[i], cb = cell_bits_of(o, key);
+        const int c = 9 * (win_ekey(o, key) - e0);
+        w.D = S.start + c;
+        w.base = S.pre[c];
+        w.total = S.pre[c + 27] - S.pre[c];
+        w.cx = (int)(cb & 1023u);
+        w.cy = (int)((cb >> 10) & 1023u);
+        w.cz = (int)(cb >> 20);
+      }
+      // an overfull window, or a row outside the cells: plain indices
+      if (o.row[i] && (cells == 0 || w.total > kWinMax)) {
+        atomicOr(o.flags, (unsigned)kFlagOffset);
+        continue;
+      }
+      assemble_row<R, FMT, MIXED>(P, v, o, i, w);
+    }
+  }
 }
 
 template <typename R>
@@ -593,9 +751,9 @@ __global__ __launch_bounds__(kRedThreads) void k_rhs_norm(int n, const int* row,
 }
 
 // number of stored entries (partials)
-__global__ __launch_bounds__(kRedThreads) void k_count_nnz(int n, const int* ccnt, double* partials) {
+__global__ __launch_bounds__(kRedThreads) void k_count_nnz(int n, const int* ccnt, int mask, double* partials) {
   double d[1] = {0.0};
-  for (RowIter it = xcd_rows(n); it.i < it.end; it.i += it.stride) d[0] += (double)ccnt[it.i];
+  for (RowIter it = xcd_rows(n); it.i < it.end; it.i += it.stride) d[0] += (double)(ccnt[it.i] & mask);
   block_partials<1>(d, partials);
 }
 
@@ -666,7 +824,7 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_mv(PpeOp o, const V* __restr
   block_partials<2>(d, partials);
 }
 
-// ----- LDS-staged inner matvec (kFmtRun8) -------------------------------------
+// ----- LDS-staged FP64 matvec (kFmtRun8) --------------------------------------
 // A block takes its rows in tiles of kRedThreads consecutive particles.  The
 // columns of a tile lie in nine particle ranges, one per (dy, dz) row of
 // neighbour cells: cell keys [kmin - 1 + off, kmax + 1 + off] with
@@ -730,12 +888,11 @@ __device__ bool stage_tile(const PpeOp& o, const XT* __restrict__ x, int i0, int
   return true;
 }
 
-template <int CM, typename V>
+template <typename V>
 __global__ __launch_bounds__(kRedThreads, 8) void k_bi_mv_staged(PpeOp o, const V* __restrict__ x,
                                                               V* __restrict__ y, const V* __restrict__ w,
                                                               double* partials, const BiState* st) {
   if (!iter_live(st)) return;
-  typedef typename std::conditional<CM == 0, float, double>::type AT;
   __shared__ Stage<V> S;
   double d[2] = {0.0, 0.0};
   const RowIter it = xcd_rows(o.n);
@@ -745,11 +902,11 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_bi_mv_staged(PpeOp o, const 
     const bool staged = stage_tile(o, x, i0, i1, S);
     const int i = i0 + t;
     if (i < i1) {
-      AT acc = 0;
+      double acc = 0;
       if (o.row[i]) {
-        const AT s = staged ? row_sum<kFmtRun8, CM, AT, V, true>(o, i, S.x, S.adj)
-                            : row_sum<kFmtRun8, CM, AT, V>(o, i, x);
-        acc = (CM == 0 ? (AT)o.dgi[i] : (AT)o.diag[i]) * (AT)x[i] - s;
+        const double s = staged ? row_sum<kFmtRun8, 2, double, V, true>(o, i, S.x, S.adj)
+                                : row_sum<kFmtRun8, 2, double, V>(o, i, x);
+        acc = o.diag[i] * (double)x[i] - s;
       }
       const V yi = (V)acc;
       y[i] = yi;
@@ -760,11 +917,84 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_bi_mv_staged(PpeOp o, const 
   block_partials<2>(d, partials);
 }
 
+// ----- window-staged operator passes (kFmtWin, win.hpp) ------------------------
+// y = A x with the inner FP32 operator; partials (w, y), (y, y).  G lanes per
+// row (win_group).
+template <int G>
+__global__ __launch_bounds__(kRedThreads, 8) void k_win_mv(PpeOp o, const float* __restrict__ x,
+                                                        float* __restrict__ y, const float* __restrict__ w,
+                                                        double* partials, const BiState* st) {
+  if (!iter_live(st)) return;
+  __shared__ WinStage<float> S;
+  double d[2] = {0.0, 0.0};
+  const int sub = (int)threadIdx.x & (G - 1);
+  win_rows<G>(o, S, x, [&](int i) {
+    WinHead<G> h;
+    h.load(o, i, sub);
+    return h;
+  }, [&](int i, int base, bool lead, WinHead<G>& h) {
+    float s = 0.f;
+    const bool on = h.row != 0;
+    if (on) s = group_sum<G>(win_row_sum<G>(o, h, S.x + base));
+    if (!lead) return;
+    const float yi = on ? o.dgi[i] * x[i] - s : 0.f;
+    y[i] = yi;
+    d[0] += (double)w[i] * (double)yi;
+    d[1] += (double)yi * (double)yi;
+  });
+  block_partials<2>(d, partials);
+}
+
+// y = A x or rhs - A x with hi + lo in FP64, optional ||y||^2 partials
+template <int G>
+__global__ __launch_bounds__(kRedThreads) void k_win_apply(PpeOp o, const double* __restrict__ x,
+                                                           double* __restrict__ y, int residual, int want_norm,
+                                                           double* partials) {
+  __shared__ WinStage<double> S;
+  double d[1] = {0.0};
+  win_rows<G>(o, S, x, [&](int i) { return WinRow{o.row[i]}; }, [&](int i, int base, bool lead, WinRow h) {
+    double s = 0;
+    const bool on = h.row != 0;
+    if (on) s = group_sum<G>(win_row_sum_full<G>(o, i, S.x + base));
+    if (!lead) return;
+    double acc = on ? o.diag[i] * x[i] - s : 0.0;
+    if (on && residual) acc = o.rhs[i] - acc;
+    y[i] = acc;
+    d[0] += acc * acc;
+  });
+  if (want_norm) block_partials<1>(d, partials);
+}
+
+// the true residual after a fold, as k_bi_true
+template <int G>
+__global__ __launch_bounds__(kRedThreads) void k_win_true(PpeOp o, const double* __restrict__ x64,
+                                                          double* __restrict__ r64, float* __restrict__ r,
+                                                          const float* __restrict__ rh, double* partials,
+                                                          const BiState* st) {
+  if (st->done || !st->update) return;
+  const double inv = 1.0 / st->xscale;
+  __shared__ WinStage<double> S;
+  double d[3] = {0.0, 0.0, 0.0};
+  win_rows<G>(o, S, x64, [&](int i) { return WinRow{o.row[i]}; }, [&](int i, int base, bool lead, WinRow h) {
+    double s = 0;
+    const bool on = h.row != 0;
+    if (on) s = group_sum<G>(win_row_sum_full<G>(o, i, S.x + base));
+    if (!lead) return;
+    const double acc = on ? o.rhs[i] - (o.diag[i] * x64[i] - s) : 0.0;
+    r64[i] = acc;
+    const float ri = (float)(acc * inv);
+    r[i] = ri;
+    d[0] += (double)ri * (double)ri;
+    d[1] += (double)rh[i] * (double)ri;
+    d[2] += acc * acc;
+  });
+  block_partials<3>(d, partials);
+}
+
 // The FP64 operator passes (y = A x or rhs - A x with an optional norm, and
 // the true residual after a fold) with x64 staged in LDS per tile like the
 // inner matvec (kFmtRun8).  Each thread sums the same rows in the same order
 // as the unstaged kernels, so the bits are the same.
-template <int CM>
 __global__ __launch_bounds__(kRedThreads) void k_apply_staged(PpeOp o, const double* __restrict__ x,
                                                               double* __restrict__ y, int residual, int want_norm,
                                                               double* partials) {
@@ -779,8 +1009,8 @@ __global__ __launch_bounds__(kRedThreads) void k_apply_staged(PpeOp o, const dou
     if (i < i1) {
       double acc = 0;
       if (o.row[i]) {
-        const double sm = staged ? row_sum<kFmtRun8, CM, double, double, true>(o, i, S.x, S.adj)
-                                 : row_sum<kFmtRun8, CM, double>(o, i, x);
+        const double sm = staged ? row_sum<kFmtRun8, 2, double, double, true>(o, i, S.x, S.adj)
+                                 : row_sum<kFmtRun8, 2, double>(o, i, x);
         acc = o.diag[i] * x[i] - sm;
         if (residual) acc = o.rhs[i] - acc;
       }
@@ -791,7 +1021,7 @@ __global__ __launch_bounds__(kRedThreads) void k_apply_staged(PpeOp o, const dou
   if (want_norm) block_partials<1>(d, partials);
 }
 
-template <int CMF, typename V>
+template <typename V>
 __global__ __launch_bounds__(kRedThreads) void k_bi_true_staged(PpeOp o, const double* __restrict__ x64,
                                                                 double* __restrict__ r64, V* __restrict__ r,
                                                                 const V* __restrict__ rh, double* partials,
@@ -809,8 +1039,8 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_true_staged(PpeOp o, const d
     if (i < i1) {
       double acc = 0;
       if (o.row[i]) {
-        const double sm = staged ? row_sum<kFmtRun8, CMF, double, double, true>(o, i, S.x, S.adj)
-                                 : row_sum<kFmtRun8, CMF, double>(o, i, x64);
+        const double sm = staged ? row_sum<kFmtRun8, 2, double, double, true>(o, i, S.x, S.adj)
+                                 : row_sum<kFmtRun8, 2, double>(o, i, x64);
         acc = o.rhs[i] - (o.diag[i] * x64[i] - sm);
       }
       r64[i] = acc;
@@ -1029,19 +1259,37 @@ __global__ void k_zero_u32(unsigned* p, int n) {
   if (i < n) p[i] = 0u;
 }
 
-void launch_fin(hipStream_t s, const PpeWork& w, int op, unsigned* count_out = nullptr) {
-  k_fin<<<1, kFinThreads, 0, s>>>(w.partials, w.nbg, op, (BiState*)w.state, count_out);
+void launch_fin(hipStream_t s, const PpeWork& w, int op, unsigned* count_out = nullptr, int G = 0) {
+  k_fin<<<1, kFinThreads, 0, s>>>(w.partials, G > 0 ? G : w.nbg, op, (BiState*)w.state, count_out);
 }
 
-// host-side dispatch on (format, coefficient mode)
-template <int CM>
+// blocks of a window-staged pass over n rows with G lanes each
+int win_grid(int n, int G) { return grid_rows((int)std::min<int64_t>((int64_t)n * G, INT32_MAX)); }
+#define WIN_LAUNCH(kern, n, ...)                                                      \
+  do {                                                                                \
+    switch (win_group(n)) {                                                           \
+      case 1: kern<1><<<win_grid(n, 1), kRedThreads, 0, s>>>(__VA_ARGS__); break;     \
+      case 2: kern<2><<<win_grid(n, 2), kRedThreads, 0, s>>>(__VA_ARGS__); break;     \
+      default: kern<4><<<win_grid(n, 4), kRedThreads, 0, s>>>(__VA_ARGS__); break;    \
+    }                                                                                 \
+  } while (0)
+int win_blocks(int n) { return win_grid(n, win_group(n)); }
+
+// y = A x in full precision by the operator's format
 void launch_apply_full(hipStream_t s, const PpeWork& w, const PpeOp& o, const double* x, double* y, bool residual,
                        bool norm) {
-  if (o.fmt == kFmtRun8)
-    k_apply_staged<CM><<<w.nbg, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
-  else
-    k_apply_full<kFmtIdx32, CM><<<w.nbg, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
-  if (norm) launch_fin(s, w, kFinNorm);
+  int G = w.nbg;
+  if (o.fmt == kFmtWin) {
+    WIN_LAUNCH(k_win_apply, w.n, o, x, y, residual, norm, w.partials);
+    G = win_blocks(w.n);
+  } else if (o.fmt == kFmtRun8) {
+    k_apply_staged<<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
+  } else if (w.mixed) {
+    k_apply_full<kFmtIdx32, 1><<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
+  } else {
+    k_apply_full<kFmtIdx32, 2><<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
+  }
+  if (norm) launch_fin(s, w, kFinNorm, nullptr, G);
 }
 
 int read_state(hipStream_t s, PpeWork& w, BiState* out) {
@@ -1115,6 +1363,8 @@ PpeOp ppe_op(const PpeWork& w) {
   o.fmt = w.fmt;
   o.NI = w.NI;
   o.NJ = w.NJ;
+  o.NK = w.NK;
+  o.pmask = w.pmask;
   o.ncell = w.ncell;
   o.keys = w.keys;
   o.cell_off = w.cell_off;
@@ -1152,33 +1402,38 @@ int ppe_assemble(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork
   w.gen++;
   w.NI = P.NI;
   w.NJ = P.NJ;
+  w.NK = P.NK;
+  w.pmask = P.pmask;
   w.ncell = P.NI * P.NJ * P.NK;
   w.rowmajor = P.z_index == 0;
-  AsmOut o{v.n, P.NI, P.NJ, P.NK, keys, cell_off, w.row, w.ccnt, w.runc, w.idx, w.hi, w.lo, w.c64,
+  AsmOut o{v.n, P.NI, P.NJ, P.NK, P.pmask, P.NI * P.NJ * P.NK, keys, cell_off, w.row, w.ccnt, w.runc, w.idx, w.hi, w.lo, w.c64,
            w.diag, w.dinv, w.rhs, w.dgi, w.flags};
   const int g = grid_xcd(v.n);
-  k_rowmask<<<g, kBlock, 0, s>>>(P, v.n, v.ptype, v.btype, v.itype, v.surf, v.pres, w.row);
-  if constexpr (std::is_same<R, float>::value) k_pack_asm<<<grid_for(v.n), kBlock, 0, s>>>(v, w.row);
-  // the x-runs of the stencil are contiguous only in row-major keys without
-  // periodic wrap
-  int fmt = (P.z_index || P.pmask) ? kFmtIdx32 : kFmtRun8;
+  // flags: overflow bits, stored entries, then the two peaks
+  const int gm = std::min(grid_for(v.n), kMaxGrid);
+  float2* peak = reinterpret_cast<float2*>(w.partials);
+  k_rowmask<<<gm, kBlock, 0, s>>>(P, v.n, v.ptype, v.btype, v.itype, v.surf, v.m, v.rho, v.por, v.pres, w.row,
+                                  w.mixed ? peak : nullptr);
+  k_asm_begin<<<1, kBlock, 0, s>>>(peak, w.mixed ? gm : 0, w.flags);
+  if constexpr (std::is_same<R, float>::value) k_pack_asm<<<grid_for(v.n), kBlock, 0, s>>>(v, w.row, keys, P.NI, P.NJ);
+  // window slots (mixed) need row-major keys; the x-runs of the FP64 format
+  // are contiguous only in row-major keys without periodic wrap
+  const int long_axis = std::max({P.NI, P.NJ, P.NK});  // images need whole coordinates in ten bits (win_step)
+  int fmt = P.z_index || (P.pmask && long_axis > 1000) ? kFmtIdx32 : (w.mixed ? kFmtWin : (P.pmask ? kFmtIdx32 : kFmtRun8));
   for (;;) {
-    k_zero_u32<<<1, 64, 0, s>>>(w.flags, 4);
-    if (fmt == kFmtRun8) {
-      if (w.mixed) k_assemble<R, kFmtRun8, 1><<<g, kBlock, 0, s>>>(P, v, o);
-      else k_assemble<R, kFmtRun8, 0><<<g, kBlock, 0, s>>>(P, v, o);
-    } else {
-      if (w.mixed) k_assemble<R, kFmtIdx32, 1><<<g, kBlock, 0, s>>>(P, v, o);
-      else k_assemble<R, kFmtIdx32, 0><<<g, kBlock, 0, s>>>(P, v, o);
-    }
-    k_count_nnz<<<w.nbg, kRedThreads, 0, s>>>(v.n, w.ccnt, w.partials);
+    if (fmt == kFmtWin) k_assemble<R, kFmtWin, 1><<<g, kBlock, 0, s>>>(P, v, o);
+    else if (fmt == kFmtRun8) k_assemble<R, kFmtRun8, 0><<<g, kBlock, 0, s>>>(P, v, o);
+    else if (w.mixed) k_assemble<R, kFmtIdx32, 1><<<g, kBlock, 0, s>>>(P, v, o);
+    else k_assemble<R, kFmtIdx32, 0><<<g, kBlock, 0, s>>>(P, v, o);
+    k_count_nnz<<<w.nbg, kRedThreads, 0, s>>>(v.n, w.ccnt, fmt == kFmtWin ? 0xFFFF : -1, w.partials);
     launch_fin(s, w, kFinCount, w.flags + 1);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(w.host_flags, w.flags, 8, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     const unsigned f = w.host_flags[0];
-    if (fmt == kFmtRun8 && (f & (kFlagOffset | kFlagRunCount))) {
-      fmt = kFmtIdx32;  // a run longer than 256 particles: plain indices
+    if (fmt != kFmtIdx32 && (f & (kFlagOffset | kFlagRunCount))) {
+      k_zero_u32<<<1, 64, 0, s>>>(w.flags, 2);
+      fmt = kFmtIdx32;  // an overfull run or window: plain indices
       continue;
     }
     if (f & kFlagOrder) {
@@ -1207,8 +1462,7 @@ int ppe_apply64(hipStream_t s, PpeWork& w, const double* x, double* y, bool resi
     return 0;
   }
   PpeOp o = ppe_op(w);
-  if (w.mixed) launch_apply_full<1>(s, w, o, x, y, residual, norm2 != nullptr);
-  else launch_apply_full<2>(s, w, o, x, y, residual, norm2 != nullptr);
+  launch_apply_full(s, w, o, x, y, residual, norm2 != nullptr);
   HIP_TRY(hipGetLastError());
   if (norm2) {
     BiState h;
@@ -1351,6 +1605,12 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
     tm->count(mv_all);
     return (w.mv_seq++ % kMvSample) == 0 ? tm : nullptr;
   };
+  const int Gm = FMT == kFmtWin ? win_blocks(n) : G;  // blocks of the operator passes
+  auto matvec = [&](const V* x, V* y, const V* ww) {
+    if constexpr (FMT == kFmtWin) WIN_LAUNCH(k_win_mv, n, o, x, y, ww, w.partials, st);
+    else if constexpr (FMT == kFmtRun8) k_bi_mv_staged<V><<<G, kRedThreads, 0, s>>>(o, x, y, ww, w.partials, st);
+    else k_bi_mv<FMT, CM, V><<<G, kRedThreads, 0, s>>>(o, x, y, ww, w.partials, st);
+  };
   int chunk = 8;
   BiState h{};
   double rr0 = 1.0;
@@ -1364,10 +1624,9 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
       }
       {
         TimeScope ts(mv_timer(), mv_name);
-        if (FMT == kFmtRun8) k_bi_mv_staged<CM, V><<<G, kRedThreads, 0, s>>>(o, ph, v, rh, w.partials, st);
-        else k_bi_mv<FMT, CM, V><<<G, kRedThreads, 0, s>>>(o, ph, v, rh, w.partials, st);
+        matvec(ph, v, rh);
       }
-      launch_fin(s, w, kFinAlpha);
+      launch_fin(s, w, kFinAlpha, nullptr, Gm);
       if (cw) {
         const CoarseUpd<V> u{w.dinv, r, p, v, sh, &st->alpha, &st->beta, &st->omega, &st->first};
         TRY(coarse_apply_update<V>(s, *cw, w, u, 2, &st->done, &st->brk));
@@ -1376,16 +1635,17 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
       }
       {
         TimeScope ts(mv_timer(), mv_name);
-        if (FMT == kFmtRun8) k_bi_mv_staged<CM, V><<<G, kRedThreads, 0, s>>>(o, sh, t, r, w.partials, st);
-        else k_bi_mv<FMT, CM, V><<<G, kRedThreads, 0, s>>>(o, sh, t, r, w.partials, st);
+        matvec(sh, t, r);
       }
-      launch_fin(s, w, kFinOmega);
+      launch_fin(s, w, kFinOmega, nullptr, Gm);
       k_bi_xr<V><<<G, kRedThreads, 0, s>>>(n, xs, ph, sh, r, t, rh, w.partials, st);
       launch_fin(s, w, kFinRho);
       k_bi_fold<V><<<G, kRedThreads, 0, s>>>(n, w.row, w.x64, xs, st);
-      if (FMT == kFmtRun8) k_bi_true_staged<CMF, V><<<G, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
+      if constexpr (FMT == kFmtWin) WIN_LAUNCH(k_win_true, n, o, w.x64, w.r64, r, rh, w.partials, st);
+      else if constexpr (FMT == kFmtRun8)
+        k_bi_true_staged<V><<<G, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
       else k_bi_true<FMT, CMF, V><<<G, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
-      launch_fin(s, w, kFinTrue);
+      launch_fin(s, w, kFinTrue, nullptr, Gm);
     }
     HIP_TRY(hipGetLastError());
     TRY(read_state(s, w, &h));
@@ -1410,8 +1670,8 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
 template <typename V, int CM, int CMF>
 int bicgstab_dispatch(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, double tol, double delta,
                       int max_iter, int* iters, int* folds, int* done, Timers* tm) {
-  if (w.fmt == kFmtRun8)
-    return bicgstab_run<V, kFmtRun8, CM, CMF>(s, w, cw, rn, tol, delta, max_iter, iters, folds, done, tm);
+  constexpr int kFmt = sizeof(V) == 4 ? kFmtWin : kFmtRun8;  // the staged format of this path
+  if (w.fmt == kFmt) return bicgstab_run<V, kFmt, CM, CMF>(s, w, cw, rn, tol, delta, max_iter, iters, folds, done, tm);
   return bicgstab_run<V, kFmtIdx32, CM, CMF>(s, w, cw, rn, tol, delta, max_iter, iters, folds, done, tm);
 }
 
@@ -1542,8 +1802,8 @@ __global__ void k_to_f64(int n, const float* __restrict__ a, double* __restrict_
 template <typename R>
 int ppe_matvec_probe(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork& w, int variant, int reps,
                      const double* x64, double* y64, float2* pk, float* ms) {
-  if (!w.mixed || w.fmt != kFmtRun8) {
-    set_error("matvec probe: needs the mixed-precision operator with run offsets");
+  if (!w.mixed || w.fmt != kFmtWin) {
+    set_error("matvec probe: needs the mixed-precision operator with window slots");
     return SOPHIA_E_STATE;
   }
   const int n = w.n;
@@ -1568,7 +1828,7 @@ int ppe_matvec_probe(hipStream_t s, const DevParams& P, const SphView<R>& v, Ppe
   for (int k = 0; k <= reps; k++) {
     if (k == 1) HIP_TRY(hipEventRecord(e0, s));  // the first launch warms the caches, untimed
     if (variant == 1) k_mf_matvec<R><<<grid_xcd(n), kBlock, 0, s>>>(P, v, w.row, w.diag, pk, x, y);
-    else k_bi_mv_staged<0, float><<<w.nbg, kRedThreads, 0, s>>>(o, x, y, rh, w.partials, st);
+    else WIN_LAUNCH(k_win_mv, n, o, x, y, rh, w.partials, st);
   }
   HIP_TRY(hipEventRecord(e1, s));
   HIP_TRY(hipEventSynchronize(e1));

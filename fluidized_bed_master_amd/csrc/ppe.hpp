@@ -7,45 +7,81 @@
 namespace sophia {
 
 // Column encodings of the compact operator.
-//   kFmtRun8 : row-major cell keys.  The 27-cell stencil of a particle is 9
-//              runs of 3 x-adjacent cells, each a contiguous range of the
-//              cell-sorted particle order; a column is stored as a u8 offset
-//              from its run's first particle, and a u64 per row holds the 9
-//              run lengths (7 bits each).  Needs every run <= 256 particles.
-//   kFmtIdx32: plain u32 column indices (Morton keys or overfull runs).
-enum { kFmtRun8 = 0, kFmtIdx32 = 1 };
+//   kFmtWin  : mixed path, row-major cell keys (periodic or not).  A column is
+//              an 11-bit slot in the row's window: the particles of the 27
+//              cells around the row's cell, plane by plane (x - 1, x, x + 1),
+//              the nine (dz, dy) cells of a plane in list order.  A tile of
+//              consecutive rows copies the planes of its cells into LDS in
+//              that order once (win_stage), so a row's window is one
+//              contiguous LDS range.  Needs windows of at most kWinMax
+//              particles.
+//   kFmtRun8 : FP64 path, row-major cell keys without periodic wrap.  The
+//              27-cell stencil of a particle is 9 runs of 3 x-adjacent cells,
+//              each a contiguous range of the cell-sorted particle order; a
+//              column is stored as a u8 offset from its run's first particle,
+//              and a u64 per row holds the 9 run lengths (7 bits each).  Needs
+//              every run <= 256 particles.
+//   kFmtIdx32: plain u32 column indices (Morton keys, overfull cells, and the
+//              FP64 path of periodic boxes).
+enum { kFmtRun8 = 0, kFmtIdx32 = 1, kFmtWin = 2 };
 constexpr int kRunBits = 7;  // kFmtRun8: bits per run length in the row's u64
 constexpr int kRunMax = (1 << kRunBits) - 1;
+constexpr int kWinBits = 11;  // kFmtWin: bits of a window slot
+constexpr int kWinMax = (1 << kWinBits) - 1;
 
 // Compact operator: per row only the columns that are PPE rows themselves
 // (wall/buffer columns live in the right-hand side), slot-quad major:
 // entry k of row i sits at ((k / 4) * n + i) * 4 + k % 4, so a wave reads
 // 64 consecutive 16 B (FP32) or 32 B (FP64) quads per four slots.
-// Mixed path: the inner coefficient is fl32(a) rounded to nearest at a
-// 16-bit significand (the low 8 bits of the FP32 word cleared), and with
-// kFmtRun8 the entry's u8 column offset rides in those 8 bits, so an entry
-// is one 4-byte word.  The inner diagonal takes up the rounding of its row,
-// dgi_i = d_i - sum_j (a_ij - hi16(a_ij)): the inner operator then maps a
+// Mixed path: the inner coefficient hi is a rounded to nearest at a 16-bit
+// significand.  With kFmtIdx32 it is the FP32 word with its low 8 bits
+// cleared (hi16_bits).  With kFmtWin an entry is one 4-byte word
+//   sign (1) | exponent (5) | fraction (15) | window slot (11),
+// the exponent counted from the row's anchor (the upper 16 bits of ccnt), so
+// that hi = win_val(word, anchor << 23) takes three integer operations.  The
+// anchor puts a bound of the row's coefficients in the top binade but one;
+// below the 31 binades hi is the nearest value of the range.
+// The inner diagonal takes up the rounding of its row,
+// dgi_i = d_i - sum_j (a_ij - hi_ij): the inner operator then maps a
 // constant vector exactly as the FP64 one does, and differs from it by
-// sum_j (a_ij - hi16(a_ij)) (x_i - x_j) only (relative 2^-16 of a
-// difference).  hi + lo keeps a to about 2^-40 for the FP64 residual.
+// sum_j (a_ij - hi_ij) (x_i - x_j) only (relative 2^-16 of a difference).
+// hi + lo keeps a to about 2^-40 for the FP64 residual.
 __device__ inline uint32_t hi16_bits(double a) { return (__float_as_uint((float)a) + 0x80u) & 0xFFFFFF00u; }
 __device__ inline float hi_val(uint32_t e) { return __uint_as_float(e & 0xFFFFFF00u); }
+__device__ inline float win_val(uint32_t w, int anchor23) {
+  return __int_as_float((((int)w >> 3) & (int)0x8FFFFF00) + anchor23);
+}
+// the word of coefficient a in window slot `off`: the nearest representable
+// value, of magnitude at least 2^(anchor - 127)
+__device__ inline uint32_t win_word(double a, int anchor, uint32_t off) {
+  const uint32_t b = __float_as_uint((float)a) + 0x80u;
+  const uint32_t sign = b & 0x80000000u;
+  int e = (int)((b >> 23) & 255u) - anchor;
+  uint32_t frac = (b >> 8) & 0x7FFFu;
+  if (e < 0) {
+    e = 0;
+    frac = 0;
+  } else if (e > 31) {
+    e = 31;
+    frac = 0x7FFFu;
+  }
+  return sign | ((uint32_t)e << 26) | (frac << kWinBits) | off;
+}
 
 struct PpeOp {
   int n = 0, nq = 0, fmt = kFmtRun8;
-  int NI = 1, NJ = 1, ncell = 1;
+  int NI = 1, NJ = 1, NK = 1, ncell = 1, pmask = 0;
   const uint32_t* keys = nullptr;      // sorted cell key per particle
   const uint32_t* cell_off = nullptr;  // first particle of each cell (dense, num_cells + 1)
   const int* row = nullptr;
-  const int* ccnt = nullptr;           // compact entries per row
+  const int* ccnt = nullptr;           // compact entries per row (kFmtWin: count | anchor << 16)
   const uint64_t* runc = nullptr;      // kFmtRun8 run lengths
-  const uint32_t* idx = nullptr;       // kFmtRun8 FP64 path: u32 [q][i] (4 offsets); kFmtIdx32: u32 [q][i][4]
-  const float* hi = nullptr;           // mixed: hi16(a) | offset    [q][i][4] (hi_bits / hi_val)
-  const float* lo = nullptr;           // mixed: fl32(a - hi16(a))   [q][i][4]
+  const uint32_t* idx = nullptr;       // kFmtRun8: u32 [q][i] (4 offsets); kFmtIdx32: u32 [q][i][4]
+  const float* hi = nullptr;           // mixed: the inner words     [q][i][4] (win_val / hi_val)
+  const float* lo = nullptr;           // mixed: fl32(a - hi)        [q][i][4]
   const double* c64 = nullptr;         // FP64 path                  [q][i][4]
   const double* diag = nullptr;
-  const float* dgi = nullptr;          // mixed: inner diagonal d_i - sum_j (a_ij - hi16(a_ij))
+  const float* dgi = nullptr;          // mixed: inner diagonal d_i - sum_j (a_ij - hi_ij)
   const double* dinv = nullptr;
   const double* rhs = nullptr;
 };
@@ -55,7 +91,7 @@ struct PpeWork {
   int64_t nnz = 0;  // stored entries of the last assembly
   bool mixed = false;
   int fmt = kFmtRun8;
-  int NI = 1, NJ = 1, ncell = 1;
+  int NI = 1, NJ = 1, NK = 1, ncell = 1, pmask = 0;
   bool rowmajor = true;  // cell keys are row-major (not Morton)
   const uint32_t* keys = nullptr;
   const uint32_t* cell_off = nullptr;

@@ -1,0 +1,282 @@
+// LDS-staged traversal of the mixed operator's window format (kFmtWin).
+//
+// A tile of consecutive rows (cell-sorted particles) needs the columns of the
+// cells around its own cells.  In the extended key e = x + 1 + (NI + 2)(y + NJ z),
+// x = -1 .. NI, the cells of the tile are a range [ea, eb], and the planes
+// e = ea - 1 .. eb + 1 hold every column: plane e is the nine (dz, dy) cells
+// around (x, y, z), in the order of the neighbour list, periodic axes
+// wrapped.  win_stage copies the planes' particles of a vector into LDS in that order,
+// so the window of a row in cell e is the planes e - 1, e, e + 1: one
+// contiguous LDS range, and a column is the window's base plus the 11-bit slot
+// of its entry.  Against run offsets (a u8 from the first particle of one of nine
+// x-runs) this takes the eight compares and selects per entry that find the
+// run out of the inner loop, and it works across a periodic wrap.
+//
+// Bound: the operator stream from HBM (4 B per entry) plus 36 B per row; the
+// staging reads about 11 values per row from L2.
+#pragma once
+
+#include "ppe.hpp"
+
+namespace sophia {
+
+constexpr int kWinThreads = 256;
+constexpr int kWinCells = 256;  // staged cells per tile: 28 planes
+// staged values per tile: a 256-row tile of the 1 mm columns takes about 2800;
+// with the tables it is 19.5 KB in FP32, eight blocks per CU
+constexpr int kWinCap = 4352;
+static_assert(kWinMax < kWinCap, "a single row's window always fits");
+
+// Where the cells of a tile's planes go: cell c = 9 (e - ea + 1) + r holds the
+// slots [pre[c], pre[c + 1]) of the staged copy.
+struct WinPlan {
+  int pre[kWinCells + 1];
+  int start[kWinCells];  // cellval of the cell
+  int wsum[kWinThreads / 64];
+};
+template <typename XT>
+struct WinStage {
+  XT x[kWinCap];
+  WinPlan p;
+};
+
+template <class O>
+__device__ inline int win_ekey(const O& o, uint32_t key) {
+  const int t = (int)(key / (uint32_t)o.NI);
+  return (int)(key - (uint32_t)t * (uint32_t)o.NI) + 1 + (o.NI + 2) * t;
+}
+
+// The block plans the longest of the row ranges [i0, i1), its first half,
+// quarter, ... whose planes fit and returns its end m (all threads alike); *e0
+// is the extended key of row i0 and *cells the planned cells, 0 when there is
+// nothing to stage: rows past the last cell, or a single particle whose window
+// does not fit (no row of an assembled operator).  `cellval(x, y, z, first)` is
+// kept per cell in S.start.
+template <class O, class CV>
+__device__ int win_plan(const O& o, int i0, int i1, WinPlan& S, int* e0, int* ncells, CV&& cellval) {
+  const int t = (int)threadIdx.x, lane = t & 63;
+  const uint32_t ka = o.keys[i0];
+  const int NI2 = o.NI + 2;
+  *e0 = 0;
+  *ncells = 0;
+  if (ka >= (uint32_t)o.ncell) return i1;
+  const int ea = win_ekey(o, ka);
+  *e0 = ea;
+  for (int m = i1;; m = i0 + (m - i0) / 2) {
+    __syncthreads();  // the previous tile is done with S
+    const uint32_t kb = o.keys[m - 1];
+    const int cells = kb < (uint32_t)o.ncell ? 9 * (win_ekey(o, kb) - ea + 3) : kWinCells + 1;
+    if (cells > kWinCells) {
+      if (m - i0 == 1) return m;
+      continue;
+    }
+    int len = 0;
+    if (t < cells) {
+      const int p = t / 9, r = t - 9 * p;
+      const int e = ea - 1 + p;
+      const int row = e / NI2;
+      int x = e - NI2 * row - 1, z = row / o.NJ;
+      int y = row - o.NJ * z;
+      y += r % 3 - 1;
+      z += r / 3 - 1;
+      int first = 0;
+      if (cell_in(o.pmask, 2, z, o.NK) && cell_in(o.pmask, 1, y, o.NJ) && cell_in(o.pmask, 0, x, o.NI)) {
+        const int k = x + o.NI * (y + o.NJ * z);
+        first = (int)o.cell_off[k];
+        len = (int)o.cell_off[k + 1] - first;
+      }
+      S.start[t] = cellval(x, y, z, first);
+    }
+    int inc = len;
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(inc, off);
+      if (lane >= off) inc += v;
+    }
+    if (lane == 63) S.wsum[t >> 6] = inc;
+    __syncthreads();
+    int add = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < kWinThreads / 64; w++) {
+      const int v = S.wsum[w];
+      add += w < (t >> 6) ? v : 0;
+      total += v;
+    }
+    if (total > kWinCap) {
+      if (m - i0 == 1) return m;
+      continue;
+    }
+    S.pre[t + 1] = inc + add;
+    if (t == 0) S.pre[0] = 0;
+    __syncthreads();
+    *ncells = cells;
+    return m;
+  }
+}
+
+// win_plan, then the values: `val(cellval, l)` is that of a cell's l-th particle
+template <typename XT, class CV, class F>
+__device__ int win_stage(const PpeOp& o, int i0, int i1, WinStage<XT>& S, int* e0, CV&& cellval, F&& val) {
+  int cells;
+  const int m = win_plan(o, i0, i1, S.p, e0, &cells, static_cast<CV&&>(cellval));
+  if (cells == 0) return m;
+  // half a wave per cell (about 23 particles), four cells in flight
+  const int h = (int)threadIdx.x >> 5, l0 = (int)threadIdx.x & 31;
+  for (int c = h; c < cells; c += 32) {
+    XT v[4];
+    int at[4], n[4], st[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int cc = c + 8 * u;
+      at[u] = cc < cells ? S.p.pre[cc] : 0;
+      n[u] = cc < cells ? S.p.pre[cc + 1] - at[u] : 0;
+      st[u] = l0 < n[u] ? S.p.start[cc] : 0;
+      if (l0 < n[u]) v[u] = val(st[u], l0);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (l0 < n[u]) S.x[at[u] + l0] = v[u];
+      for (int l = l0 + 32; l < n[u]; l += 32) S.x[at[u] + l] = val(st[u], l);
+    }
+  }
+  __syncthreads();
+  return m;
+}
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <bool NT>
+__device__ __forceinline__ u32x4 ldq(const u32x4* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+
+// What a lane has in hand of its row before the tile is staged: the row's
+// first two quads travel while the block stages.  G = 1 (large operators,
+// streamed from HBM once per pass) loads past the caches, so that x stays in
+// L2: 83.3 -> 78.5 us at 1.16 M rows, 69.4 -> 64.4 us for the 10^6-row box;
+// an operator that fits the last-level cache is better left to it.  Two quads
+// in flight: one 92, three 90, four 96 us (registers spill at eight waves).
+constexpr int kWinQ = 2;
+template <int G>
+struct WinHead {
+  int i, row, cnt, anc;
+  u32x4 w[kWinQ];
+  __device__ void load(const PpeOp& o, int ii, int sub) {
+    i = ii;
+    row = o.row[i];
+    const int meta = o.ccnt[i];
+    cnt = meta & 0xFFFF;
+    anc = (meta >> 16) << 23;
+    const u32x4* hp = reinterpret_cast<const u32x4*>(o.hi) + i;
+#pragma unroll
+    for (int u = 0; u < kWinQ; u++) w[u] = ldq<G == 1>(hp + (size_t)min(sub + u * G, o.nq - 1) * (size_t)o.n);
+  }
+};
+
+// The head of a pass that only asks whether the row is one.
+struct WinRow {
+  int row;
+};
+
+// f(i, base, lead, head(i)) for every row of this block's share, by G lanes
+// each: base is the LDS slot of row i's window, lead marks the first of its
+// lanes, and head(i) has run before the tile was staged.  (Leaving out the
+// staging of tiles without rows, behind a barrier vote, costs every tile more
+// than the walls' tiles save: 78.4 -> 85.2 us at 1.16 M rows.)
+template <int G, typename XT, class H, class F>
+__device__ __forceinline__ void win_rows(const PpeOp& o, WinStage<XT>& S, const XT* __restrict__ x, H&& head, F&& f) {
+  constexpr int TR = kWinThreads / G;
+  const int per = (int)gridDim.x >> 3;
+  const int chunk = ((((o.n + 7) >> 3) + 63) >> 6) << 6;  // rows per XCD, as xcd_rows
+  const int lo = (int)(blockIdx.x & 7) * chunk, hi = min(o.n, lo + chunk);
+  const int t = (int)threadIdx.x, tr = t / G;
+  for (int i0 = lo + (int)(blockIdx.x >> 3) * TR; i0 < hi; i0 += per * TR) {
+    const int i1 = min(i0 + TR, hi);
+    for (int s0 = i0; s0 < i1;) {
+      int e0;
+      auto hd = head(min(s0 + tr, i1 - 1));
+      const int m = win_stage(
+          o, s0, i1, S, &e0, [](int, int, int, int first) { return first; }, [&](int first, int l) { return x[first + l]; });
+      const int i = s0 + tr;
+      if (i < m) {
+        const uint32_t key = o.keys[i];
+        const int c = key < (uint32_t)o.ncell ? 9 * (win_ekey(o, key) - e0) : 0;
+        f(i, S.p.pre[min(max(c, 0), kWinCells)], (t & (G - 1)) == 0, hd);
+      }
+      s0 = m;
+    }
+  }
+}
+
+// This lane's share of sum_j hi_ij x_j over the stored columns of row i (quads
+// sub, sub + G, ...); xw is the row's window.  Padding entries need no mask:
+// they are a value on the row's own column that the inner diagonal takes up.
+// Two quads are consumed while the next two are in flight.
+template <int G>
+__device__ __forceinline__ float win_row_sum(const PpeOp& o, WinHead<G>& h, const float* xw) {
+  constexpr int Q = kWinQ;
+  const int nq = (h.cnt + 3) >> 2, last = nq - 1;
+  const int sub = (int)threadIdx.x & (G - 1);
+  float s = 0.f;
+  const u32x4* hp = reinterpret_cast<const u32x4*>(o.hi) + h.i;
+  const size_t n = (size_t)o.n;
+  // quads past the row's last were read ahead of its count: slot 0, unused
+#pragma unroll
+  for (int u = 0; u < Q; u++)
+    if (sub + u * G >= nq) h.w[u] = 0u;
+  for (int q = sub; q < nq; q += Q * G) {
+    u32x4 c[Q];
+    float xv[Q][4];
+#pragma unroll
+    for (int u = 0; u < Q; u++) {
+      c[u] = h.w[u];
+#pragma unroll
+      for (int k = 0; k < 4; k++) xv[u][k] = xw[c[u][k] & (uint32_t)kWinMax];
+    }
+#pragma unroll
+    for (int u = 0; u < Q; u++) h.w[u] = ldq<G == 1>(hp + (size_t)min(q + (Q + u) * G, last) * n);
+#pragma unroll
+    for (int u = 0; u < Q; u++)
+      if (q + u * G < nq) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) s += win_val(c[u][k], h.anc) * xv[u][k];
+      }
+  }
+  return s;
+}
+
+// the same with hi + lo in FP64
+template <int G>
+__device__ __forceinline__ double win_row_sum_full(const PpeOp& o, int i, const double* xw) {
+  const int meta = o.ccnt[i];
+  const int nq = ((meta & 0xFFFF) + 3) >> 2, last = nq - 1;
+  const int anc = (meta >> 16) << 23;
+  const int sub = (int)threadIdx.x & (G - 1);
+  double s = 0;
+  if (sub >= nq) return s;
+  const uint4* hp = reinterpret_cast<const uint4*>(o.hi) + i;
+  const float4* lp = reinterpret_cast<const float4*>(o.lo) + i;
+  const size_t n = (size_t)o.n;
+  uint4 w = hp[(size_t)sub * n];
+  float4 l = lp[(size_t)sub * n];
+  for (int q = sub; q < nq; q += G) {
+    const uint32_t c[4] = {w.x, w.y, w.z, w.w};
+    const float lv[4] = {l.x, l.y, l.z, l.w};
+    double xv[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) xv[u] = xw[c[u] & (uint32_t)kWinMax];
+    w = hp[(size_t)min(q + G, last) * n];
+    l = lp[(size_t)min(q + G, last) * n];
+#pragma unroll
+    for (int u = 0; u < 4; u++) s += ((double)win_val(c[u], anc) + (double)lv[u]) * xv[u];
+  }
+  return s;
+}
+
+// Lanes per row of the window-staged passes.  One lane walks about 20 quads in
+// turn, which hides behind other waves only when there are many: at 4,200 /
+// 92,000 / 276,000 / 1,160,000 rows the inner product takes 14.7 / 15.3 / 27.2 /
+// 78.5 us with one lane, 8.2 / 10.5 / 22.7 / 86 with two and 7.1 / 11.2 / 26 / 110
+// with four (a tile has 256 / G rows, so more lanes stage more per row).
+inline int win_group(int n) { return n >= 500000 ? 1 : (n >= 40000 ? 2 : 4); }
+
+}  // namespace sophia
