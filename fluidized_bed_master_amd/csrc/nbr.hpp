@@ -44,14 +44,53 @@ __device__ inline Nb<R> load_nb(const SphView<R>& v, int j, const NbOrigin& o) {
   return q;
 }
 
+// Lanes per particle of the pair kernels.  With one lane a particle's ~81
+// neighbours are ~20 dependent batches, which only other waves hide, and small
+// runs have few (4,200 particles are 66 waves on 1024 SIMDs).  With G lanes
+// lane g takes the quads g, g + G, ... of the list and the lanes' sums meet in
+// a butterfly (group_sum): the order of a sum changes, not its terms.
+template <int G>
+__device__ inline int pair_particle() { return particle_index() / G; }
+template <int G>
+__device__ inline int pair_sub() { return (int)threadIdx.x & (G - 1); }
+
+// Measured with 1 / 2 / 4 / 8 lanes (us): advection 72 / 41 / 27 / 17 at 4,200
+// particles, 116 / 121 / 124 / 119 at 56,000 (FP64), 112 / 112 / 111 / 115 at 118,000,
+// 292 / 265 / 278 / 304 at 281,000, 1139 / 1112 / 1209 / 1362 at 1.16 M; prep 52 / 29 /
+// 18 / 11, 84 / 62 / 61 / 62, 64 / 48 / 52 / 50, 128 / 112 / 118 / 121 and 605 / 506 / 499 /
+// 523: past 90,000 particles two lanes are the better half of the gathers in
+// flight per wave, below there are too few waves and more lanes win.
+inline int pair_lanes(int n) { return n >= 90000 ? 2 : (n >= 40000 ? 4 : 8); }
+
+// f(lanes as an integral constant, grid) for n particles
+template <class F>
+inline int pair_launch(int n, int lanes, F&& f) {
+  if (n <= 0) return 0;
+  switch (lanes) {
+    case 1: f(std::integral_constant<int, 1>{}, grid_xcd(n)); break;
+    case 2: f(std::integral_constant<int, 2>{}, grid_xcd(n * 2)); break;
+    case 4: f(std::integral_constant<int, 4>{}, grid_xcd(n * 4)); break;
+    default: f(std::integral_constant<int, 8>{}, grid_xcd(n * 8)); break;
+  }
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+template <class F>
+inline int pair_launch(int n, F&& f) {
+  // two lanes per particle stay within an int: 2^30 particles do not fit the
+  // device's memory
+  return pair_launch(n, pair_lanes(n), static_cast<F&&>(f));
+}
+
 // The list in batches of four, in list order, in two phases: the fields of
 // all four neighbours are gathered (straight-line code, so every load of the
 // batch is in flight together), then f(q, on) runs per neighbour; the next
 // batch's indices are loaded before this batch is consumed.  Loads of fields
 // a body never reads are dropped by the compiler.  Slots past the count
 // repeat the last entry with on = false; bodies add `on ? term : 0` (a
-// select: exact, and NaN-safe for the unused slots).
-template <bool REL = false, typename R, class F>
+// select: exact, and NaN-safe for the unused slots).  With G lanes each visits
+// every G-th quad, and the caller sums over the lanes.
+template <bool REL = false, int G = 1, typename R, class F>
 __device__ inline void for_nbrs4(const SphView<R>& v, int i, bool eps_rule, F&& f) {
   const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
   if (cnt <= 0) return;
@@ -63,8 +102,9 @@ __device__ inline void for_nbrs4(const SphView<R>& v, int i, bool eps_rule, F&& 
     o.x = v.x[i]; o.y = v.y[i]; o.z = v.z[i];
   }
   const int last4 = (cnt - 1) & ~3;
-  uint4 en4 = *(const uint4*)(v.nbr + nbr_slot(0, i, (int)n));
-  for (int k = 0; k < cnt; k += 4) {
+  const int k0 = G == 1 ? 0 : 4 * pair_sub<G>();
+  uint4 en4 = *(const uint4*)(v.nbr + nbr_slot(min(k0, last4), i, (int)n));
+  for (int k = k0; k < cnt; k += 4 * G) {
     const uint32_t en[4] = {en4.x, en4.y, en4.z, en4.w};
     uint32_t e[4];
 #pragma unroll
@@ -72,7 +112,7 @@ __device__ inline void for_nbrs4(const SphView<R>& v, int i, bool eps_rule, F&& 
     Nb<R> q[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) q[u] = load_nb<REL>(v, (int)(e[u] & ~kNbrFlag), o);
-    en4 = *(const uint4*)(v.nbr + nbr_slot(min(k + 4, last4), i, (int)n));
+    en4 = *(const uint4*)(v.nbr + nbr_slot(min(k + 4 * G, last4), i, (int)n));
 #pragma unroll
     for (int u = 0; u < 4; u++) {
       const bool on = (k + u < cnt) && !(eps_rule && (e[u] & kNbrFlag));
@@ -98,15 +138,16 @@ struct NbP {
 // place of twelve or seven.  With VEL on the mixed path pk, pkb = {rho, p,
 // u, T} and pkc = {S, h, p_type}: three.  dx = x_i - x_j (minimum image on periodic axes),
 // the same bits as pdiff.
-template <bool VEL, typename R, class F>
+template <bool VEL, int G = 1, typename R, class F>
 __device__ inline void for_nbrs4_pk(const SphView<R>& v, int i, bool eps_rule, F&& f) {
   const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
   if (cnt <= 0) return;
   const int n = v.n;
   const double4 pi = v.pk[i];
   const int last4 = (cnt - 1) & ~3;
-  uint4 en4 = *(const uint4*)(v.nbr + nbr_slot(0, i, n));
-  for (int k = 0; k < cnt; k += 4) {
+  const int k0 = G == 1 ? 0 : 4 * pair_sub<G>();
+  uint4 en4 = *(const uint4*)(v.nbr + nbr_slot(min(k0, last4), i, n));
+  for (int k = k0; k < cnt; k += 4 * G) {
     const uint32_t en[4] = {en4.x, en4.y, en4.z, en4.w};
     NbP<R> q[4];
 #pragma unroll
@@ -141,7 +182,7 @@ __device__ inline void for_nbrs4_pk(const SphView<R>& v, int i, bool eps_rule, F
       }
       q[u].j = j;
     }
-    en4 = *(const uint4*)(v.nbr + nbr_slot(min(k + 4, last4), i, n));
+    en4 = *(const uint4*)(v.nbr + nbr_slot(min(k + 4 * G, last4), i, n));
 #pragma unroll
     for (int u = 0; u < 4; u++) {
       const bool on = (k + u < cnt) && !(eps_rule && (en[u] & kNbrFlag));
@@ -168,15 +209,16 @@ struct NbR {
 // The list in batches of four like for_nbrs4<true>, reading r32 (and with
 // VEL pkv = {ux, uy, uz, T}): one or two gathers per neighbour in place of
 // four to eight, the same values.
-template <bool VEL, class F>
+template <bool VEL, int G = 1, class F>
 __device__ inline void for_nbrs4_r32(const SphView<float>& v, int i, bool eps_rule, F&& f) {
   const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
   if (cnt <= 0) return;
   const int n = v.n;
   const float4 pi4 = v.pos4[i];
   const int last4 = (cnt - 1) & ~3;
-  uint4 en4 = *(const uint4*)(v.nbr + nbr_slot(0, i, n));
-  for (int k = 0; k < cnt; k += 4) {
+  const int k0 = G == 1 ? 0 : 4 * pair_sub<G>();
+  uint4 en4 = *(const uint4*)(v.nbr + nbr_slot(min(k0, last4), i, n));
+  for (int k = k0; k < cnt; k += 4 * G) {
     const uint32_t en[4] = {en4.x, en4.y, en4.z, en4.w};
     NbR q[4];
 #pragma unroll
@@ -193,7 +235,7 @@ __device__ inline void for_nbrs4_r32(const SphView<float>& v, int i, bool eps_ru
       q[u].j = j;
       q[u].flag = (en[u] & kNbrFlag) != 0;
     }
-    en4 = *(const uint4*)(v.nbr + nbr_slot(min(k + 4, last4), i, n));
+    en4 = *(const uint4*)(v.nbr + nbr_slot(min(k + 4 * G, last4), i, n));
 #pragma unroll
     for (int u = 0; u < 4; u++) {
       const bool on = (k + u < cnt) && !(eps_rule && (en[u] & kNbrFlag));

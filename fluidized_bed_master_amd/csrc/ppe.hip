@@ -428,13 +428,19 @@ __global__ void k_pack_asm(SphView<float> v, const int* __restrict__ row, const 
   v.ra[i] = r;
 }
 
-template <typename R, int FMT, int MIXED>
+// One row by G lanes.  With one lane the quads of stored columns collect in
+// registers and leave whole; with more, the lanes of a round rank their columns
+// by a scan over the group, so the stored order is the list's either way, and
+// store them one by one.
+template <typename R, int FMT, int MIXED, int G>
 __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R>& v, const AsmOut& o, int i,
                                              const WinSlots& ww) {
   const int n = v.n;
   const size_t nn = (size_t)n;
   const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
+  const int sub = pair_sub<G>();
   if (!o.row[i]) {
+    if (sub != 0) return;
     o.ccnt[i] = 0;
     o.runc[i] = 0;
     o.diag[i] = 0;
@@ -525,6 +531,18 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
       reinterpret_cast<double2*>(o.c64)[2 * qs + 1] = make_double2(qc4[2], qc4[3]);
     }
   };
+  // column k of the row (G > 1)
+  auto store_one = [&](int k, uint32_t jj, uint32_t h, float l, double c, uint32_t off8) {
+    const size_t e = ((size_t)(k >> 2) * nn + i) * 4 + (size_t)(k & 3);
+    if (FMT == kFmtIdx32) o.idx[e] = jj;
+    if (FMT == kFmtRun8) reinterpret_cast<uint8_t*>(o.idx)[e] = (uint8_t)off8;
+    if (MIXED) {
+      reinterpret_cast<uint32_t*>(o.hi)[e] = h;
+      o.lo[e] = l;
+    } else {
+      o.c64[e] = c;
+    }
+  };
   unsigned bad = 0;
   // the list in batches of four: every field of the batch is gathered
   // before any is used (straight-line loads, all in flight together), the
@@ -538,8 +556,9 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
     int slot;       // kFmtWin: its slot in the row's window
   };
   const int last4 = (cnt - 1) & ~3;
-  uint4 en4 = cnt > 0 ? *(const uint4*)(v.nbr + nbr_slot(0, i, (int)n)) : make_uint4(0u, 0u, 0u, 0u);
-  for (int k0 = 0; k0 < cnt; k0 += 4) {
+  uint4 en4 = cnt > 0 ? *(const uint4*)(v.nbr + nbr_slot(min(4 * sub, last4), i, (int)n)) : make_uint4(0u, 0u, 0u, 0u);
+  for (int kr = 0; kr < cnt; kr += 4 * G) {
+    const int k0 = kr + 4 * sub;
     uint32_t eb[4];
     const uint32_t en[4] = {en4.x, en4.y, en4.z, en4.w};
     AsmNb nb[4];
@@ -565,7 +584,11 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
         nb[u].slot = FMT == kFmtWin ? win_slot(o, ww, cell_bits_of(o, o.keys[j]), j) : 0;
       }
     }
-    en4 = *(const uint4*)(v.nbr + nbr_slot(min(k0 + 4, last4), i, (int)n));
+    en4 = *(const uint4*)(v.nbr + nbr_slot(min(k0 + 4 * G, last4), i, (int)n));
+    uint32_t ej[4], eh[4], eo[4];
+    float el[4];
+    double ec[4];
+    int ne = 0, keep[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int ub = 0; ub < 4; ub++) {
     if (k0 + ub >= cnt) break;
@@ -610,7 +633,7 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
         else rcw += 1ull << (kRunBits * run);
       }
       off8 = (uint32_t)off & 255u;
-      if (!MIXED) {
+      if (G == 1 && !MIXED) {
         word |= off8 << (8 * u);
         if (u == 3) {
           o.idx[(size_t)q * nn + i] = word;
@@ -618,21 +641,65 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
         }
       }
     }
-    if (FMT == kFmtWin) {
-      const uint32_t w = win_word(a, anchor, (uint32_t)nq.slot & (uint32_t)kWinMax);
-      const double hv = (double)win_val(w, anchor << 23);
+    uint32_t hw = 0;
+    float lw = 0.f;
+    if (MIXED) {
+      double hv;
+      if (FMT == kFmtWin) {
+        hw = win_word(a, anchor, (uint32_t)nq.slot & (uint32_t)kWinMax);
+        hv = (double)win_val(hw, anchor << 23);
+      } else {
+        hw = hi16_bits(a);
+        hv = (double)hi_val(hw);
+      }
       dcomp += a - hv;
-      push_quad(0u, w, (float)(a - hv), a);
-    } else if (MIXED) {
-      const uint32_t hb = hi16_bits(a);
-      const double hv = (double)hi_val(hb);
-      dcomp += a - hv;
-      push_quad((uint32_t)j, hb, (float)(a - hv), a);
-    } else {
-      push_quad((uint32_t)j, 0u, 0.f, a);
+      lw = (float)(a - hv);
     }
+    if (G > 1) {
+      ej[ub] = (uint32_t)j;
+      eh[ub] = hw;
+      el[ub] = lw;
+      ec[ub] = a;
+      eo[ub] = off8;
+      keep[ub] = 1;
+      ne++;
+      continue;
+    }
+    push_quad((uint32_t)j, hw, lw, a);
     kc++;
     if ((kc & 3) == 0) store_quad(q);
+    }
+    if (G > 1) {
+      int at = ne;  // columns of the lanes up to this one
+#pragma unroll
+      for (int off = 1; off < G; off <<= 1) {
+        const int p = __shfl_up(at, off, G);
+        if (sub >= off) at += p;
+      }
+      const int all = __shfl(at, G - 1, G);
+      at += kc - ne;
+#pragma unroll
+      for (int ub = 0; ub < 4; ub++)
+        if (keep[ub]) store_one(at++, ej[ub], eh[ub], el[ub], ec[ub], eo[ub]);
+      kc += all;
+    }
+  }
+  if (G > 1) {
+    bx = group_sum<G>(bx);
+    by = group_sum<G>(by);
+    bz = group_sum<G>(bz);
+    Aij = group_sum<G>(Aij);
+    AP = group_sum<G>(AP);
+    lag = group_sum<G>(lag);
+    dcomp = group_sum<G>(dcomp);
+    if (FMT == kFmtRun8) {
+      // the lanes' run lengths; a field past its 7 bits would carry into the
+      // next one and the fields no longer add up to the columns
+      rcw = group_sum<G>(rcw);
+      int tot = 0;
+#pragma unroll
+      for (int r = 0; r < 9; r++) tot += (int)((rcw >> (kRunBits * r)) & kRunMax);
+      if (tot != kc) bad |= kFlagRunCount;
     }
   }
   // pad the last quad so whole-quad loads read defined values
@@ -646,15 +713,21 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
       const float t = win_val(w, anchor << 23);
       for (int u = kc & 3; u < 4; u++) {
         dcomp -= (double)t;
-        push_quad(0u, w, -t, 0.0);
+        if (G == 1) push_quad(0u, w, -t, 0.0);
+        else if (sub == 0) store_one(4 * q + u, 0u, w, -t, 0.0, 0u);
       }
     } else {
-      for (int u = kc & 3; u < 4; u++) push_quad((uint32_t)i, 0u, 0.f, 0.0);
+      for (int u = kc & 3; u < 4; u++)
+        if (G == 1) push_quad((uint32_t)i, 0u, 0.f, 0.0);
+        else if (sub == 0) store_one(4 * q + u, (uint32_t)i, 0u, 0.f, 0.0, 0u);
     }
-    store_quad(q);
-    if (FMT == kFmtRun8 && !MIXED) o.idx[(size_t)q * nn + i] = word;
+    if (G == 1) {
+      store_quad(q);
+      if (FMT == kFmtRun8 && !MIXED) o.idx[(size_t)q * nn + i] = word;
+    }
   }
   if (bad) atomicOr(o.flags, bad);
+  if (G > 1 && sub != 0) return;
   o.ccnt[i] = FMT == kFmtWin ? kc | (anchor << 16) : kc;
   o.runc[i] = rcw;
   const double tdt = P.dt_sph;
@@ -673,21 +746,21 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
 // takes each neighbour's window slot from the plan.  (A walk over the row's 27
 // cells through the cell table in place of the plan took 3.3 ms at 1.16 M
 // particles, nearly three times the rest of the assembly.)
-template <typename R, int FMT, int MIXED>
+template <typename R, int FMT, int MIXED, int G>
 __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, AsmOut o) {
   if constexpr (FMT != kFmtWin) {
-    const int i = particle_index();
-    if (i < v.n) assemble_row<R, FMT, MIXED>(P, v, o, i, WinSlots{});
+    const int i = pair_particle<G>();
+    if (i < v.n) assemble_row<R, FMT, MIXED, G>(P, v, o, i, WinSlots{});
   } else {
     static_assert(kBlock == kWinThreads, "a tile is a block");
     __shared__ WinPlan S;
-    const int i0 = particle_index() - (int)threadIdx.x, i1 = min(i0 + kBlock, v.n);
+    const int i0 = (particle_index() - (int)threadIdx.x) / G, i1 = min(i0 + kBlock / G, v.n);
     for (int s0 = i0; s0 < i1;) {
       int e0, cells;
       const int m = win_plan(o, s0, i1, S, &e0, &cells, [](int, int, int, int first) { return first; });
       if ((int)threadIdx.x < cells) S.start[threadIdx.x] = S.pre[threadIdx.x] - S.start[threadIdx.x];
       __syncthreads();
-      const int i = s0 + (int)threadIdx.x;
+      const int i = s0 + (int)threadIdx.x / G;
       s0 = m;
       if (i >= m) continue;
       WinSlots w{};
@@ -706,7 +779,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
         atomicOr(o.flags, (unsigned)kFlagOffset);
         continue;
       }
-      assemble_row<R, FMT, MIXED>(P, v, o, i, w);
+      assemble_row<R, FMT, MIXED, G>(P, v, o, i, w);
     }
   }
 }
@@ -1388,6 +1461,12 @@ int cell_offsets(hipStream_t s, int n, const uint32_t* keys, int num_cells, uint
   return 0;
 }
 
+// Lanes per row of the assembly: as the pair kernels, but one for large
+// operators, whose whole-quad stores beat the lanes' single ones (1 / 2 / 4 / 8
+// lanes: 99 / 59 / 34 / 23 us at 4,200 particles, 147 / 134 / 142 / 161 at 118,000,
+// 330 / 294 / 329 / 392 at 281,000, 1220 / 1298 / 1433 / 1751 at 1.16 M).
+inline int asm_lanes(int n) { return n >= 500000 ? 1 : pair_lanes(n); }
+
 template <typename R>
 int ppe_assemble(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork& w, const uint32_t* keys,
                  const uint32_t* cell_off) {
@@ -1408,7 +1487,6 @@ int ppe_assemble(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork
   w.rowmajor = P.z_index == 0;
   AsmOut o{v.n, P.NI, P.NJ, P.NK, P.pmask, P.NI * P.NJ * P.NK, keys, cell_off, w.row, w.ccnt, w.runc, w.idx, w.hi, w.lo, w.c64,
            w.diag, w.dinv, w.rhs, w.dgi, w.flags};
-  const int g = grid_xcd(v.n);
   // flags: overflow bits, stored entries, then the two peaks
   const int gm = std::min(grid_for(v.n), kMaxGrid);
   float2* peak = reinterpret_cast<float2*>(w.partials);
@@ -1421,10 +1499,13 @@ int ppe_assemble(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork
   const int long_axis = std::max({P.NI, P.NJ, P.NK});  // images need whole coordinates in ten bits (win_step)
   int fmt = P.z_index || (P.pmask && long_axis > 1000) ? kFmtIdx32 : (w.mixed ? kFmtWin : (P.pmask ? kFmtIdx32 : kFmtRun8));
   for (;;) {
-    if (fmt == kFmtWin) k_assemble<R, kFmtWin, 1><<<g, kBlock, 0, s>>>(P, v, o);
-    else if (fmt == kFmtRun8) k_assemble<R, kFmtRun8, 0><<<g, kBlock, 0, s>>>(P, v, o);
-    else if (w.mixed) k_assemble<R, kFmtIdx32, 1><<<g, kBlock, 0, s>>>(P, v, o);
-    else k_assemble<R, kFmtIdx32, 0><<<g, kBlock, 0, s>>>(P, v, o);
+    TRY(pair_launch(v.n, asm_lanes(v.n), [&](auto gl, int grid) {
+      constexpr int G = decltype(gl)::value;
+      if (fmt == kFmtWin) k_assemble<R, kFmtWin, 1, G><<<grid, kBlock, 0, s>>>(P, v, o);
+      else if (fmt == kFmtRun8) k_assemble<R, kFmtRun8, 0, G><<<grid, kBlock, 0, s>>>(P, v, o);
+      else if (w.mixed) k_assemble<R, kFmtIdx32, 1, G><<<grid, kBlock, 0, s>>>(P, v, o);
+      else k_assemble<R, kFmtIdx32, 0, G><<<grid, kBlock, 0, s>>>(P, v, o);
+    }));
     k_count_nnz<<<w.nbg, kRedThreads, 0, s>>>(v.n, w.ccnt, fmt == kFmtWin ? 0xFFFF : -1, w.partials);
     launch_fin(s, w, kFinCount, w.flags + 1);
     HIP_TRY(hipGetLastError());

@@ -15,6 +15,13 @@ namespace sophia {
 
 namespace {
 
+// the spheres around a particle by its G lanes (periodic boxes have none)
+template <int G, class F>
+__device__ inline void pair_cells(const DevParams& P, double x, double y, double z, const CellView& cv, F&& f) {
+  if constexpr (G == 1) for_cells(P, x, y, z, cv, static_cast<F&&>(f));
+  else group_for_cells<G>(P, x, y, z, cv, static_cast<F&&>(f));
+}
+
 // KERNEL_clc_mass_init_sph (functions_MASS.cuh:24-43): vol0 = vol =
 // (h/1.6)^dim, rho0 <- rho
 template <typename R>
@@ -68,10 +75,10 @@ int pack_r32(hipStream_t s, const SphView<R>& v, bool aux, bool vel) {
 }
 
 // KERNEL_clc_correction_KGC_3D_sph (functions_PREP2.cuh:452-568)
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_kgc(DevParams P, SphView<R> v) {
   typedef R T;
-  int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int n = v.n;
   if (v.itype[i] > 2 || v.ptype[i] > 1000) {
@@ -96,8 +103,15 @@ __global__ __launch_bounds__(kBlock) void k_kgc(DevParams P, SphView<R> v) {
     yz += use ? -mtd * dy * dz * rtd : (T)0;
     zz += use ? -mtd * dz * dz * rtd : (T)0;
   };
-  if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false>(v, i, false, term);
-  else for_nbrs4<true>(v, i, false, term);
+  if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false, G>(v, i, false, term);
+  else for_nbrs4<true, G>(v, i, false, term);
+  xx = group_sum<G>(xx);
+  yy = group_sum<G>(yy);
+  zz = group_sum<G>(zz);
+  xy = group_sum<G>(xy);
+  yz = group_sum<G>(yz);
+  zx = group_sum<G>(zx);
+  if (G > 1 && pair_sub<G>() != 0) return;
   T det = xx * (yy * zz - yz * yz);
   det -= xy * (xy * zz - yz * zx);
   det += zx * (xy * yz - yy * zx);
@@ -119,13 +133,13 @@ __global__ __launch_bounds__(kBlock) void k_kgc(DevParams P, SphView<R> v) {
 
 // KERNEL_clc_prep3D_coupling_sph (functions_PREP2.cuh:3190-3364): porosity
 // eps_i = 1 - sum_a V_a W_ia / sum_{j fluid} V_j W_ij and its rate.
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_porosity_sph(DevParams P, SphView<R> v, DemView d, CellView dc) {
   typedef R T;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;  // linear: work concentrates near walls/spheres
+  // linear: work concentrates near walls/spheres
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) / G;
   if (i >= v.n) return;
   if (v.itype[i] > 2) return;
-  v.dpor_prev[i] = v.dpor[i];
   const double hd = v.h[i];
   const T h = (T)hd, A = knl_tmpA<T>(P.kernel_type, P.dim, h);
   const double Rs = P.kappa * hd;
@@ -140,10 +154,10 @@ __global__ __launch_bounds__(kBlock) void k_porosity_sph(DevParams P, SphView<R>
     const bool use = on && pti <= 1000 && ptj <= 1000 && ptj == 1;
     flt += use ? (T)q.m / (T)q.rho * w : (T)0;
   };
-  if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false>(v, i, true, term);
-  else for_nbrs4<true>(v, i, true, term);
+  if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false, G>(v, i, true, term);
+  else for_nbrs4<true, G>(v, i, true, term);
   if (d.n > 0) {
-    for_cells(P, xi, yi, zi, dc, [&](int j) {
+    pair_cells<G>(P, xi, yi, zi, dc, [&](int j) {
       double rd = dist_exact(xi - d.x[j], yi - d.y[j], zi - d.z[j]) + 1e-20;
       if (!(rd < Rs)) return;
       if (!(pti <= 1000 && d.ptype[j] > 1000)) return;
@@ -159,6 +173,13 @@ __global__ __launch_bounds__(kBlock) void k_porosity_sph(DevParams P, SphView<R>
       dfz += dw * dz / r * (T)d.uz[j] * Vj;
     });
   }
+  flt = group_sum<G>(flt);
+  por = group_sum<G>(por);
+  dfx = group_sum<G>(dfx);
+  dfy = group_sum<G>(dfy);
+  dfz = group_sum<G>(dfz);
+  if (G > 1 && pair_sub<G>() != 0) return;
+  v.dpor_prev[i] = v.dpor[i];
   if (pti <= 1000) {
     v.por[i] = (T)1 - (por / (flt + (T)1e-20));
     v.dpor[i] = (dfx + dfy + dfz) / (flt + (T)1e-20);
@@ -169,10 +190,10 @@ __global__ __launch_bounds__(kBlock) void k_porosity_sph(DevParams P, SphView<R>
 // the same 32 B records, each kernel's own terms, neighbour rules (KGC takes
 // every list entry, the porosity only those without the eps flag) and
 // arithmetic, so the results are those of the two kernels.
-template <bool KGC>
+template <bool KGC, int G>
 __global__ __launch_bounds__(kBlock) void k_kgc_porosity(DevParams P, SphView<float> v, DemView d, CellView dc) {
   typedef float T;
-  const int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int n = v.n;
   const int iti = v.itype[i], pti = v.ptype[i];
@@ -180,14 +201,13 @@ __global__ __launch_bounds__(kBlock) void k_kgc_porosity(DevParams P, SphView<fl
   if (KGC && !krow)
     for (int c = 0; c < 6; c++) v.cm[c * n + i] = 0;
   if (iti > 2) return;
-  v.dpor_prev[i] = v.dpor[i];
   const double hd = v.h[i];
   const T h = (T)hd, ih = (T)(1.0 / hd), A = knl_tmpA<T>(P.kernel_type, P.dim, h), Rk = (T)(P.kappa * hd);
   const double Rs = P.kappa * hd;
   const double xi = v.x[i], yi = v.y[i], zi = v.z[i];
   T xx = 0, yy = 0, zz = 0, xy = 0, yz = 0, zx = 0;
   T flt = 0, por = 0, dfx = 0, dfy = 0, dfz = 0;
-  for_nbrs4_r32<false>(v, i, false, [&](const NbR& q, bool on) {
+  for_nbrs4_r32<false, G>(v, i, false, [&](const NbR& q, bool on) {
     const T dx = q.dx, dy = q.dy, dz = q.dz;
     const T r = sqrt(dx * dx + dy * dy + dz * dz);
     if (krow) {
@@ -207,7 +227,13 @@ __global__ __launch_bounds__(kBlock) void k_kgc_porosity(DevParams P, SphView<fl
     const bool usep = on && !q.flag && pti <= 1000 && q.pt <= 1000 && q.pt == 1;
     flt += usep ? q.m / q.rho * w : (T)0;
   });
-  if (krow) {
+  xx = group_sum<G>(xx);
+  yy = group_sum<G>(yy);
+  zz = group_sum<G>(zz);
+  xy = group_sum<G>(xy);
+  yz = group_sum<G>(yz);
+  zx = group_sum<G>(zx);
+  if (krow && (G == 1 || pair_sub<G>() == 0)) {
     T det = xx * (yy * zz - yz * yz);
     det -= xy * (xy * zz - yz * zx);
     det += zx * (xy * yz - yy * zx);
@@ -227,7 +253,7 @@ __global__ __launch_bounds__(kBlock) void k_kgc_porosity(DevParams P, SphView<fl
     v.cm[3 * n + i] = c3; v.cm[4 * n + i] = c4; v.cm[5 * n + i] = c5;
   }
   if (d.n > 0) {
-    for_cells(P, xi, yi, zi, dc, [&](int j) {
+    pair_cells<G>(P, xi, yi, zi, dc, [&](int j) {
       double rd = dist_exact(xi - d.x[j], yi - d.y[j], zi - d.z[j]) + 1e-20;
       if (!(rd < Rs)) return;
       if (!(pti <= 1000 && d.ptype[j] > 1000)) return;
@@ -243,6 +269,13 @@ __global__ __launch_bounds__(kBlock) void k_kgc_porosity(DevParams P, SphView<fl
       dfz += dw * dz / r * (T)d.uz[j] * Vj;
     });
   }
+  flt = group_sum<G>(flt);
+  por = group_sum<G>(por);
+  dfx = group_sum<G>(dfx);
+  dfy = group_sum<G>(dfy);
+  dfz = group_sum<G>(dfz);
+  if (G > 1 && pair_sub<G>() != 0) return;
+  v.dpor_prev[i] = v.dpor[i];
   if (pti <= 1000) {
     v.por[i] = (T)1 - (por / (flt + (T)1e-20));
     v.dpor[i] = (dfx + dfy + dfz) / (flt + (T)1e-20);
@@ -271,10 +304,10 @@ __global__ void k_prep_prep(DevParams P, SphView<R> v) {
 
 // KERNEL_clc_prep3D_sph (functions_PREP2.cuh:1985-2227): Shepard filter and
 // the Antuono density gradient.
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_prep(DevParams P, SphView<R> v) {
   typedef R T;
-  int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   if (v.itype[i] > 2 || v.ptype[i] > 1000) return;
   const int n = v.n;
@@ -303,8 +336,13 @@ __global__ __launch_bounds__(kBlock) void k_prep(DevParams P, SphView<R> v) {
       rz += use ? c * gz : (T)0;
     }
   };
-  if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false>(v, i, true, term);
-  else for_nbrs4<true>(v, i, true, term);
+  if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false, G>(v, i, true, term);
+  else for_nbrs4<true, G>(v, i, true, term);
+  flt = group_sum<G>(flt);
+  rx = group_sum<G>(rx);
+  ry = group_sum<G>(ry);
+  rz = group_sum<G>(rz);
+  if (G > 1 && pair_sub<G>() != 0) return;
   if (P.filt_step) v.flt_s[i] = flt;
   if (anto) {
     v.grx[i] = rx;
@@ -320,22 +358,23 @@ __global__ __launch_bounds__(kBlock) void k_prep(DevParams P, SphView<R> v) {
 __device__ inline bool flux_receiver(const DevParams& P, int pt, int it, int bt) {
   return it <= 2 && !(P.open_boundary > 0 && bt > 0) && pt > 0 && pt < 1000;
 }
-template <typename R>
+template <typename R, int G>
 __global__ void k_flux_walls(DevParams P, SphView<R> v) {
-  const int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   double S = 0;
   const double x = v.x[i], y = v.y[i], z = v.z[i];
   const double* b = P.heat_flux_box;
   if (v.ptype[i] == 0 && x >= b[0] && y >= b[1] && z >= b[2] && x <= b[3] && y <= b[4] && z <= b[5]) {
     const double h = v.h[i], A = knl_tmpA<double>(P.kernel_type, P.dim, h);
-    for_nbrs4<false>(v, i, false, [&](const Nb<R>& q, bool on) {
+    for_nbrs4<false, G>(v, i, false, [&](const Nb<R>& q, bool on) {
       const bool use = on && flux_receiver(P, q.pt, v.itype[q.j], v.btype[q.j]);
       const double r = sqrt(q.dx * q.dx + q.dy * q.dy + q.dz * q.dz);
       S += use ? q.m / q.rho * knl_w<double>(P.kernel_type, A, h, r) : 0.0;
     });
   }
-  v.flux_s[i] = S;
+  S = group_sum<G>(S);
+  if (G == 1 || pair_sub<G>() == 0) v.flux_s[i] = S;
 }
 
 // viscosity() and conductivity() of every SPH particle at its temperature
@@ -393,10 +432,10 @@ __device__ __host__ inline bool packed_geometry(const DevParams& P) {
 // KERNEL_advection_force3D_sph (functions_PPE2.cuh:1251-1607): viscous,
 // artificial viscosity, Eulerian advection, conduction, gravity and the
 // pressure-gradient force density used by the coupling.
-template <typename R, bool FLUX>
+template <typename R, bool FLUX, int G>
 __global__ __launch_bounds__(kBlock) void k_advection(DevParams P, SphView<R> v) {
   typedef R T;
-  int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int pti = v.ptype[i];
   if (v.itype[i] > 2) return;
@@ -510,8 +549,21 @@ __global__ __launch_bounds__(kBlock) void k_advection(DevParams P, SphView<R> v)
   // the difference-form pressure gradient carries no hydrostatic offset, so
   // with FP32 fields the position records give the geometry; the symmetric
   // form keeps FP64 geometry, read from the packed records
-  if (packed_geometry<R>(P)) for_nbrs4_pk<true>(v, i, true, term);
-  else for_nbrs4<true>(v, i, true, term);
+  if (packed_geometry<R>(P)) for_nbrs4_pk<true, G>(v, i, true, term);
+  else for_nbrs4<true, G>(v, i, true, term);
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  tz = group_sum<G>(tz);
+  ex = group_sum<G>(ex);
+  ey = group_sum<G>(ey);
+  ez = group_sum<G>(ez);
+  Rc = group_sum<G>(Rc);
+  et = group_sum<G>(et);
+  px = group_sum<G>(px);
+  py = group_sum<G>(py);
+  pz = group_sum<G>(pz);
+  fl = group_sum<G>(fl);
+  if (G > 1 && pair_sub<G>() != 0) return;
   if (P.fg_solve) tz += -(T)P.gravity;
   v.fx[i] = tx - ex;
   v.fy[i] = ty - ey;
@@ -733,10 +785,10 @@ __global__ __launch_bounds__(kBlock) void k_surface(DevParams P, SphView<R> v) {
   v.surf[i] = surf ? 1 : 0;
 }
 
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_pressure_force(DevParams P, SphView<R> v) {
   typedef double T;  // FP64 pair sums: see the note on pressure-gradient cancellation
-  int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int pti = v.ptype[i];
   if (v.itype[i] > 2) return;
@@ -769,9 +821,13 @@ __global__ __launch_bounds__(kBlock) void k_pressure_force(DevParams P, SphView<
     // the difference form carries no hydrostatic offset, so geometry from
     // the position records is enough; the symmetric form keeps FP64
     // geometry, read from the packed records
-    if (packed_geometry<R>(P)) for_nbrs4_pk<false>(v, i, true, term);
-    else for_nbrs4<true>(v, i, true, term);
+    if (packed_geometry<R>(P)) for_nbrs4_pk<false, G>(v, i, true, term);
+    else for_nbrs4<true, G>(v, i, true, term);
   }
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  tz = group_sum<G>(tz);
+  if (G > 1 && pair_sub<G>() != 0) return;
   v.fpx[i] = (R)tx;
   v.fpy[i] = (R)ty;
   v.fpz[i] = (R)tz;
@@ -842,10 +898,10 @@ __global__ void k_corrector(DevParams P, SphView<R> v) {
 
 // KERNEL_xsph3D_sph + KERNEL_xsph3D_calc_sph (functions_TIME.cuh:1735-1850,
 // 1985-1997): Shepard-normalised XSPH velocity and temperature smoothing
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_xsph(DevParams P, SphView<R> v) {
   typedef R T;
-  int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int pti = v.ptype[i];
   if (v.itype[i] != 1 || pti > 1000 || pti == 0 || pti == 9) return;
@@ -867,8 +923,14 @@ __global__ __launch_bounds__(kBlock) void k_xsph(DevParams P, SphView<R> v) {
     tt += use ? (T)0.01 * c * vj * ((T)q.temp - ti) * w : (T)0;
     fl += use ? vj * w : (T)0;
   };
-  if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<true>(v, i, false, term);
-  else for_nbrs4<true>(v, i, false, term);
+  if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<true, G>(v, i, false, term);
+  else for_nbrs4<true, G>(v, i, false, term);
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  tz = group_sum<G>(tz);
+  tt = group_sum<G>(tt);
+  fl = group_sum<G>(fl);
+  if (G > 1 && pair_sub<G>() != 0) return;
   const T on = (T)(pti > 0);
   v.xsx[i] = (uxi + tx / fl) * on;
   v.xsy[i] = (uyi + ty / fl) * on;
@@ -974,12 +1036,14 @@ template int monitor_max<double>(hipStream_t, int, const int*, const int*, const
 template <typename R> int sph_mass_init(hipStream_t s, const DevParams& P, const SphView<R>& v) { LAUNCH(k_mass_init, P, v); }
 template <typename R> int sph_kgc(hipStream_t s, const DevParams& P, const SphView<R>& v) {
   TRY(pack_r32(s, v, false, false));
-  LAUNCH(k_kgc, P, v);
+  return pair_launch(v.n, [&](auto g, int grid) { k_kgc<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
 }
 template <typename R>
 int sph_porosity(hipStream_t s, const DevParams& P, const SphView<R>& v, const DemView& d, const CellView& dc) {
   TRY(pack_r32(s, v, false, false));
-  LAUNCH(k_porosity_sph, P, v, d, dc);
+  return pair_launch(v.n, [&](auto g, int grid) {
+    k_porosity_sph<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v, d, dc);
+  });
 }
 template <typename R>
 int sph_kgc_porosity(hipStream_t s, const DevParams& P, const SphView<R>& v, const DemView& d, const CellView& dc,
@@ -987,45 +1051,45 @@ int sph_kgc_porosity(hipStream_t s, const DevParams& P, const SphView<R>& v, con
   if constexpr (std::is_same<R, float>::value) {
     if (v.n <= 0) return 0;
     TRY(pack_r32(s, v, false, false));
-    if (kgc) k_kgc_porosity<true><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v, d, dc);
-    else k_kgc_porosity<false><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v, d, dc);
-    HIP_TRY(hipGetLastError());
-    return 0;
+    // one lane for large runs: the spheres around a particle are few, and lanes
+    // that share them idle (914 us with one, 1010 with two at 1.16 M)
+    return pair_launch(v.n, v.n >= 500000 ? 1 : pair_lanes(v.n), [&](auto g, int grid) {
+      constexpr int G = decltype(g)::value;
+      if (kgc) k_kgc_porosity<true, G><<<grid, kBlock, 0, s>>>(P, v, d, dc);
+      else k_kgc_porosity<false, G><<<grid, kBlock, 0, s>>>(P, v, d, dc);
+    });
   } else {
     if (kgc) TRY(sph_kgc(s, P, v));
     return sph_porosity(s, P, v, d, dc);
   }
 }
+template <typename R> int sph_prep_sums(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  TRY(pack_r32(s, v, P.delsph == 2, false));
+  return pair_launch(v.n, [&](auto g, int grid) { k_prep<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
+}
 template <typename R> int sph_prep(hipStream_t s, const DevParams& P, const SphView<R>& v) {
   if (v.n > 0) {
     k_prep_prep<R><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
     HIP_TRY(hipGetLastError());
-    TRY(pack_r32(s, v, P.delsph == 2, false));
-    k_prep<R><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
-    HIP_TRY(hipGetLastError());
+    return sph_prep_sums<R>(s, P, v);
   }
   return 0;
 }
 template <typename R> int sph_prep_prep(hipStream_t s, const DevParams& P, const SphView<R>& v) { LAUNCH(k_prep_prep, P, v); }
-template <typename R> int sph_prep_sums(hipStream_t s, const DevParams& P, const SphView<R>& v) {
-  TRY(pack_r32(s, v, P.delsph == 2, false));
-  LAUNCH(k_prep, P, v);
-}
 template <typename R> int sph_advection(hipStream_t s, const DevParams& P, const SphView<R>& v) {
   if (v.n > 0) {
     if (packed_geometry<R>(P)) k_pack_records<R, true><<<grid_for(v.n), kBlock, 0, s>>>(v, P.heat_flux != 0.0);
-    if (P.heat_flux != 0.0) k_advection<R, true><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
-    else k_advection<R, false><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
-    HIP_TRY(hipGetLastError());
+    return pair_launch(v.n, [&](auto g, int grid) {
+      constexpr int G = decltype(g)::value;
+      if (P.heat_flux != 0.0) k_advection<R, true, G><<<grid, kBlock, 0, s>>>(P, v);
+      else k_advection<R, false, G><<<grid, kBlock, 0, s>>>(P, v);
+    });
   }
   return 0;
 }
 template <typename R> int sph_flux_walls(hipStream_t s, const DevParams& P, const SphView<R>& v) {
-  if (v.n > 0 && P.heat_flux != 0.0) {
-    k_flux_walls<R><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
-    HIP_TRY(hipGetLastError());
-  }
-  return 0;
+  if (P.heat_flux == 0.0) return 0;
+  return pair_launch(v.n, [&](auto g, int grid) { k_flux_walls<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
 }
 template <typename R> int sph_neumann(hipStream_t s, const DevParams& P, const SphView<R>& v, const CellView& cv) {
   const double m = fmax(fmax(fmax(fabs(P.x_min), fabs(P.x_max)), fmax(fabs(P.y_min), fabs(P.y_max))),
@@ -1049,9 +1113,8 @@ template <typename R> int sph_props(hipStream_t s, const DevParams& P, const Sph
 template <typename R> int sph_pressure_force(hipStream_t s, const DevParams& P, const SphView<R>& v) {
   if (v.n <= 0) return 0;
   if (P.fp_solve && packed_geometry<R>(P)) k_pack_records<R, false><<<grid_for(v.n), kBlock, 0, s>>>(v, false);
-  k_pressure_force<R><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
-  HIP_TRY(hipGetLastError());
-  return 0;
+  return pair_launch(v.n,
+                     [&](auto g, int grid) { k_pressure_force<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
 }
 template <typename R>
 int sph_open_boundary(hipStream_t s, const DevParams& P, const SphView<R>& v, const CellView& cv,
@@ -1068,16 +1131,13 @@ template <typename R> int sph_corrector(hipStream_t s, const DevParams& P, const
 template <typename R> int sph_xsph_only(hipStream_t s, const DevParams& P, const SphView<R>& v) {
   if (v.n > 0) {
     TRY(pack_r32(s, v, false, true));
-    k_xsph<R><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
-    HIP_TRY(hipGetLastError());
+    return pair_launch(v.n, [&](auto g, int grid) { k_xsph<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
   }
   return 0;
 }
 template <typename R> int sph_xsph(hipStream_t s, const DevParams& P, const SphView<R>& v) {
   if (v.n > 0) {
-    TRY(pack_r32(s, v, false, true));
-    k_xsph<R><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
-    HIP_TRY(hipGetLastError());
+    TRY(sph_xsph_only<R>(s, P, v));
     k_xsph_calc<R><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
     HIP_TRY(hipGetLastError());
   }

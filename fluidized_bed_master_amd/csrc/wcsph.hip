@@ -105,10 +105,10 @@ __global__ void k_mass_update(DevParams P, SphView<R> v) {
 // velocity divergence, the eps-advection term of Eulerian particles and
 // the delta-SPH diffusion (Molteni, or Antuono with the density gradient).
 // FP64 sums: drho integrates into rho, which the Tait EOS raises to gamma.
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_continuity(DevParams P, SphView<R> v) {
   typedef double T;
-  int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   if (v.itype[i] > 2 || v.ptype[i] > 1000) return;
   if (P.open_boundary > 0 && v.btype[i] > 0) return;
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(kBlock) void k_continuity(DevParams P, SphView<R> v
   const T el = P.eulerian ? 0.0 : 1.0;
   const bool dsph = P.delsph > 0, anto = P.delsph == 2;
   T tx = 0, ty = 0, tz = 0, px = 0, py = 0, pz = 0, tR = 0;
-  for_nbrs4<true>(v, i, true, [&](const Nb<R>& q, bool on) {
+  for_nbrs4<true, G>(v, i, true, [&](const Nb<R>& q, bool on) {
     const bool use = on && q.pt <= 1000;
     const T dx = (T)q.dx, dy = (T)q.dy, dz = (T)q.dz;
     const T r = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
@@ -149,6 +149,14 @@ __global__ __launch_bounds__(kBlock) void k_continuity(DevParams P, SphView<R> v
       tR += use ? trr : 0.0;
     }
   });
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  tz = group_sum<G>(tz);
+  px = group_sum<G>(px);
+  py = group_sum<G>(py);
+  pz = group_sum<G>(pz);
+  tR = group_sum<G>(tR);
+  if (G > 1 && pair_sub<G>() != 0) return;
   v.drho[i] = (R)((tx + ty + tz) + pori * (px + py + pz) * (1 - el) + tR * (dsph ? 1.0 : 0.0));
 }
 
@@ -169,10 +177,10 @@ __global__ void k_eos(DevParams P, SphView<R> v) {
 // Eulerian advection term (interface, repulsive, surface-tension,
 // Boussinesq and concentration terms are off in this build).  Geometry and
 // the pressure term in FP64, as in the ISPH force kernels.
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<R> v) {
   typedef R T;
-  int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   if (v.itype[i] != 1 || v.ptype[i] > 1000) return;
   const int pti = v.ptype[i];
@@ -193,7 +201,7 @@ __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<
   const bool euler = el < (T)1;
   T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0;
   double ptx = 0, pty = 0, ptz = 0, px = 0, py = 0, pz = 0;
-  for_nbrs4(v, i, true, [&](const Nb<R>& q, bool on) {
+  for_nbrs4<false, G>(v, i, true, [&](const Nb<R>& q, bool on) {
     const bool use = on && q.pt <= 1000;
     const double dxd = q.dx, dyd = q.dy, dzd = q.dz;
     const double rd = sqrt(dxd * dxd + dyd * dyd + dzd * dzd) + 1e-20;
@@ -257,6 +265,21 @@ __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<
       }
     }
   });
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  tz = group_sum<G>(tz);
+  Rc = group_sum<G>(Rc);
+  ex = group_sum<G>(ex);
+  ey = group_sum<G>(ey);
+  ez = group_sum<G>(ez);
+  et = group_sum<G>(et);
+  ptx = group_sum<G>(ptx);
+  pty = group_sum<G>(pty);
+  ptz = group_sum<G>(ptz);
+  px = group_sum<G>(px);
+  py = group_sum<G>(py);
+  pz = group_sum<G>(pz);
+  if (G > 1 && pair_sub<G>() != 0) return;
   // pressure first, then the other terms, in the reference's per-pair order
   // of one accumulator; FP32 rounding of the sum of both is below the tests'
   // tolerance
@@ -337,9 +360,14 @@ int wc_volume_mass(hipStream_t s, const DevParams& P, const SphView<R>& v, const
   HIP_TRY(hipGetLastError());
   return 0;
 }
-template <typename R> int wc_continuity(hipStream_t s, const DevParams& P, const SphView<R>& v) { WC_LAUNCH(k_continuity, P, v); }
+template <typename R> int wc_continuity(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  return pair_launch(v.n, [&](auto g, int grid) { k_continuity<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
+}
 template <typename R> int wc_eos(hipStream_t s, const DevParams& P, const SphView<R>& v) { WC_LAUNCH(k_eos, P, v); }
-template <typename R> int wc_interaction(hipStream_t s, const DevParams& P, const SphView<R>& v) { WC_LAUNCH(k_wc_interaction, P, v); }
+template <typename R> int wc_interaction(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  return pair_launch(v.n,
+                     [&](auto g, int grid) { k_wc_interaction<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
+}
 template <typename R> int wc_corrector(hipStream_t s, const DevParams& P, const SphView<R>& v) { WC_LAUNCH(k_wc_corrector, P, v); }
 
 #define WC_INST(R)                                                                                           \

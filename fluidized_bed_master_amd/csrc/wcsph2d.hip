@@ -30,15 +30,15 @@ __device__ inline double dist2d(double dx, double dy) {
 // 2x2 moment matrix sum_j -m_j dW (x_ij x_ij^T) / (rho_j r) over r > 0,
 // identity when |det| <= Min_det.  Stored in the symmetric 3x3 slots
 // (xx, xy, 0, yy, 0, 0) so the 3D correction applies it to (gx, gy, 0).
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_kgc2d(DevParams P, SphView<R> v) {
-  const int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   if (v.itype[i] > 2 || v.ptype[i] > 1000) return;
   const int n = v.n;
   const double h = v.h[i], A = knl_tmpA<double>(P.kernel_type, P.dim, h);
   double xx = 0, xy = 0, yy = 0;
-  for_nbrs4(v, i, false, [&](const Nb<R>& q, bool on) {
+  for_nbrs4<false, G>(v, i, false, [&](const Nb<R>& q, bool on) {
     const double dx = q.dx, dy = q.dy;
     const double r = dist2d(dx, dy);
     const bool use = on && q.pt <= 1000 && r > 0;
@@ -50,6 +50,10 @@ __global__ __launch_bounds__(kBlock) void k_kgc2d(DevParams P, SphView<R> v) {
     t = -mtd * dy * dx; t *= rtd; xy += use ? t : 0.0;
     t = -mtd * dy * dy; t *= rtd; yy += use ? t : 0.0;
   });
+  xx = group_sum<G>(xx);
+  xy = group_sum<G>(xy);
+  yy = group_sum<G>(yy);
+  if (G > 1 && pair_sub<G>() != 0) return;
   const double det = xx * yy - xy * xy;
   double a = 1, b = 0, d = 1;
   if (fabs(det) > 1e-4) {  // Min_det (Parameters.cuh:125)
@@ -71,9 +75,9 @@ __global__ __launch_bounds__(kBlock) void k_kgc2d(DevParams P, SphView<R> v) {
 // due, reference density m / (h / 1.6)^2 every step, the Antuono density
 // gradient -(rho_j - rho_i) m_j / rho_j grad~W; porosity 1 (no spheres in
 // 2D).  Turbulence, p_type switching and surface-tension normals are off.
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_prep2d(DevParams P, SphView<R> v) {
-  const int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   if (v.itype[i] > 2) return;
   v.por[i] = 1.0;
@@ -83,7 +87,7 @@ __global__ __launch_bounds__(kBlock) void k_prep2d(DevParams P, SphView<R> v) {
   const double rhoi = v.rho[i];
   const bool anto = P.delsph == 2;
   double flt = 0, rx = 0, ry = 0;
-  for_nbrs4(v, i, true, [&](const Nb<R>& q, bool on) {
+  for_nbrs4<false, G>(v, i, true, [&](const Nb<R>& q, bool on) {
     const bool use = on && q.pt <= 1000;
     const double dx = q.dx, dy = q.dy;
     const double r = dist2d(dx, dy) + 1e-20;
@@ -97,6 +101,10 @@ __global__ __launch_bounds__(kBlock) void k_prep2d(DevParams P, SphView<R> v) {
       ry += use ? -(rhoj - rhoi) * (mj / rhoj) * gy : 0.0;
     }
   });
+  flt = group_sum<G>(flt);
+  rx = group_sum<G>(rx);
+  ry = group_sum<G>(ry);
+  if (G > 1 && pair_sub<G>() != 0) return;
   const double hv = h / P.h_over_dx;
   v.rho_ref[i] = v.m[i] / (hv * hv);
   if (P.filt_step) v.flt_s[i] = (R)flt;
@@ -116,15 +124,15 @@ __device__ inline bool noslip_wall(int pt) {
   const uint32_t u = (uint32_t)pt;
   return !(u > 0 && u != (uint32_t)kMoving);
 }
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_boundary2d(DevParams P, SphView<R> v) {
-  const int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int pti = v.ptype[i];
   if (v.itype[i] > 2 || pti > 1000 || !noslip_wall(pti)) return;
   const double h = v.h[i], A = knl_tmpA<double>(P.kernel_type, P.dim, h);
-  double tx = 0, ty = 0, fl = 1.0e-10;
-  for_nbrs4(v, i, true, [&](const Nb<R>& q, bool on) {
+  double tx = 0, ty = 0, fl = 0;
+  for_nbrs4<false, G>(v, i, true, [&](const Nb<R>& q, bool on) {
     const bool use = on && q.pt <= 1000 && (uint32_t)q.pt > 0;
     const double r = dist2d(q.dx, q.dy) + 1e-20;
     const double w = knl_w<double>(P.kernel_type, A, h, r);
@@ -132,6 +140,10 @@ __global__ __launch_bounds__(kBlock) void k_boundary2d(DevParams P, SphView<R> v
     ty += use ? (double)q.uy * w : 0.0;
     fl += use ? w : 0.0;
   });
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  fl = group_sum<G>(fl) + 1.0e-10;
+  if (G > 1 && pair_sub<G>() != 0) return;
   const double mv = pti == kMoving ? 1.0 : 0.0;
   v.xsx[i] = (R)(2 * (double)v.ux[i] * mv - tx / fl);
   v.xsy[i] = (R)(2 * (double)v.uy[i] * mv - ty / fl);
@@ -150,9 +162,9 @@ __global__ void k_boundary2d_apply(SphView<R> v) {
 // included with their velocity taken as 0: the divergence
 // sum m_j (rho_i / rho_j) (u_i - u_j) . grad~W times rho_i / rho_ref_i, and
 // delta-SPH on rho_j - rho_i (Molteni, or Antuono with the gradients).
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_continuity2d(DevParams P, SphView<R> v) {
-  const int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int pti = v.ptype[i];
   if (v.itype[i] > 2 || pti > 1000) return;
@@ -162,7 +174,7 @@ __global__ __launch_bounds__(kBlock) void k_continuity2d(DevParams P, SphView<R>
   const double rhoi = v.rho[i], gxi = (double)v.grx[i], gyi = (double)v.gry[i];
   const bool dsph = P.delsph > 0, anto = P.delsph == 2;
   double tx = 0, ty = 0, tR = 0;
-  for_nbrs4(v, i, true, [&](const Nb<R>& q, bool on) {
+  for_nbrs4<false, G>(v, i, true, [&](const Nb<R>& q, bool on) {
     const bool use = on && q.pt <= 1000;
     const double dx = q.dx, dy = q.dy;
     const double r = dist2d(dx, dy) + 1e-20;
@@ -183,6 +195,10 @@ __global__ __launch_bounds__(kBlock) void k_continuity2d(DevParams P, SphView<R>
       tR += use ? tr : 0.0;
     }
   });
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  tR = group_sum<G>(tR);
+  if (G > 1 && pair_sub<G>() != 0) return;
   v.drho[i] = (R)((tx + ty) * (rhoi / v.rho_ref[i]) + tR * (dsph ? 1.0 : 0.0));
 }
 
@@ -191,9 +207,9 @@ __global__ __launch_bounds__(kBlock) void k_continuity2d(DevParams P, SphView<R>
 // (no eps factor), artificial viscosity, gravity on y and conduction
 // divided by m_i, as the reference writes them; interface, repulsive,
 // surface-tension, Boussinesq and concentration terms are off.
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_interaction2d(DevParams P, SphView<R> v) {
-  const int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int pti = v.ptype[i];
   if (v.itype[i] != 1 || pti > 1000) return;
@@ -210,7 +226,7 @@ __global__ __launch_bounds__(kBlock) void k_interaction2d(DevParams P, SphView<R
     eta = 0.001 * h;
   }
   double tx = 0, ty = 0, Rc = 0, pgx = 0, pgy = 0;
-  for_nbrs4(v, i, true, [&](const Nb<R>& q, bool on) {
+  for_nbrs4<false, G>(v, i, true, [&](const Nb<R>& q, bool on) {
     const bool use = on && q.pt <= 1000;
     const double dx = q.dx, dy = q.dy;
     const double r = dist2d(dx, dy) + 1e-20;
@@ -258,6 +274,12 @@ __global__ __launch_bounds__(kBlock) void k_interaction2d(DevParams P, SphView<R
       Rc += use ? H : 0.0;
     }
   });
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  Rc = group_sum<G>(Rc);
+  pgx = group_sum<G>(pgx);
+  pgy = group_sum<G>(pgy);
+  if (G > 1 && pair_sub<G>() != 0) return;
   if (P.fg_solve) ty += -P.gravity;
   v.fx[i] = (R)tx;
   v.fy[i] = (R)ty;
@@ -319,9 +341,9 @@ __global__ void k_time_update2d(DevParams P, SphView<R> v) {
 // m_j / rho_j (u_j - u_i) W / flt_s_i) dt for fluid, x0 for walls, x0 + u dt
 // for moving walls; corrected velocities, predicted positions and
 // densities; r < kappa h without the 1e-20 (flagged entries count).
-template <typename R>
+template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_xsph2d(DevParams P, SphView<R> v) {
-  const int i = particle_index();
+  const int i = pair_particle<G>();
   if (i >= v.n) return;
   const int pti = v.ptype[i];
   if (v.itype[i] != 1 || pti > 1000) return;
@@ -331,7 +353,7 @@ __global__ __launch_bounds__(kBlock) void k_xsph2d(DevParams P, SphView<R> v) {
   const double uxi = v.ux[i], uyi = v.uy[i], fl = v.flt_s[i], c = P.c_xsph;
   double tx = 0, ty = 0;
   const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
-  for (int k = 0; k < cnt; k++) {
+  for (int k = pair_sub<G>(); k < cnt; k += G) {
     const int j = (int)(v.nbr[nbr_slot(k, i, n)] & ~kNbrFlag);
     if (v.ptype[j] > 1000) continue;
     const double r = dist2d(xi - v.xp[j], yi - v.yp[j]);
@@ -341,6 +363,9 @@ __global__ __launch_bounds__(kBlock) void k_xsph2d(DevParams P, SphView<R> v) {
     tx += c * mj / rhoj * (-uxi + (double)v.ux[j]) * w / fl;
     ty += c * mj / rhoj * (-uyi + (double)v.uy[j]) * w / fl;
   }
+  tx = group_sum<G>(tx);
+  ty = group_sum<G>(ty);
+  if (G > 1 && pair_sub<G>() != 0) return;
   const double dt = P.dt_sph;
   if (pti == kMoving) {
     v.x[i] = v.x0[i] + uxi * dt;
@@ -363,19 +388,29 @@ __global__ __launch_bounds__(kBlock) void k_xsph2d(DevParams P, SphView<R> v) {
     return 0;                                                \
   } while (0)
 
-template <typename R> int wc2_kgc(hipStream_t s, const DevParams& P, const SphView<R>& v) { W2_LAUNCH(k_kgc2d, P, v); }
-template <typename R> int wc2_prep(hipStream_t s, const DevParams& P, const SphView<R>& v) { W2_LAUNCH(k_prep2d, P, v); }
+template <typename R> int wc2_kgc(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  return pair_launch(v.n, [&](auto g, int grid) { k_kgc2d<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
+}
+template <typename R> int wc2_prep(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  return pair_launch(v.n, [&](auto g, int grid) { k_prep2d<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
+}
 template <typename R> int wc2_boundary(hipStream_t s, const DevParams& P, const SphView<R>& v) {
   if (v.n <= 0) return 0;
-  k_boundary2d<R><<<grid_xcd(v.n), kBlock, 0, s>>>(P, v);
+  TRY(pair_launch(v.n, [&](auto g, int grid) { k_boundary2d<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); }));
   k_boundary2d_apply<R><<<grid_xcd(v.n), kBlock, 0, s>>>(v);
   HIP_TRY(hipGetLastError());
   return 0;
 }
-template <typename R> int wc2_continuity(hipStream_t s, const DevParams& P, const SphView<R>& v) { W2_LAUNCH(k_continuity2d, P, v); }
-template <typename R> int wc2_interaction(hipStream_t s, const DevParams& P, const SphView<R>& v) { W2_LAUNCH(k_interaction2d, P, v); }
+template <typename R> int wc2_continuity(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  return pair_launch(v.n, [&](auto g, int grid) { k_continuity2d<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
+}
+template <typename R> int wc2_interaction(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  return pair_launch(v.n, [&](auto g, int grid) { k_interaction2d<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
+}
 template <typename R> int wc2_time_update(hipStream_t s, const DevParams& P, const SphView<R>& v) { W2_LAUNCH(k_time_update2d, P, v); }
-template <typename R> int wc2_xsph(hipStream_t s, const DevParams& P, const SphView<R>& v) { W2_LAUNCH(k_xsph2d, P, v); }
+template <typename R> int wc2_xsph(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  return pair_launch(v.n, [&](auto g, int grid) { k_xsph2d<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
+}
 
 #define W2_INST(R)                                                                \
   template int wc2_kgc<R>(hipStream_t, const DevParams&, const SphView<R>&);        \

@@ -1,0 +1,78 @@
+"""The pair kernels' lane counts (eight lanes per particle for small runs, then
+four, two and one): whole steps against the FP64 oracle at sizes on both sides
+of each step of the rule, with the spheres' and walls' terms on."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from fluidized_bed_master_amd import abi, configs
+from tests.helpers import compare_fields
+
+pytestmark = pytest.mark.gpu
+
+# FP64: the terms are the oracle's and only the order of ~81 of them changes,
+# 81 * 2^-53 ~ 1e-14 per sum, amplified to ~1e-11 by the pressure gradient's
+# cancellation (H / h ~ 1e3): 1e-9 as in the stage tests.  Mixed: 1e-5, theirs.
+TOL = {abi.PREC_FP64: 1e-9, abi.PREC_MIXED: 1e-5}
+
+
+def _compare(g, o, tol, where):
+    a1, _, a3 = g.get_particles(abi.SPH)
+    b1, _, b3 = o.get_particles(abi.SPH)
+    compare_fields(a1, b1, ["rho", "m", "DEMpor", "flt_s", "grad_rhoz", "pres", "ux", "uy", "uz", "temp"], tol, where)
+    compare_fields(a3, b3, ["Cm", "ftotalx", "ftotaly", "ftotalz", "fpz"], tol, where + "/p3")
+
+
+@pytest.mark.parametrize("prec", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("n", [(22, 21, 23), (32, 28, 30), (37, 41, 36), (70, 66, 62)],
+                         ids=["8_lanes", "4_lanes", "2_lanes", "2_lanes_large"])
+def test_isph_step_at_every_lane_count(n, prec):
+    from fluidized_bed_master_amd.sophia import Sophia
+    from oracle.oracle import Oracle
+    p, parts = configs.isph_dem_column(*n, 1.0e-3, d_dem=2.0e-3, dem_height=0.4e-3 * n[2], phi=0.6, jitter=0.02, seed=8,
+                                       u_noise=0.05, dem_u_noise=0.05)
+    configs.heated(p, parts)
+    g, o = Sophia(p, parts, precision=prec), Oracle(p, parts)
+    opts = abi.ppe_opts(method=abi.PPE_JACOBI)
+    g.step(opts)
+    o.step(opts)
+    _compare(g, o, TOL[prec], str(n))
+    d, b, r = g.get_ppe_system()
+    do, bo, ro = o.get_ppe_system()
+    assert np.array_equal(r, ro)
+    x = np.random.default_rng(2).normal(0, 1, len(r)) * ro
+    y, yo = g.ppe_apply(x), o.ppe_apply(x)
+    assert np.abs(y - yo).max() <= TOL[prec] * np.abs(yo).max()
+    g.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(150, 130), (230, 170), (400, 220)], ids=["8_lanes", "4_lanes", "2_lanes"])
+def test_2d_step_at_every_lane_count(nx, ny):
+    from fluidized_bed_master_amd.sophia import Sophia
+    from oracle.oracle import Oracle
+    p, parts = configs.dam_break_2d(nx, ny, tank=(2 * nx, ny + 10), u_noise=0.05)
+    g, o = Sophia(p, parts, precision=abi.PREC_FP64), Oracle(p, parts)
+    for _ in range(2):
+        g.step()
+        o.step()
+    a1, _, a3 = g.get_particles(abi.SPH)
+    b1, _, b3 = o.get_particles(abi.SPH)
+    compare_fields(a1, b1, ["x", "y", "ux", "uy", "rho", "pres", "flt_s", "grad_rhox"], 1e-9, "2d")
+    compare_fields(a3, b3, ["drho", "ftotalx", "ftotaly"], 1e-9, "2d/p3")
+    g.close()
+
+
+@pytest.mark.parametrize("n", [(20, 20, 30), (34, 30, 36), (40, 44, 40)], ids=["8_lanes", "4_lanes", "2_lanes"])
+def test_wcsph_step_at_every_lane_count(n):
+    from fluidized_bed_master_amd.sophia import Sophia
+    from oracle.oracle import Oracle
+    p, parts = configs.wcsph_dem_column(*n, con=1)
+    g, o = Sophia(p, parts, precision=abi.PREC_FP64), Oracle(p, parts)
+    g.step()
+    o.step()
+    a1, _, a3 = g.get_particles(abi.SPH)
+    b1, _, b3 = o.get_particles(abi.SPH)
+    compare_fields(a1, b1, ["ux", "uy", "uz", "rho", "pres", "flt_s", "DEMpor", "temp"], 1e-9, "wcsph")
+    compare_fields(a3, b3, ["drho", "ftotalx", "ftotaly", "ftotalz", "dtemp"], 1e-9, "wcsph/p3")
+    g.close()
