@@ -159,7 +159,7 @@ __global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, double
     int e0;
     const int m = win_stage(
         o, s0, i1, S, &e0, [](int x, int y, int z, int) { return (int)agg_parity(x, y, z); },
-        [](int par, int) { return (uint8_t)par; });
+        [](int par, int, int) { return (uint8_t)par; });
     const int i = s0 + (int)threadIdx.x;
     s0 = m;
     if (i >= m) continue;
@@ -606,14 +606,14 @@ int coarse_setup(hipStream_t s, CoarseWork& c, const PpeWork& w, bool* usable, T
 
 template <typename V>
 int coarse_apply_update(hipStream_t s, const CoarseWork& c, const PpeWork& w, const CoarseUpd<V>& u, int kind,
-                        const int* done, const int* brk) {
+                        bool prolong, const int* done, const int* brk) {
   const PpeOp o = ppe_op(w);
   const AggGrid g = agg_grid(c);
   if (kind == 1) k_update_restrict<V, 1><<<c.na + 1, 256, 0, s>>>(o, g, c.na, u, c.c, done, brk);
   else k_update_restrict<V, 2><<<c.na + 1, 256, 0, s>>>(o, g, c.na, u, c.c, done, brk);
   const int gb = (c.na + 3) / 4;
   k_coarse_gemv<<<gb, 256, 0, s>>>(c.X, c.na, c.ld, c.c, c.y, done, brk);
-  k_prolong_add<V><<<grid_for(w.n), kBlock, 0, s>>>(o, g, c.y, u.out, done, brk);
+  if (prolong) k_prolong_add<V><<<grid_for(w.n), kBlock, 0, s>>>(o, g, c.y, u.out, done, brk);
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -643,8 +643,8 @@ void coarse_free(CoarseWork& c) {
 }
 
 template int coarse_apply_update<float>(hipStream_t, const CoarseWork&, const PpeWork&, const CoarseUpd<float>&,
-                                        int, const int*, const int*);
+                                        int, bool, const int*, const int*);
 template int coarse_apply_update<double>(hipStream_t, const CoarseWork&, const PpeWork&, const CoarseUpd<double>&,
-                                         int, const int*, const int*);
+                                         int, bool, const int*, const int*);
 
 }  // namespace sophia

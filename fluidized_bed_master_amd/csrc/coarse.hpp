@@ -75,12 +75,12 @@ struct CoarseUpd {
   const double *alpha, *beta, *omega;
   const int* first;
 };
-// The update of kind `kind`, then out += Z X Z^T of the updated vector over
-// rows; the update and the restriction Z^T are one pass (skipped when *done or
-// *brk).
+// The update of kind `kind`, then c.y = X Z^T of the updated vector and, with
+// prolong, out += Z c.y over rows (the window-staged matvec adds Z c.y itself);
+// the update and the restriction Z^T are one pass (skipped when *done or *brk).
 template <typename V>
 int coarse_apply_update(hipStream_t s, const CoarseWork& c, const PpeWork& w, const CoarseUpd<V>& u, int kind,
-                        const int* done, const int* brk);
+                        bool prolong, const int* done, const int* brk);
 void coarse_free(CoarseWork& c);
 // copy E and X (row-major na x na, FP32) to the host where non-null (synchronises)
 int coarse_export(hipStream_t s, const CoarseWork& c, float* E, float* X);

@@ -69,6 +69,7 @@ struct BiState {
   int iter, max_iter;
   int done;         // 1 converged, 2 breakdown, 3 iteration limit
   int update, stop, brk, first, folds;
+  int fresh;        // no correction gathered since the start or the last fold: xs counts as zero
 };
 
 __device__ inline double wave_sum(double v) {
@@ -991,30 +992,51 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_bi_mv_staged(PpeOp o, const 
 }
 
 // ----- window-staged operator passes (kFmtWin, win.hpp) ------------------------
-// y = A x with the inner FP32 operator; partials (w, y), (y, y).  G lanes per
-// row (win_group).
-template <int G>
+// The coarse correction that a matvec adds to its operand (two-level
+// preconditioner): x_i + y[agg(i)] over the rows, also written to xc, which
+// saves the pass that would add it.
+struct WinCoarse {
+  const double* y = nullptr;
+  float* xc = nullptr;
+  int AX = 0, AY = 0;
+};
+
+// y = A x with the inner FP32 operator, or with CZ of the corrected operand;
+// partials (w, y), (y, y).  G lanes per row (win_group).
+template <int G, bool CZ>
 __global__ __launch_bounds__(kRedThreads, 8) void k_win_mv(PpeOp o, const float* __restrict__ x,
                                                         float* __restrict__ y, const float* __restrict__ w,
-                                                        double* partials, const BiState* st) {
+                                                        WinCoarse cz, double* partials, const BiState* st) {
   if (!iter_live(st)) return;
   __shared__ WinStage<float> S;
+  __shared__ float yc[CZ ? kWinCells : 1];  // the correction of each planned cell
   double d[2] = {0.0, 0.0};
   const int sub = (int)threadIdx.x & (G - 1);
-  win_rows<G>(o, S, x, [&](int i) {
-    WinHead<G> h;
-    h.load(o, i, sub);
-    return h;
-  }, [&](int i, int base, bool lead, WinHead<G>& h) {
-    float s = 0.f;
-    const bool on = h.row != 0;
-    if (on) s = group_sum<G>(win_row_sum<G>(o, h, S.x + base));
-    if (!lead) return;
-    const float yi = on ? o.dgi[i] * x[i] - s : 0.f;
-    y[i] = yi;
-    d[0] += (double)w[i] * (double)yi;
-    d[1] += (double)yi * (double)yi;
-  });
+  win_rows<G>(
+      o, S,
+      [&](int i) {
+        WinHead<G> h;
+        h.load(o, i, sub);
+        return h;
+      },
+      [&](int cx, int cy, int cz_, int first) {
+        if (CZ && first >= 0)
+          yc[threadIdx.x] = (float)cz.y[cx / kAgg + cz.AX * (cy / kAgg + cz.AY * (cz_ / kAgg))];
+        return first;
+      },
+      [&](int first, int l, int c) { return CZ ? x[first + l] + yc[c] : x[first + l]; },
+      [&](int i, int base, bool lead, WinHead<G>& h, int cell) {
+        float s = 0.f;
+        const bool on = h.row != 0;
+        if (on) s = group_sum<G>(win_row_sum<G>(o, h, S.x + base));
+        if (!lead) return;
+        const float xi = on ? (CZ ? x[i] + yc[cell] : x[i]) : 0.f;
+        const float yi = on ? o.dgi[i] * xi - s : 0.f;
+        y[i] = yi;
+        if (CZ) cz.xc[i] = xi;
+        d[0] += (double)w[i] * (double)yi;
+        d[1] += (double)yi * (double)yi;
+      });
   block_partials<2>(d, partials);
 }
 
@@ -1025,42 +1047,57 @@ __global__ __launch_bounds__(kRedThreads) void k_win_apply(PpeOp o, const double
                                                            double* partials) {
   __shared__ WinStage<double> S;
   double d[1] = {0.0};
-  win_rows<G>(o, S, x, [&](int i) { return WinRow{o.row[i]}; }, [&](int i, int base, bool lead, WinRow h) {
-    double s = 0;
-    const bool on = h.row != 0;
-    if (on) s = group_sum<G>(win_row_sum_full<G>(o, i, S.x + base));
-    if (!lead) return;
-    double acc = on ? o.diag[i] * x[i] - s : 0.0;
-    if (on && residual) acc = o.rhs[i] - acc;
-    y[i] = acc;
-    d[0] += acc * acc;
-  });
+  win_rows<G>(
+      o, S, [&](int i) { return WinRow{o.row[i]}; }, [](int, int, int, int first) { return first; },
+      [&](int first, int l, int) { return x[first + l]; },
+      [&](int i, int base, bool lead, WinRow h, int) {
+        double s = 0;
+        const bool on = h.row != 0;
+        if (on) s = group_sum<G>(win_row_sum_full<G>(o, i, S.x + base));
+        if (!lead) return;
+        double acc = on ? o.diag[i] * x[i] - s : 0.0;
+        if (on && residual) acc = o.rhs[i] - acc;
+        y[i] = acc;
+        d[0] += acc * acc;
+      });
   if (want_norm) block_partials<1>(d, partials);
 }
 
-// the true residual after a fold, as k_bi_true
+// Fold and true residual in one pass (k_bi_fold and k_bi_true of the other
+// formats): the staged solution is x64 + xscale xs, each row writes its own to
+// the other of the two solution buffers, which the parity of the folds selects,
+// and xs counts as zero from then on (BiState::fresh).
 template <int G>
-__global__ __launch_bounds__(kRedThreads) void k_win_true(PpeOp o, const double* __restrict__ x64,
-                                                          double* __restrict__ r64, float* __restrict__ r,
-                                                          const float* __restrict__ rh, double* partials,
-                                                          const BiState* st) {
+__global__ __launch_bounds__(kRedThreads) void k_win_true(PpeOp o, double* xa, double* xb,
+                                                          const float* __restrict__ xs, double* __restrict__ r64,
+                                                          float* __restrict__ r, const float* __restrict__ rh,
+                                                          double* partials, const BiState* st) {
   if (st->done || !st->update) return;
-  const double inv = 1.0 / st->xscale;
+  // nothing gathered since the last fold (a breakdown right after it): xs still
+  // holds what that fold took
+  const double sc = st->fresh ? 0.0 : st->xscale, inv = 1.0 / st->xscale;
+  const double* __restrict__ xo = (st->folds & 1) ? xb : xa;
+  double* __restrict__ xn = (st->folds & 1) ? xa : xb;
   __shared__ WinStage<double> S;
   double d[3] = {0.0, 0.0, 0.0};
-  win_rows<G>(o, S, x64, [&](int i) { return WinRow{o.row[i]}; }, [&](int i, int base, bool lead, WinRow h) {
-    double s = 0;
-    const bool on = h.row != 0;
-    if (on) s = group_sum<G>(win_row_sum_full<G>(o, i, S.x + base));
-    if (!lead) return;
-    const double acc = on ? o.rhs[i] - (o.diag[i] * x64[i] - s) : 0.0;
-    r64[i] = acc;
-    const float ri = (float)(acc * inv);
-    r[i] = ri;
-    d[0] += (double)ri * (double)ri;
-    d[1] += (double)rh[i] * (double)ri;
-    d[2] += acc * acc;
-  });
+  win_rows<G>(
+      o, S, [&](int i) { return WinRow{o.row[i]}; }, [](int, int, int, int first) { return first; },
+      [&](int first, int l, int) { return xo[first + l] + sc * (double)xs[first + l]; },
+      [&](int i, int base, bool lead, WinRow h, int) {
+        double s = 0;
+        const bool on = h.row != 0;
+        if (on) s = group_sum<G>(win_row_sum_full<G>(o, i, S.x + base));
+        if (!lead) return;
+        const double xi = on ? xo[i] + sc * (double)xs[i] : xo[i];
+        xn[i] = xi;
+        const double acc = on ? o.rhs[i] - (o.diag[i] * xi - s) : 0.0;
+        r64[i] = acc;
+        const float ri = (float)(acc * inv);
+        r[i] = ri;
+        d[0] += (double)ri * (double)ri;
+        d[1] += (double)rh[i] * (double)ri;
+        d[2] += acc * acc;
+      });
   block_partials<3>(d, partials);
 }
 
@@ -1150,10 +1187,11 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_xr(int n, V* __restrict__ xs
                                                        double* partials, const BiState* st) {
   if (!iter_live(st)) return;
   const double alpha = st->alpha, omega = st->omega;
+  const bool fresh = st->fresh != 0;
   double d[2] = {0.0, 0.0};
   for (RowIter it = xcd_rows(n); it.i < it.end; it.i += it.stride) {
     const int i = it.i;
-    xs[i] = (V)((double)xs[i] + alpha * (double)ph[i] + omega * (double)sh[i]);
+    xs[i] = (V)((fresh ? 0.0 : (double)xs[i]) + alpha * (double)ph[i] + omega * (double)sh[i]);
     const V ri = (V)((double)r[i] - omega * (double)t[i]);
     r[i] = ri;
     d[0] += (double)ri * (double)ri;
@@ -1206,8 +1244,10 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_true(PpeOp o, const double* 
 // state.  Skips exactly when the producer skipped.
 __global__ __launch_bounds__(kFinThreads) void k_fin(const double* partials, int G, int op, BiState* st,
                                                      unsigned* count_out) {
-  if ((op == kFinAlpha || op == kFinOmega || op == kFinRho) && !iter_live(st)) return;
-  if (op == kFinTrue && (st->done || !st->update)) return;
+  // the state travels to registers while the partials are summed
+  BiState s = *st;
+  if ((op == kFinAlpha || op == kFinOmega || op == kFinRho) && !iter_live(&s)) return;
+  if (op == kFinTrue && (s.done || !s.update)) return;
   double tot[3];
   if (op == kFinTrue) {
     sum_partials<3>(partials, G, tot);
@@ -1224,82 +1264,86 @@ __global__ __launch_bounds__(kFinThreads) void k_fin(const double* partials, int
   if (threadIdx.x != 0) return;
   switch (op) {
     case kFinNorm:
-      st->norm = tot[0];
+      s.norm = tot[0];
       break;
     case kFinCount:
       if (count_out) count_out[0] = (unsigned)tot[0];
       break;
     case kFinInit:
-      st->rho = tot[0];
-      st->rho_old = 1;
-      st->alpha = 1;
-      st->omega = 1;
-      st->beta = 0;
-      st->rr = tot[0];
-      st->max_rr = tot[0];
-      st->first = 1;
-      st->done = 0;
-      st->update = 0;
-      st->stop = 0;
-      st->brk = 0;
+      s.rho = tot[0];
+      s.rho_old = 1;
+      s.alpha = 1;
+      s.omega = 1;
+      s.beta = 0;
+      s.rr = tot[0];
+      s.max_rr = tot[0];
+      s.first = 1;
+      s.fresh = 1;
+      s.done = 0;
+      s.update = 0;
+      s.stop = 0;
+      s.brk = 0;
       break;
     case kFinAlpha: {
       const double rv = tot[0];
       if (rv != 0 && rv == rv) {
-        st->alpha = st->rho / rv;
+        s.alpha = s.rho / rv;
       } else {
-        st->brk = 1;
-        st->update = 1;
+        s.brk = 1;
+        s.update = 1;
       }
       break;
     }
     case kFinOmega: {
       const double ts = tot[0], tt = tot[1];
       if (tt > 0 && ts != 0) {
-        st->omega = ts / tt;
+        s.omega = ts / tt;
       } else {
-        st->brk = 1;
-        st->update = 1;
+        s.brk = 1;
+        s.update = 1;
       }
       break;
     }
     case kFinRho: {
       const double rr = tot[0], rho = tot[1];
-      const double alpha = st->alpha, omega = st->omega;
-      st->rho_old = st->rho;
-      st->rho = rho;
-      st->beta = (st->rho_old != 0 && omega != 0) ? (rho / st->rho_old) * (alpha / omega) : 0;
-      st->rr = rr;
-      st->first = 0;
-      st->iter += 1;
-      if (rr > st->max_rr) st->max_rr = rr;
-      bool upd = rr <= st->tol2 || rr < st->delta2 * st->max_rr;
-      if (st->iter >= st->max_iter) {
-        st->stop = 1;
+      const double alpha = s.alpha, omega = s.omega;
+      s.rho_old = s.rho;
+      s.rho = rho;
+      s.beta = (s.rho_old != 0 && omega != 0) ? (rho / s.rho_old) * (alpha / omega) : 0;
+      s.rr = rr;
+      s.first = 0;
+      s.fresh = 0;
+      s.iter += 1;
+      if (rr > s.max_rr) s.max_rr = rr;
+      bool upd = rr <= s.tol2 || rr < s.delta2 * s.max_rr;
+      if (s.iter >= s.max_iter) {
+        s.stop = 1;
         upd = true;
       }
       if (rho == 0 || !(rr == rr)) {
-        st->brk = 1;
+        s.brk = 1;
         upd = true;
       }
-      st->update = upd ? 1 : 0;
+      s.update = upd ? 1 : 0;
       break;
     }
     case kFinTrue: {
       const double rho = tot[1];
-      st->rr = tot[0];
-      st->rr_true = tot[2];
-      st->max_rr = tot[0];
-      st->rho = rho;
-      st->beta = (st->rho_old != 0 && st->omega != 0) ? (rho / st->rho_old) * (st->alpha / st->omega) : 0;
-      st->update = 0;
-      st->folds += 1;
-      if (tot[2] <= st->tol2_true) st->done = 1;
-      else if (st->stop) st->done = 3;
-      else if (st->brk || rho == 0) st->done = 2;
+      s.rr = tot[0];
+      s.rr_true = tot[2];
+      s.max_rr = tot[0];
+      s.rho = rho;
+      s.beta = (s.rho_old != 0 && s.omega != 0) ? (rho / s.rho_old) * (s.alpha / s.omega) : 0;
+      s.update = 0;
+      s.fresh = 1;
+      s.folds += 1;
+      if (tot[2] <= s.tol2_true) s.done = 1;
+      else if (s.stop) s.done = 3;
+      else if (s.brk || rho == 0) s.done = 2;
       break;
     }
   }
+  *st = s;
 }
 
 __global__ void k_gather_rows_guess(int n, const int* row, const double* pres, double* x, int zero) {
@@ -1347,6 +1391,16 @@ int win_grid(int n, int G) { return grid_rows((int)std::min<int64_t>((int64_t)n 
     }                                                                                 \
   } while (0)
 int win_blocks(int n) { return win_grid(n, win_group(n)); }
+
+void launch_win_mv(hipStream_t s, const PpeOp& o, const float* x, float* y, const float* wv, const WinCoarse& cz,
+                   const PpeWork& w, const BiState* st) {
+  const int G = win_group(o.n), g = win_grid(o.n, G);
+  if (cz.y && G == 2) k_win_mv<2, true><<<g, kRedThreads, 0, s>>>(o, x, y, wv, cz, w.partials, st);
+  else if (cz.y) k_win_mv<4, true><<<g, kRedThreads, 0, s>>>(o, x, y, wv, cz, w.partials, st);
+  else if (G == 1) k_win_mv<1, false><<<g, kRedThreads, 0, s>>>(o, x, y, wv, cz, w.partials, st);
+  else if (G == 2) k_win_mv<2, false><<<g, kRedThreads, 0, s>>>(o, x, y, wv, cz, w.partials, st);
+  else k_win_mv<4, false><<<g, kRedThreads, 0, s>>>(o, x, y, wv, cz, w.partials, st);
+}
 
 // y = A x in full precision by the operator's format
 void launch_apply_full(hipStream_t s, const PpeWork& w, const PpeOp& o, const double* x, double* y, bool residual,
@@ -1398,7 +1452,8 @@ int ppe_workspace_alloc(PpeWork& w, int n, int cap, bool mixed) {
   HIP_TRY(A((void**)&w.flags, 16));
   HIP_TRY(hipHostMalloc((void**)&w.host_flags, 16, hipHostMallocDefault));
   w.vec_bytes = mixed ? 4 : 8;
-  for (int k = 0; k < 8; k++) HIP_TRY(A(&w.vec[k], N * w.vec_bytes));
+  for (int k = 0; k < (mixed ? 10 : 8); k++) HIP_TRY(A(&w.vec[k], N * w.vec_bytes));
+  if (mixed) HIP_TRY(A((void**)&w.x64b, N * 8));
   w.mixed = mixed;
   if (mixed) {
     HIP_TRY(A((void**)&w.hi, E * 4));
@@ -1420,7 +1475,8 @@ void ppe_workspace_free(PpeWork& w) {
   F(w.partials); F(w.state); F(w.flags);
   if (w.host_state) (void)hipHostFree(w.host_state);
   if (w.host_flags) (void)hipHostFree(w.host_flags);
-  for (int k = 0; k < 8; k++) F(w.vec[k]);
+  for (void* p : w.vec) F(p);
+  F(w.x64b);
   F(w.hi); F(w.lo); F(w.dgi); F(w.c64);
   if (w.coarse) {
     coarse_free(*w.coarse);
@@ -1687,8 +1743,17 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
     return (w.mv_seq++ % kMvSample) == 0 ? tm : nullptr;
   };
   const int Gm = FMT == kFmtWin ? win_blocks(n) : G;  // blocks of the operator passes
-  auto matvec = [&](const V* x, V* y, const V* ww) {
-    if constexpr (FMT == kFmtWin) WIN_LAUNCH(k_win_mv, n, o, x, y, ww, w.partials, st);
+  // With the two-level preconditioner the window-staged matvec of a run that
+  // launches bound adds the coarse correction to its operand and leaves the sum
+  // in phc / shc: an iteration goes 85.0 -> 77 us at 4,200 rows and 123.7 -> 121.2
+  // at 276,000.  At 1.16 M rows the prolongation pass (6 us) is cheaper than
+  // the gather of the correction in every tile (345 -> 356 us per iteration).
+  constexpr bool kWin = FMT == kFmtWin;
+  const bool fused = kWin && cw && win_group(n) > 1;
+  V* phc = fused ? (V*)w.vec[8] : ph;
+  V* shc = fused ? (V*)w.vec[9] : sh;
+  auto matvec = [&](const V* x, V* y, const V* ww, V* xc) {
+    if constexpr (kWin) launch_win_mv(s, o, x, y, ww, fused ? WinCoarse{cw->y, xc, cw->AX, cw->AY} : WinCoarse{}, w, st);
     else if constexpr (FMT == kFmtRun8) k_bi_mv_staged<V><<<G, kRedThreads, 0, s>>>(o, x, y, ww, w.partials, st);
     else k_bi_mv<FMT, CM, V><<<G, kRedThreads, 0, s>>>(o, x, y, ww, w.partials, st);
   };
@@ -1699,30 +1764,30 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
     for (int c = 0; c < chunk; c++) {
       if (cw) {
         const CoarseUpd<V> u{w.dinv, r, p, v, ph, &st->alpha, &st->beta, &st->omega, &st->first};
-        TRY(coarse_apply_update<V>(s, *cw, w, u, 1, &st->done, &st->brk));
+        TRY(coarse_apply_update<V>(s, *cw, w, u, 1, !fused, &st->done, &st->brk));
       } else {
         k_bi_dir<V><<<G, kRedThreads, 0, s>>>(n, w.dinv, r, p, v, ph, st);
       }
       {
         TimeScope ts(mv_timer(), mv_name);
-        matvec(ph, v, rh);
+        matvec(ph, v, rh, phc);
       }
       launch_fin(s, w, kFinAlpha, nullptr, Gm);
       if (cw) {
         const CoarseUpd<V> u{w.dinv, r, p, v, sh, &st->alpha, &st->beta, &st->omega, &st->first};
-        TRY(coarse_apply_update<V>(s, *cw, w, u, 2, &st->done, &st->brk));
+        TRY(coarse_apply_update<V>(s, *cw, w, u, 2, !fused, &st->done, &st->brk));
       } else {
         k_bi_s<V><<<G, kRedThreads, 0, s>>>(n, w.dinv, r, v, sh, st);
       }
       {
         TimeScope ts(mv_timer(), mv_name);
-        matvec(sh, t, r);
+        matvec(sh, t, r, shc);
       }
       launch_fin(s, w, kFinOmega, nullptr, Gm);
-      k_bi_xr<V><<<G, kRedThreads, 0, s>>>(n, xs, ph, sh, r, t, rh, w.partials, st);
+      k_bi_xr<V><<<G, kRedThreads, 0, s>>>(n, xs, phc, shc, r, t, rh, w.partials, st);
       launch_fin(s, w, kFinRho);
-      k_bi_fold<V><<<G, kRedThreads, 0, s>>>(n, w.row, w.x64, xs, st);
-      if constexpr (FMT == kFmtWin) WIN_LAUNCH(k_win_true, n, o, w.x64, w.r64, r, rh, w.partials, st);
+      if constexpr (!kWin) k_bi_fold<V><<<G, kRedThreads, 0, s>>>(n, w.row, w.x64, xs, st);
+      if constexpr (kWin) WIN_LAUNCH(k_win_true, n, o, w.x64, w.x64b, xs, w.r64, r, rh, w.partials, st);
       else if constexpr (FMT == kFmtRun8)
         k_bi_true_staged<V><<<G, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
       else k_bi_true<FMT, CMF, V><<<G, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
@@ -1742,6 +1807,7 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
       chunk = 8;
     }
   }
+  if (kWin && (h.folds & 1)) std::swap(w.x64, w.x64b);  // the buffer of the last fold
   *iters = h.iter;
   *folds = h.folds;
   *done = h.done;
@@ -1909,7 +1975,7 @@ int ppe_matvec_probe(hipStream_t s, const DevParams& P, const SphView<R>& v, Ppe
   for (int k = 0; k <= reps; k++) {
     if (k == 1) HIP_TRY(hipEventRecord(e0, s));  // the first launch warms the caches, untimed
     if (variant == 1) k_mf_matvec<R><<<grid_xcd(n), kBlock, 0, s>>>(P, v, w.row, w.diag, pk, x, y);
-    else WIN_LAUNCH(k_win_mv, n, o, x, y, rh, w.partials, st);
+    else launch_win_mv(s, o, x, y, rh, WinCoarse{}, w, st);
   }
   HIP_TRY(hipEventRecord(e1, s));
   HIP_TRY(hipEventSynchronize(e1));

@@ -108,7 +108,8 @@ struct PpeWork {
   void* host_state = nullptr;  // pinned mirror
   unsigned* flags = nullptr;   // assembly overflow flags
   unsigned* host_flags = nullptr;
-  void* vec[8] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  void* vec[10] = {};
+  double* x64b = nullptr;  // mixed: the other buffer of the folded solution
   int vec_bytes = 0;
   struct CoarseWork* coarse = nullptr;  // two-level preconditioner, created on first use
   unsigned mv_seq = 0;                  // inner matvec launches seen by the timers

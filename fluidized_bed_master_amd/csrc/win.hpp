@@ -24,7 +24,7 @@ constexpr int kWinThreads = 256;
 constexpr int kWinCells = 256;  // staged cells per tile: 28 planes
 // staged values per tile: a 256-row tile of the 1 mm columns takes about 2800;
 // with the tables it is 19.5 KB in FP32, eight blocks per CU
-constexpr int kWinCap = 4352;
+constexpr int kWinCap = 4096;  // the coarse correction's table leaves no room for more
 static_assert(kWinMax < kWinCap, "a single row's window always fits");
 
 // Where the cells of a tile's planes go: cell c = 9 (e - ea + 1) + r holds the
@@ -51,7 +51,7 @@ __device__ inline int win_ekey(const O& o, uint32_t key) {
 // is the extended key of row i0 and *cells the planned cells, 0 when there is
 // nothing to stage: rows past the last cell, or a single particle whose window
 // does not fit (no row of an assembled operator).  `cellval(x, y, z, first)` is
-// kept per cell in S.start.
+// kept per cell in S.start; first is -1 for places outside the grid.
 template <class O, class CV>
 __device__ int win_plan(const O& o, int i0, int i1, WinPlan& S, int* e0, int* ncells, CV&& cellval) {
   const int t = (int)threadIdx.x, lane = t & 63;
@@ -79,7 +79,7 @@ __device__ int win_plan(const O& o, int i0, int i1, WinPlan& S, int* e0, int* nc
       int y = row - o.NJ * z;
       y += r % 3 - 1;
       z += r / 3 - 1;
-      int first = 0;
+      int first = -1;  // outside the grid: no particles
       if (cell_in(o.pmask, 2, z, o.NK) && cell_in(o.pmask, 1, y, o.NJ) && cell_in(o.pmask, 0, x, o.NI)) {
         const int k = x + o.NI * (y + o.NJ * z);
         first = (int)o.cell_off[k];
@@ -113,7 +113,8 @@ __device__ int win_plan(const O& o, int i0, int i1, WinPlan& S, int* e0, int* nc
   }
 }
 
-// win_plan, then the values: `val(cellval, l)` is that of a cell's l-th particle
+// win_plan, then the values: `val(cellval, l, c)` is that of the l-th particle of
+// planned cell c
 template <typename XT, class CV, class F>
 __device__ int win_stage(const PpeOp& o, int i0, int i1, WinStage<XT>& S, int* e0, CV&& cellval, F&& val) {
   int cells;
@@ -130,12 +131,12 @@ __device__ int win_stage(const PpeOp& o, int i0, int i1, WinStage<XT>& S, int* e
       at[u] = cc < cells ? S.p.pre[cc] : 0;
       n[u] = cc < cells ? S.p.pre[cc + 1] - at[u] : 0;
       st[u] = l0 < n[u] ? S.p.start[cc] : 0;
-      if (l0 < n[u]) v[u] = val(st[u], l0);
+      if (l0 < n[u]) v[u] = val(st[u], l0, cc);
     }
 #pragma unroll
     for (int u = 0; u < 4; u++) {
       if (l0 < n[u]) S.x[at[u] + l0] = v[u];
-      for (int l = l0 + 32; l < n[u]; l += 32) S.x[at[u] + l] = val(st[u], l);
+      for (int l = l0 + 32; l < n[u]; l += 32) S.x[at[u] + l] = val(st[u], l, c + 8 * u);
     }
   }
   __syncthreads();
@@ -177,13 +178,14 @@ struct WinRow {
   int row;
 };
 
-// f(i, base, lead, head(i)) for every row of this block's share, by G lanes
-// each: base is the LDS slot of row i's window, lead marks the first of its
-// lanes, and head(i) has run before the tile was staged.  (Leaving out the
+// f(i, base, lead, head(i), cell) for every row of this block's share, by G
+// lanes each: base is the LDS slot of row i's window, cell the planned cell that
+// holds the row, lead marks the first of its lanes, and head(i) has run before
+// the tile was staged (cellval and val as in win_stage).  (Leaving out the
 // staging of tiles without rows, behind a barrier vote, costs every tile more
 // than the walls' tiles save: 78.4 -> 85.2 us at 1.16 M rows.)
-template <int G, typename XT, class H, class F>
-__device__ __forceinline__ void win_rows(const PpeOp& o, WinStage<XT>& S, const XT* __restrict__ x, H&& head, F&& f) {
+template <int G, typename XT, class H, class CV, class VL, class F>
+__device__ __forceinline__ void win_rows(const PpeOp& o, WinStage<XT>& S, H&& head, CV&& cellval, VL&& val, F&& f) {
   constexpr int TR = kWinThreads / G;
   const int per = (int)gridDim.x >> 3;
   const int chunk = ((((o.n + 7) >> 3) + 63) >> 6) << 6;  // rows per XCD, as xcd_rows
@@ -194,13 +196,14 @@ __device__ __forceinline__ void win_rows(const PpeOp& o, WinStage<XT>& S, const 
     for (int s0 = i0; s0 < i1;) {
       int e0;
       auto hd = head(min(s0 + tr, i1 - 1));
-      const int m = win_stage(
-          o, s0, i1, S, &e0, [](int, int, int, int first) { return first; }, [&](int first, int l) { return x[first + l]; });
+      const int m = win_stage(o, s0, i1, S, &e0, cellval, val);
       const int i = s0 + tr;
       if (i < m) {
+        // particles that no cell or plan holds are not rows: any slot will do
         const uint32_t key = o.keys[i];
         const int c = key < (uint32_t)o.ncell ? 9 * (win_ekey(o, key) - e0) : 0;
-        f(i, S.p.pre[min(max(c, 0), kWinCells)], (t & (G - 1)) == 0, hd);
+        const int cw = min(max(c, 0), kWinCells - 27);
+        f(i, S.p.pre[cw], (t & (G - 1)) == 0, hd, cw + 13);
       }
       s0 = m;
     }
