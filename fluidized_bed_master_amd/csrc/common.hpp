@@ -135,13 +135,21 @@ template <typename R> struct alignas(2 * sizeof(R)) HRec {
 
 // Packed neighbour records of the FP32 pair kernels (mixed path), rebuilt
 // before each kernel that reads them: one 32 B record per particle (a single
-// cache-line gather) in place of four to five field gathers.  aux: rho/rho_ref
-// - 1 for the prep sums, else 0.
+// cache-line gather) in place of four to five field gathers.  vol: m / rho,
+// taken in FP64; aux: rho/rho_ref - 1 for the prep sums, else 0 (vol and pt
+// side by side: kernels that read no aux then take them in one load).
 struct alignas(32) Rec32 {
   float4 p;  // pos4
-  float m, rho;
+  float vol;
   int pt;
-  float aux;
+  float aux, pad;
+};
+// WCSPH continuity (mixed path): V = m/rho, rho/eps and rho/rho_ref in FP64,
+// the velocity and the delta-SPH density gradient.
+struct alignas(64) RecCont {
+  float4 p;  // pos4
+  double vol, rhopor, ratio;
+  float ux, uy, uz, grx, gry, grz;
 };
 // PPE assembly (mixed path): V = m/rho, eps, eps rho and p in FP64 with the
 // FP32 velocity; flags = the cell's coordinates (ten bits per axis) | PPE row
@@ -154,9 +162,9 @@ struct alignas(64) RecAsm {
 };
 
 // Advection's neighbour records on the mixed path, after pk = {x, y, z, m}:
-// {rho, p, u, T} and {S (the flux-wall sum), h, p_type}
+// {V = m/rho, p, u, T} and {S (the flux-wall sum), h, p_type}
 struct alignas(32) PkB {
-  double rho, p;
+  double vol, p;
   float ux, uy, uz, temp;
 };
 struct alignas(16) PkC {
@@ -202,7 +210,7 @@ struct SphView {
   double *ppe1, *ppe2, *ppe3, *ppe4;
   // Packed neighbour records of the pair sums that take FP64 geometry
   // (the symmetric pressure gradient, and every sum of the FP64 path),
-  // rebuilt before each use: {x, y, z, m}, {rho, p}, and for advection
+  // rebuilt before each use: {x, y, z, m}, {V = m/rho, p}, and for advection
   // {ux, uy, uz, T} and {h, p_type}
   double4* pk;
   double2* pk2;
@@ -210,6 +218,7 @@ struct SphView {
   HRec<R>* pkh;
   Rec32* r32;
   RecAsm* ra;
+  RecCont* rc;  // shares ra's memory: WCSPH has no PPE
   RecNeu* rn;
   PkB* pkb;
   PkC* pkc;
@@ -619,6 +628,47 @@ __host__ __device__ inline T knl_dw_ih(int kt, T tA, T tH, T ih, T rr) {
   return knl_dw<T>(kt, tA, tH, rr);
 }
 
+// 1 / r of a pair from d2 = r^2: the hardware's reciprocal square root and one
+// Newton step in FP32, one third-order step in FP64 (2^-23 -> 2^-68 before
+// rounding), 6 and 10 operations in place of the correctly rounded square root
+// and division (about 20 and 45); within an ulp or two of them.  The offset,
+// far below any pair's d2, keeps the self pair (d2 = 0) finite: its r is 0 and
+// its 1 / r at most 1e15 (FP32) or 1e20.
+__device__ inline float pair_rinv(float d2) {
+  d2 += 1e-30f;
+  const float y = __builtin_amdgcn_rsqf(d2);
+  return fmaf(0.5f * y, fmaf(-d2 * y, y, 1.0f), y);
+}
+__device__ inline double pair_rinv(double d2) {
+  d2 += 1e-40;
+  const double y = __builtin_amdgcn_rsq(d2);
+  const double e = fma(-d2 * y, y, 1.0);
+  return fma(fma(0.375, e, 0.5), y * e, y);
+}
+
+// The symmetric KGC inverse of one particle (identity without the correction).
+// The corrected gradient Cm g of a pair enters its sums linearly, so the pair
+// loops add uncorrected terms and correct the sum, or use the identities
+// u . (Cm g) = (Cm u) . g and x . (Cm x).
+template <typename T>
+struct Kgc {
+  T a = 1, b = 0, c = 0, d = 1, e = 0, f = 1;
+  template <typename R>
+  __device__ Kgc(bool on, const R* cm, int n, int i) {
+    if (!on) return;
+    a = (T)cm[i]; b = (T)cm[n + i]; c = (T)cm[2 * n + i];
+    d = (T)cm[3 * n + i]; e = (T)cm[4 * n + i]; f = (T)cm[5 * n + i];
+  }
+  __device__ void apply(T& x, T& y, T& z) const {
+    const T u = a * x + b * y + c * z, v = b * x + d * y + e * z, w = c * x + e * y + f * z;
+    x = u; y = v; z = w;
+  }
+  // x . (Cm x)
+  __device__ T quad(T x, T y, T z) const {
+    return x * (a * x + (b * y + c * z) * (T)2) + y * (d * y + e * z * (T)2) + f * z * z;
+  }
+};
+
 // KGC-corrected gradient with the symmetric inverse stored as 6 entries
 template <typename R, typename T>
 __device__ inline void kgc_apply(const DevParams& P, const R* cm, int n, int i, T& gx, T& gy, T& gz) {
@@ -701,6 +751,9 @@ int sph_kgc_porosity(hipStream_t s, const DevParams& P, const SphView<R>& v, con
                      bool kgc);
 // k_prep_prep alone (the ISPH density reset that sph_prep runs before its sums)
 template <typename R> int sph_prep_prep(hipStream_t s, const DevParams& P, const SphView<R>& v);
+// the packed records of the FP64-geometry pair sums with velocities (NbP)
+template <typename R>
+int sph_pack_velocity_records(hipStream_t s, const SphView<R>& v, bool flux);
 template <typename R> int sph_advection(hipStream_t s, const DevParams& P, const SphView<R>& v);
 // fluid Shepard sums of the flux walls (no-op without a wall heat flux)
 template <typename R> int sph_flux_walls(hipStream_t s, const DevParams& P, const SphView<R>& v);

@@ -430,6 +430,8 @@ struct Ctx : public sophia_ctx {
     TRY(arena.alloc(&v.pkh, NS));
     TRY(arena.alloc(&v.r32, NS));
     TRY(arena.alloc(&v.ra, NS));
+    static_assert(sizeof(RecCont) == sizeof(RecAsm), "one buffer");
+    v.rc = reinterpret_cast<RecCont*>(v.ra);
     TRY(arena.alloc(&v.rn, NS));
     TRY(arena.alloc(&v.pkb, NS));
     TRY(arena.alloc(&v.pkc, NS));

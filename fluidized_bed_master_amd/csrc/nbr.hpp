@@ -125,7 +125,7 @@ __device__ inline void for_nbrs4(const SphView<R>& v, int i, bool eps_rule, F&& 
 // FP64-geometry pair sums read (h and the velocities only with VEL).
 template <typename R>
 struct NbP {
-  double dx, dy, dz, m, rho, pres;
+  double dx, dy, dz, m, vol, pres;
   R ux, uy, uz, temp, h;
   int pt;
   int j;
@@ -133,9 +133,9 @@ struct NbP {
 };
 
 // The list in batches of four like for_nbrs4, reading the packed records
-// pk = {x, y, z, m} and pk2 = {rho, p}, then with VEL pkv = {ux, uy, uz, T}
+// pk = {x, y, z, m} and pk2 = {V, p}, then with VEL pkv = {ux, uy, uz, T}
 // and pkh = {h, p_type}, else p_type: four or three gathers per neighbour in
-// place of twelve or seven.  With VEL on the mixed path pk, pkb = {rho, p,
+// place of twelve or seven.  With VEL on the mixed path pk, pkb = {V, p,
 // u, T} and pkc = {S, h, p_type}: three.  dx = x_i - x_j (minimum image on periodic axes),
 // the same bits as pdiff.
 template <bool VEL, int G = 1, typename R, class F>
@@ -162,14 +162,14 @@ __device__ inline void for_nbrs4_pk(const SphView<R>& v, int i, bool eps_rule, F
         // mixed path: two more records, {rho, p, u, T} and {S, h, p_type}
         const PkB b = v.pkb[j];
         const PkC c = v.pkc[j];
-        q[u].rho = b.rho; q[u].pres = b.p;
+        q[u].vol = b.vol; q[u].pres = b.p;
         q[u].ux = b.ux; q[u].uy = b.uy; q[u].uz = b.uz; q[u].temp = b.temp;
         q[u].S = c.S; q[u].h = c.h; q[u].pt = c.pt;
         q[u].j = j;
         continue;
       }
       const double2 b = v.pk2[j];
-      q[u].rho = b.x;
+      q[u].vol = b.x;
       q[u].pres = b.y;
       if constexpr (VEL) {
         const auto w = v.pkv[j];
@@ -199,7 +199,7 @@ __device__ inline void for_nbrs4_pk(const SphView<R>& v, int i, bool eps_rule, F
 // One neighbour from the 32 B records (FP32 pair kernels): the members of Nb
 // those kernels read, the differences from the position records.
 struct NbR {
-  float dx, dy, dz, m, rho, aux;
+  float dx, dy, dz, vol, aux;
   float ux, uy, uz, temp;
   int pt;
   int j;
@@ -227,7 +227,7 @@ __device__ inline void for_nbrs4_r32(const SphView<float>& v, int i, bool eps_ru
       const Rec32 a = v.r32[j];
       const float3 d = rel_diff(pi4, a.p, v.pgrid, v.pmask);
       q[u].dx = d.x; q[u].dy = d.y; q[u].dz = d.z;
-      q[u].m = a.m; q[u].rho = a.rho; q[u].aux = a.aux; q[u].pt = a.pt;
+      q[u].vol = a.vol; q[u].aux = a.aux; q[u].pt = a.pt;
       if constexpr (VEL) {
         const float4 w = v.pkv[j];
         q[u].ux = w.x; q[u].uy = w.y; q[u].uz = w.z; q[u].temp = w.w;
@@ -243,5 +243,16 @@ __device__ inline void for_nbrs4_r32(const SphView<float>& v, int i, bool eps_ru
     }
   }
 }
+
+// V = m / rho of a neighbour, from its record where there is one
+template <typename R>
+__device__ inline double nb_vol(const Nb<R>& q) { return q.m / q.rho; }
+template <typename R>
+__device__ inline double nb_vol(const NbP<R>& q) { return q.vol; }
+__device__ inline float nb_vol(const NbR& q) { return q.vol; }
+template <typename R>
+__device__ inline double nb_rho(const Nb<R>& q) { return q.rho; }
+template <typename R>
+__device__ inline double nb_rho(const NbP<R>& q) { return q.m / q.vol; }
 
 }  // namespace sophia

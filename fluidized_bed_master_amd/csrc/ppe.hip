@@ -500,7 +500,8 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
     const int top = (int)((__float_as_uint((float)bound) >> 23) & 255u);
     anchor = min(max(top + 1 - 31, 1), 223);
   }
-  double bx = 0, by = 0, bz = 0, Aij = 0, AP = 0, lag = 0;
+  const Kgc<double> K(P.kgc == 1, v.cm, n, i);
+  double bd = 0, Aij = 0, AP = 0, lag = 0;  // bd: -div of eps u
   double dcomp = 0;  // sum over stored columns of a - hi16(a) (mixed)
   int kc = 0, run = 0;
   uint64_t rcw = 0;
@@ -599,19 +600,14 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
     if (e & kNbrFlag) continue;
     if (!nq.use) continue;
     double dx = nq.x, dy = nq.y, dz = nq.z;
-    double r = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
-    // two reciprocals per pair (1/r, V_j = m_j / rho_j) in place of the
-    // reference expressions' divisions; the rounding moves by an ulp
-    const double ir = 1.0 / r;
-    double dw = knl_dw_ih<double>(P.kernel_type, A, hd, ihd, r);
-    const double sd = dw * ir;
-    double gx = sd * dx, gy = sd * dy, gz = sd * dz;
-    kgc_apply(P, v.cm, n, i, gx, gy, gz);
+    const double d2 = dx * dx + dy * dy + dz * dz, ir = pair_rinv(d2);
+    const double sd = knl_dw_ih<double>(P.kernel_type, A, hd, ihd, d2 * ir) * ir;
+    double gx = dx, gy = dy, gz = dz;  // Cm x; the corrected gradient is sd Cm x
+    K.apply(gx, gy, gz);
     const double porj = nq.por, Vj = nq.vol;
-    bx += Vj * (pori * uxi - porj * (double)nq.ux) * gx;
-    by += Vj * (pori * uyi - porj * (double)nq.uy) * gy;
-    bz += Vj * (pori * uzi - porj * (double)nq.uz) * gz;
-    double c = -(dx * gx + dy * gy + dz * gz) * (ir * ir);
+    bd += Vj * sd * ((pori * uxi - porj * (double)nq.ux) * gx + (pori * uyi - porj * (double)nq.uy) * gy +
+                     (pori * uzi - porj * (double)nq.uz) * gz);
+    const double c = -sd * (dx * gx + dy * gy + dz * gz) * (ir * ir);
     double a = (pori * rhoi + nq.porrho) * Vj * irhoi * c;
     Aij += a;
     AP += a * nq.pres;
@@ -686,9 +682,7 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
     }
   }
   if (G > 1) {
-    bx = group_sum<G>(bx);
-    by = group_sum<G>(by);
-    bz = group_sum<G>(bz);
+    bd = group_sum<G>(bd);
     Aij = group_sum<G>(Aij);
     AP = group_sum<G>(AP);
     lag = group_sum<G>(lag);
@@ -732,10 +726,10 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
   o.ccnt[i] = FMT == kFmtWin ? kc | (anchor << 16) : kc;
   o.runc[i] = rcw;
   const double tdt = P.dt_sph;
-  const double bi = P.rho_fluid * (bx + by + bz + 2 * (double)v.dpor[i] - (double)v.dpor_prev[i]) / tdt;
+  const double bi = P.rho_fluid * (bd + 2 * (double)v.dpor[i] - (double)v.dpor_prev[i]) / tdt;
   v.ppe3[i] = bi;
   v.ppe4[i] = AP;
-  v.ppe1[i] = rhoi * (bx + by + bz) / tdt;
+  v.ppe1[i] = rhoi * bd / tdt;
   v.ppe2[i] = Aij;
   o.diag[i] = Aij;
   if (MIXED) o.dgi[i] = (float)(Aij - dcomp);
@@ -1642,12 +1636,26 @@ __global__ __launch_bounds__(kBlock) void k_mean_part(int n, const int* row, con
     part[2 * blockIdx.x + 1] = tc;
   }
 }
-__global__ void k_mean_fin(const double* part, int nb, double* mean) {
-  if (threadIdx.x != 0) return;
+// one block, fixed order: thread t adds the partials t, t + kBlock, ..., then
+// waves and lanes (one thread adding all 2048 pairs took 177 us)
+__global__ __launch_bounds__(kBlock) void k_mean_fin(const double* part, int nb, double* mean) {
+  __shared__ double sa[kBlock / 64], sc[kBlock / 64];
   double ta = 0, tc = 0;
-  for (int b = 0; b < nb; b++) {
+  for (int b = threadIdx.x; b < nb; b += kBlock) {
     ta += part[2 * b];
     tc += part[2 * b + 1];
+  }
+  ta = group_sum<64>(ta);
+  tc = group_sum<64>(tc);
+  if ((threadIdx.x & 63) == 0) {
+    sa[threadIdx.x >> 6] = ta;
+    sc[threadIdx.x >> 6] = tc;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < kBlock / 64; w++) {
+    ta += sa[w];
+    tc += sc[w];
   }
   *mean = tc > 0 ? ta / tc : 0.0;
 }
@@ -1659,7 +1667,7 @@ int ppe_project_mean(hipStream_t s, PpeWork& w, double* v) {
   if (w.n <= 0) return 0;
   const int nb = std::min(grid_for(w.n), kMaxGrid);
   k_mean_part<<<nb, kBlock, 0, s>>>(w.n, w.row, v, w.partials);
-  k_mean_fin<<<1, 64, 0, s>>>(w.partials, nb, w.partials + 2 * kMaxGrid);
+  k_mean_fin<<<1, kBlock, 0, s>>>(w.partials, nb, w.partials + 2 * kMaxGrid);
   k_mean_sub<<<grid_for(w.n), kBlock, 0, s>>>(w.n, w.row, v, w.partials + 2 * kMaxGrid);
   HIP_TRY(hipGetLastError());
   if (v == w.rhs) w.bn = -1;  // the cached norm belongs to the old rhs

@@ -52,8 +52,7 @@ __global__ void k_pack_r32(SphView<float> v) {
   if (i >= v.n) return;
   Rec32 r;
   r.p = v.pos4[i];
-  r.m = (float)v.m[i];
-  r.rho = (float)v.rho[i];
+  r.vol = (float)(v.m[i] / v.rho[i]);
   r.pt = v.ptype[i];
   r.aux = AUX ? (float)(v.rho[i] / v.rho_ref[i] - 1.0) : 0.f;
   v.r32[i] = r;
@@ -91,17 +90,16 @@ __global__ __launch_bounds__(kBlock) void k_kgc(DevParams P, SphView<R> v) {
   T xx = 0, yy = 0, zz = 0, xy = 0, yz = 0, zx = 0;
   auto term = [&](const auto& q, bool on) {
     T dx = (T)q.dx, dy = (T)q.dy, dz = (T)q.dz;
-    T r = sqrt(dx * dx + dy * dy + dz * dz);
+    const T d2 = dx * dx + dy * dy + dz * dz, ir = pair_rinv(d2), r = d2 * ir;
     const bool use = on && q.pt <= 1000 && r > 0 && r < Rs;
-    T dw = knl_dw_ih<T>(P.kernel_type, A, h, ih, r);
-    T mtd = (T)q.m * dw;
-    T rtd = (T)1 / ((T)q.rho * r);
-    xx += use ? -mtd * dx * dx * rtd : (T)0;
-    xy += use ? -mtd * dy * dx * rtd : (T)0;
-    yy += use ? -mtd * dy * dy * rtd : (T)0;
-    zx += use ? -mtd * dx * dz * rtd : (T)0;
-    yz += use ? -mtd * dy * dz * rtd : (T)0;
-    zz += use ? -mtd * dz * dz * rtd : (T)0;
+    const T k = use ? -(T)nb_vol(q) * knl_dw_ih<T>(P.kernel_type, A, h, ih, r) * ir : (T)0;
+    const T kx = k * dx, ky = k * dy;
+    xx += kx * dx;
+    xy += kx * dy;
+    yy += ky * dy;
+    zx += kx * dz;
+    yz += ky * dz;
+    zz += k * dz * dz;
   };
   if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false, G>(v, i, false, term);
   else for_nbrs4<true, G>(v, i, false, term);
@@ -141,18 +139,17 @@ __global__ __launch_bounds__(kBlock) void k_porosity_sph(DevParams P, SphView<R>
   if (i >= v.n) return;
   if (v.itype[i] > 2) return;
   const double hd = v.h[i];
-  const T h = (T)hd, A = knl_tmpA<T>(P.kernel_type, P.dim, h);
+  const T h = (T)hd, ih = (T)(1.0 / hd), A = knl_tmpA<T>(P.kernel_type, P.dim, h);
   const double Rs = P.kappa * hd;
   const double xi = v.x[i], yi = v.y[i], zi = v.z[i];
   const int pti = v.ptype[i];
   T flt = 0, por = 0, dfx = 0, dfy = 0, dfz = 0;
   auto term = [&](const auto& q, bool on) {
     T dx = (T)q.dx, dy = (T)q.dy, dz = (T)q.dz;
-    T r = sqrt(dx * dx + dy * dy + dz * dz) + (T)1e-20;
-    T w = knl_w<T>(P.kernel_type, A, h, r);
-    int ptj = q.pt;
-    const bool use = on && pti <= 1000 && ptj <= 1000 && ptj == 1;
-    flt += use ? (T)q.m / (T)q.rho * w : (T)0;
+    const T d2 = dx * dx + dy * dy + dz * dz;
+    const T w = knl_w_ih<T>(P.kernel_type, A, h, ih, d2 * pair_rinv(d2));
+    const bool use = on && pti <= 1000 && q.pt == 1;
+    flt += use ? (T)nb_vol(q) * w : (T)0;
   };
   if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false, G>(v, i, true, term);
   else for_nbrs4<true, G>(v, i, true, term);
@@ -209,23 +206,21 @@ __global__ __launch_bounds__(kBlock) void k_kgc_porosity(DevParams P, SphView<fl
   T flt = 0, por = 0, dfx = 0, dfy = 0, dfz = 0;
   for_nbrs4_r32<false, G>(v, i, false, [&](const NbR& q, bool on) {
     const T dx = q.dx, dy = q.dy, dz = q.dz;
-    const T r = sqrt(dx * dx + dy * dy + dz * dz);
+    const T d2 = dx * dx + dy * dy + dz * dz, ir = pair_rinv(d2), r = d2 * ir;
     if (krow) {
       const bool use = on && q.pt <= 1000 && r > 0 && r < Rk;
-      T dw = knl_dw_ih<T>(P.kernel_type, A, h, ih, r);
-      T mtd = q.m * dw;
-      T rtd = (T)1 / (q.rho * r);
-      xx += use ? -mtd * dx * dx * rtd : (T)0;
-      xy += use ? -mtd * dy * dx * rtd : (T)0;
-      yy += use ? -mtd * dy * dy * rtd : (T)0;
-      zx += use ? -mtd * dx * dz * rtd : (T)0;
-      yz += use ? -mtd * dy * dz * rtd : (T)0;
-      zz += use ? -mtd * dz * dz * rtd : (T)0;
+      const T k = use ? -q.vol * knl_dw_ih<T>(P.kernel_type, A, h, ih, r) * ir : (T)0;
+      const T kx = k * dx, ky = k * dy;
+      xx += kx * dx;
+      xy += kx * dy;
+      yy += ky * dy;
+      zx += kx * dz;
+      yz += ky * dz;
+      zz += k * dz * dz;
     }
-    const T rp = r + (T)1e-20;
-    const T w = knl_w<T>(P.kernel_type, A, h, rp);
-    const bool usep = on && !q.flag && pti <= 1000 && q.pt <= 1000 && q.pt == 1;
-    flt += usep ? q.m / q.rho * w : (T)0;
+    const T w = knl_w_ih<T>(P.kernel_type, A, h, ih, r);
+    const bool usep = on && !q.flag && pti <= 1000 && q.pt == 1;
+    flt += usep ? q.vol * w : (T)0;
   });
   xx = group_sum<G>(xx);
   yy = group_sum<G>(yy);
@@ -322,18 +317,15 @@ __global__ __launch_bounds__(kBlock) void k_prep(DevParams P, SphView<R> v) {
   auto term = [&](const auto& q, bool on) {
     const bool use = on && q.pt <= 1000;
     T dx = (T)q.dx, dy = (T)q.dy, dz = (T)q.dz;
-    T r = sqrt(dx * dx + dy * dy + dz * dz) + (T)1e-20;
-    const T Vj = (T)q.m / (T)q.rho;
+    const T d2 = dx * dx + dy * dy + dz * dz, ir = pair_rinv(d2), r = d2 * ir;
+    const T Vj = (T)nb_vol(q);
     if (P.filt_step) flt += use ? Vj * knl_w_ih<T>(P.kernel_type, A, h, ih, r) : (T)0;
     if (anto) {
-      T dw = knl_dw_ih<T>(P.kernel_type, A, h, ih, r);
-      const T sd = dw / r;
-      T gx = sd * dx, gy = sd * dy, gz = sd * dz;
-      kgc_apply(P, v.cm, n, i, gx, gy, gz);
-      T c = (T)(-ratio_diff(q, ratio_i, ratio_i1)) * Vj;
-      rx += use ? c * gx : (T)0;
-      ry += use ? c * gy : (T)0;
-      rz += use ? c * gz : (T)0;
+      const T sd = knl_dw_ih<T>(P.kernel_type, A, h, ih, r) * ir;
+      const T c = use ? (T)(-ratio_diff(q, ratio_i, ratio_i1)) * Vj * sd : (T)0;
+      rx += c * dx;
+      ry += c * dy;
+      rz += c * dz;
     }
   };
   if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<false, G>(v, i, true, term);
@@ -345,6 +337,7 @@ __global__ __launch_bounds__(kBlock) void k_prep(DevParams P, SphView<R> v) {
   if (G > 1 && pair_sub<G>() != 0) return;
   if (P.filt_step) v.flt_s[i] = flt;
   if (anto) {
+    Kgc<T>(P.kgc == 1, v.cm, n, i).apply(rx, ry, rz);
     v.grx[i] = rx;
     v.gry[i] = ry;
     v.grz[i] = rz;
@@ -398,7 +391,7 @@ __global__ void k_pack_records(SphView<R> v, bool flux) {
   v.pk[i] = make_double4(v.x[i], v.y[i], v.z[i], v.m[i]);
   if constexpr (VEL && std::is_same<R, float>::value) {
     PkB b;
-    b.rho = v.rho[i];
+    b.vol = v.m[i] / v.rho[i];
     b.p = v.pres[i];
     b.ux = v.ux[i]; b.uy = v.uy[i]; b.uz = v.uz[i]; b.temp = v.temp[i];
     v.pkb[i] = b;
@@ -409,7 +402,7 @@ __global__ void k_pack_records(SphView<R> v, bool flux) {
     v.pkc[i] = c;
     return;
   }
-  v.pk2[i] = make_double2(v.rho[i], v.pres[i]);
+  v.pk2[i] = make_double2(v.m[i] / v.rho[i], v.pres[i]);
   if constexpr (VEL) {
     typename Vec4Of<R>::type w;
     w.x = v.ux[i]; w.y = v.uy[i]; w.z = v.uz[i]; w.w = v.temp[i];
@@ -462,7 +455,11 @@ __global__ __launch_bounds__(kBlock) void k_advection(DevParams P, SphView<R> v)
   const T vis_const = (visi * visf) / (visi + visf);
   const T cv_i = 4 * pori / rhoi;
   const T kc_const = (T)4 * pori * kcf * kci / (rhoi * (kci + kcf));
-  T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0;
+  const Kgc<double> K(P.kgc == 1, v.cm, n, i);
+  // u_i . (Cm g) = (Cm u_i) . g
+  double wx = (double)uxi, wy = (double)uyi, wz = (double)uzi;
+  K.apply(wx, wy, wz);
+  T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0, ax = 0, ay = 0, az = 0;
   double px = 0, py = 0, pz = 0, fl = 0;
   auto term = [&](const auto& q, bool on) {
     const bool use = on && q.pt < 1000;
@@ -477,62 +474,51 @@ __global__ __launch_bounds__(kBlock) void k_advection(DevParams P, SphView<R> v)
       }
     }
     // geometry in FP64 arithmetic: the symmetric pressure-gradient term
-    // cancels a hydrostatic offset of order H/h times its result.  Two
-    // reciprocals per pair (1/r, 1/rho_j) replace the divisions of the
-    // reference's expressions; the rounding moves by an ulp
+    // cancels a hydrostatic offset of order H/h times its result
     const double dxd = q.dx, dyd = q.dy, dzd = q.dz;
-    const double rd = sqrt(dxd * dxd + dyd * dyd + dzd * dzd) + 1e-20;
-    const double ird = 1.0 / rd, irhod = 1.0 / q.rho;
+    const double d2 = dxd * dxd + dyd * dyd + dzd * dzd;
+    const double ird = pair_rinv(d2), rd = d2 * ird, Vd = nb_vol(q);
     const double dwd = knl_dw_ih<double>(P.kernel_type, Ad, hd, ihd, rd);
-    const double sd = dwd * ird;
-    double gxd = sd * dxd, gyd = sd * dyd, gzd = sd * dzd;
-    kgc_apply(P, v.cm, n, i, gxd, gyd, gzd);
+    const double sd = dwd * ird;  // grad W = sd (x_i - x_j)
     if (P.fp_solve) {
       // (rho_i / eps_i) Cp with Cp = -eps_i m_j pp / (rho_i rho_j)
       const double pp = P.pgrad_form ? q.pres - pid : pid + q.pres;
-      const double Vpp = q.m * pp * irhod;
-      px -= use ? Vpp * gxd : 0.0;
-      py -= use ? Vpp * gyd : 0.0;
-      pz -= use ? Vpp * gzd : 0.0;
+      const double c = use ? Vd * pp * sd : 0.0;
+      px -= c * dxd;
+      py -= c * dyd;
+      pz -= c * dzd;
     }
-    const T dx = (T)dxd, dy = (T)dyd, dz = (T)dzd, r = (T)rd, dw = (T)dwd, ir = (T)ird;
-    const T gx = (T)gxd, gy = (T)gyd, gz = (T)gzd;
-    const T mj = (T)q.m, irhoj = (T)irhod, Vj = mj * irhoj;
+    const T dw = (T)dwd, ir = (T)ird, Vj = (T)Vd;
     const T uxj = q.ux, uyj = q.uy, uzj = q.uz;
     if (P.fv_solve) {
       const T visj = tab ? v.visp[q.j] : visf;
       const T vm = tab ? (visi * visj) / (visi + visj) : vis_const;
-      // (x.g / r) / r: the self pair (x = 0, 1/r = 1e20) stays 0 in FP32,
-      // where a product 1/r^2 would overflow
-      T Cv = (dx * gx + dy * gy + dz * gz) * ir;
-      Cv *= ir;
-      Cv *= vm * cv_i * Vj;
+      // x . (Cm grad W) / r^2
+      const T Cv = (T)(sd * K.quad(dxd, dyd, dzd) * ird * ird) * (vm * cv_i * Vj);
       tx += use ? Cv * (uxi - uxj) : (T)0;
       ty += use ? Cv * (uyi - uyj) : (T)0;
       tz += use ? Cv * (uzi - uzj) : (T)0;
     }
     if (P.fva_solve) {
+      const T dx = (T)dxd, dy = (T)dyd, dz = (T)dzd, r = (T)rd;
       T uij_xij = (uxi - uxj) * dx + (uyi - uyj) * dy + (uzi - uzj) * dz;
       T hij = (h + (T)q.h) * (T)0.5;
       T phi = hij * uij_xij;
       phi /= (r * r + (T)0.01 * hij * hij);
       T Pij = mi * phi * ((T)(-0.1 * P.soundspeed) + (T)0.02 * phi);
-      Pij /= (rhoi + (T)q.rho);
+      Pij /= (rhoi + (T)nb_rho(q));
       Pij *= (T)0.5;
-      const bool av = use && uij_xij < 0;
-      tx += av ? -Pij * gx : (T)0;
-      ty += av ? -Pij * gy : (T)0;
-      tz += av ? -Pij * gz : (T)0;
+      const T c = use && uij_xij < 0 ? -Pij * (T)sd : (T)0;
+      ax += c * dx;
+      ay += c * dy;
+      az += c * dz;
     }
     if (euler) {
-      const T c = Vj * (1 - eli);
-      ex += use ? (uxi * (uxj - uxi) * gx + uyi * (uxj - uxi) * gy + uzi * (uxj - uxi) * gz) * c : (T)0;
-      ey += use ? (uxi * (uyj - uyi) * gx + uyi * (uyj - uyi) * gy + uzi * (uyj - uyi) * gz) * c : (T)0;
-      ez += use ? (uxi * (uzj - uzi) * gx + uyi * (uzj - uzi) * gy + uzi * (uzj - uzi) * gz) * c : (T)0;
-      if (P.con_solve) {
-        T tj = q.temp;
-        et += use ? (uxi * (tj - tempi) * gx + uyi * (tj - tempi) * gy + uzi * (tj - tempi) * gz) * c : (T)0;
-      }
+      const T ug = (T)(sd * (wx * dxd + wy * dyd + wz * dzd)) * Vj * (1 - eli);
+      ex += use ? ug * (uxj - uxi) : (T)0;
+      ey += use ? ug * (uyj - uyi) : (T)0;
+      ez += use ? ug * (uzj - uzi) : (T)0;
+      if (P.con_solve) et += use ? ug * ((T)q.temp - tempi) : (T)0;
     }
     if (P.con_solve) {
       // 4 eps_i m_j k_j k_i (T_i - T_j) dW / ((r + 1e-10) rho_i rho_j (k_i + k_j))
@@ -563,7 +549,19 @@ __global__ __launch_bounds__(kBlock) void k_advection(DevParams P, SphView<R> v)
   py = group_sum<G>(py);
   pz = group_sum<G>(pz);
   fl = group_sum<G>(fl);
+  if (P.fva_solve) {
+    ax = group_sum<G>(ax);
+    ay = group_sum<G>(ay);
+    az = group_sum<G>(az);
+  }
   if (G > 1 && pair_sub<G>() != 0) return;
+  K.apply(px, py, pz);
+  if (P.fva_solve) {
+    Kgc<T>(P.kgc == 1, v.cm, n, i).apply(ax, ay, az);
+    tx += ax;
+    ty += ay;
+    tz += az;
+  }
   if (P.fg_solve) tz += -(T)P.gravity;
   v.fx[i] = tx - ex;
   v.fy[i] = ty - ey;
@@ -799,23 +797,19 @@ __global__ __launch_bounds__(kBlock) void k_pressure_force(DevParams P, SphView<
   const T h = hd, ih = 1.0 / hd, A = knl_tmpA<T>(P.kernel_type, P.dim, h);
   const double xi = v.x[i], yi = v.y[i], zi = v.z[i], pid = v.pres[i];
   const T rhoi = v.rho[i], pori = v.por[i];
-  // Cp = -eps_i m_j pp / (rho_i rho_j): the per-particle factor hoisted and
-  // 1/r, 1/rho_j taken once per pair (the rounding moves by an ulp)
+  // Cp = -eps_i m_j pp / (rho_i rho_j)
   const T ci = -pori / rhoi;
   T tx = 0, ty = 0, tz = 0;
   auto term = [&](const auto& q, bool on) {
     const bool use = on && q.pt < 1000;
     T dx = (T)q.dx, dy = (T)q.dy, dz = (T)q.dz;
-    T r = sqrt(dx * dx + dy * dy + dz * dz) + (T)1e-20;
-    T dw = knl_dw_ih<T>(P.kernel_type, A, h, ih, r);
-    const T sd = dw / r;
-    T gx = sd * dx, gy = sd * dy, gz = sd * dz;
-    kgc_apply(P, v.cm, n, i, gx, gy, gz);
+    const T d2 = dx * dx + dy * dy + dz * dz, ir = pair_rinv(d2);
+    const T sd = knl_dw_ih<T>(P.kernel_type, A, h, ih, d2 * ir) * ir;
     const T pp = P.pgrad_form ? q.pres - pid : pid + q.pres;
-    const T Cp = ci * (q.m * pp / q.rho);
-    tx += use ? Cp * gx : (T)0;
-    ty += use ? Cp * gy : (T)0;
-    tz += use ? Cp * gz : (T)0;
+    const T Cp = use ? nb_vol(q) * pp * sd : (T)0;
+    tx += Cp * dx;
+    ty += Cp * dy;
+    tz += Cp * dz;
   };
   if (P.fp_solve) {
     // the difference form carries no hydrostatic offset, so geometry from
@@ -828,9 +822,11 @@ __global__ __launch_bounds__(kBlock) void k_pressure_force(DevParams P, SphView<
   ty = group_sum<G>(ty);
   tz = group_sum<G>(tz);
   if (G > 1 && pair_sub<G>() != 0) return;
-  v.fpx[i] = (R)tx;
-  v.fpy[i] = (R)ty;
-  v.fpz[i] = (R)tz;
+  // Cm and -eps_i / rho_i on the sum
+  Kgc<T>(P.kgc == 1, v.cm, n, i).apply(tx, ty, tz);
+  v.fpx[i] = (R)(ci * tx);
+  v.fpy[i] = (R)(ci * ty);
+  v.fpz[i] = (R)(ci * tz);
 }
 
 // KERNEL_clc_projection_sph (functions_TIME_ISPH2.cuh:104-212): predictor
@@ -914,14 +910,13 @@ __global__ __launch_bounds__(kBlock) void k_xsph(DevParams P, SphView<R> v) {
     int ptj = q.pt;
     const bool use = on && (ptj == 1 || ptj == 3);
     T dx = (T)q.dx, dy = (T)q.dy, dz = (T)q.dz;
-    T r = sqrt(dx * dx + dy * dy + dz * dz);
-    T w = knl_w_ih<T>(P.kernel_type, A, h, ih, r);
-    T vj = (T)q.m / (T)q.rho;
-    tx += use ? c * vj * (-uxi + (T)q.ux) * w : (T)0;
-    ty += use ? c * vj * (-uyi + (T)q.uy) * w : (T)0;
-    tz += use ? c * vj * (-uzi + (T)q.uz) * w : (T)0;
-    tt += use ? (T)0.01 * c * vj * ((T)q.temp - ti) * w : (T)0;
-    fl += use ? vj * w : (T)0;
+    const T d2 = dx * dx + dy * dy + dz * dz;
+    const T vw = (T)nb_vol(q) * knl_w_ih<T>(P.kernel_type, A, h, ih, d2 * pair_rinv(d2));
+    tx += use ? vw * (-uxi + (T)q.ux) : (T)0;
+    ty += use ? vw * (-uyi + (T)q.uy) : (T)0;
+    tz += use ? vw * (-uzi + (T)q.uz) : (T)0;
+    tt += use ? vw * ((T)q.temp - ti) : (T)0;
+    fl += use ? vw : (T)0;
   };
   if constexpr (std::is_same<R, float>::value) for_nbrs4_r32<true, G>(v, i, false, term);
   else for_nbrs4<true, G>(v, i, false, term);
@@ -932,10 +927,10 @@ __global__ __launch_bounds__(kBlock) void k_xsph(DevParams P, SphView<R> v) {
   fl = group_sum<G>(fl);
   if (G > 1 && pair_sub<G>() != 0) return;
   const T on = (T)(pti > 0);
-  v.xsx[i] = (uxi + tx / fl) * on;
-  v.xsy[i] = (uyi + ty / fl) * on;
-  v.xsz[i] = (uzi + tz / fl) * on;
-  v.xst[i] = (ti + tt / fl) * on;
+  v.xsx[i] = (uxi + c * tx / fl) * on;
+  v.xsy[i] = (uyi + c * ty / fl) * on;
+  v.xsz[i] = (uzi + c * tz / fl) * on;
+  v.xst[i] = (ti + (T)0.01 * c * tt / fl) * on;
 }
 
 template <typename R>
@@ -1076,9 +1071,15 @@ template <typename R> int sph_prep(hipStream_t s, const DevParams& P, const SphV
   return 0;
 }
 template <typename R> int sph_prep_prep(hipStream_t s, const DevParams& P, const SphView<R>& v) { LAUNCH(k_prep_prep, P, v); }
+template <typename R> int sph_pack_velocity_records(hipStream_t s, const SphView<R>& v, bool flux) {
+  if (v.n <= 0) return 0;
+  k_pack_records<R, true><<<grid_for(v.n), kBlock, 0, s>>>(v, flux);
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
 template <typename R> int sph_advection(hipStream_t s, const DevParams& P, const SphView<R>& v) {
   if (v.n > 0) {
-    if (packed_geometry<R>(P)) k_pack_records<R, true><<<grid_for(v.n), kBlock, 0, s>>>(v, P.heat_flux != 0.0);
+    if (packed_geometry<R>(P)) TRY(sph_pack_velocity_records(s, v, P.heat_flux != 0.0));
     return pair_launch(v.n, [&](auto g, int grid) {
       constexpr int G = decltype(g)::value;
       if (P.heat_flux != 0.0) k_advection<R, true, G><<<grid, kBlock, 0, s>>>(P, v);
@@ -1153,6 +1154,7 @@ template <typename R> int sph_xsph(hipStream_t s, const DevParams& P, const SphV
   template int sph_prep_prep<R>(hipStream_t, const DevParams&, const SphView<R>&);                          \
   template int sph_kgc_porosity<R>(hipStream_t, const DevParams&, const SphView<R>&, const DemView&,         \
                                    const CellView&, bool);                                                  \
+  template int sph_pack_velocity_records<R>(hipStream_t, const SphView<R>&, bool);                            \
   template int sph_advection<R>(hipStream_t, const DevParams&, const SphView<R>&);                          \
   template int sph_flux_walls<R>(hipStream_t, const DevParams&, const SphView<R>&);                         \
   template int sph_neumann<R>(hipStream_t, const DevParams&, const SphView<R>&, const CellView&);           \

@@ -105,6 +105,60 @@ __global__ void k_mass_update(DevParams P, SphView<R> v) {
 // velocity divergence, the eps-advection term of Eulerian particles and
 // the delta-SPH diffusion (Molteni, or Antuono with the density gradient).
 // FP64 sums: drho integrates into rho, which the Tait EOS raises to gamma.
+// Bound by its gathers and FP64 arithmetic: the mixed path reads one 64 B
+// record per neighbour in place of thirteen field gathers, with V_j and the two
+// ratios taken once per particle in place of seven FP64 divisions per pair.
+__global__ void k_pack_cont(SphView<float> v) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= v.n) return;
+  RecCont r;
+  r.p = v.pos4[i];
+  const double rho = v.rho[i];
+  r.vol = v.m[i] / rho;
+  r.rhopor = rho / v.por[i];
+  r.ratio = rho / v.rho_ref[i];
+  r.ux = v.ux[i]; r.uy = v.uy[i]; r.uz = v.uz[i];
+  r.grx = v.grx[i]; r.gry = v.gry[i]; r.grz = v.grz[i];
+  v.rc[i] = r;
+}
+
+// One neighbour of the continuity sums.
+struct NbC {
+  double dx, dy, dz, vol, rhopor, ratio;
+  double ux, uy, uz, grx, gry, grz;
+};
+// f(neighbour, counted) over the list by G lanes, from the records (mixed) or
+// the fields
+template <int G, typename R, class F>
+__device__ inline void for_nbrs_cont(const SphView<R>& v, int i, F&& f) {
+  if constexpr (std::is_same<R, float>::value) {
+    const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
+    if (cnt <= 0) return;
+    const int n = v.n, last4 = (cnt - 1) & ~3, k0 = 4 * pair_sub<G>();
+    const float4 pi4 = v.pos4[i];
+    uint4 en4 = *(const uint4*)(v.nbr + nbr_slot(min(k0, last4), i, n));
+    for (int k = k0; k < cnt; k += 4 * G) {
+      const uint32_t en[4] = {en4.x, en4.y, en4.z, en4.w};
+      RecCont r[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) r[u] = v.rc[(int)(en[u] & ~kNbrFlag)];
+      en4 = *(const uint4*)(v.nbr + nbr_slot(min(k + 4 * G, last4), i, n));
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const float3 d = rel_diff(pi4, r[u].p, v.pgrid, v.pmask);
+        const NbC q{d.x, d.y, d.z, r[u].vol, r[u].rhopor, r[u].ratio, r[u].ux, r[u].uy, r[u].uz,
+                    r[u].grx, r[u].gry, r[u].grz};
+        f(q, k + u < cnt && !(en[u] & kNbrFlag));
+      }
+    }
+  } else {
+    for_nbrs4<true, G>(v, i, true, [&](const Nb<R>& q, bool on) {
+      const NbC c{q.dx, q.dy, q.dz, q.m / q.rho, q.rho / q.por, q.rho / q.rref, q.ux, q.uy, q.uz, q.grx, q.gry, q.grz};
+      f(c, on);
+    });
+  }
+}
+
 template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_continuity(DevParams P, SphView<R> v) {
   typedef double T;
@@ -114,50 +168,41 @@ __global__ __launch_bounds__(kBlock) void k_continuity(DevParams P, SphView<R> v
   if (P.open_boundary > 0 && v.btype[i] > 0) return;
   if (v.ptype[i] <= 0) return;
   const int n = v.n;
-  const T h = v.h[i], A = knl_tmpA<T>(P.kernel_type, P.dim, h);
-  const T xi = v.x[i], yi = v.y[i], zi = v.z[i];
+  const T h = v.h[i], ih = 1.0 / h, A = knl_tmpA<T>(P.kernel_type, P.dim, h);
   const T uxi = v.ux[i], uyi = v.uy[i], uzi = v.uz[i];
   const T rhoi = v.rho[i], pori = v.por[i];
   const T gxi = v.grx[i], gyi = v.gry[i], gzi = v.grz[i];
-  const T rri = v.rho_ref[i];
+  const T rri = v.rho_ref[i], rpi = rhoi / pori, ratio_i = rhoi / rri;
   const T el = P.eulerian ? 0.0 : 1.0;
   const bool dsph = P.delsph > 0, anto = P.delsph == 2;
-  T tx = 0, ty = 0, tz = 0, px = 0, py = 0, pz = 0, tR = 0;
-  for_nbrs4<true, G>(v, i, true, [&](const Nb<R>& q, bool on) {
-    const bool use = on && q.pt <= 1000;
-    const T dx = (T)q.dx, dy = (T)q.dy, dz = (T)q.dz;
-    const T r = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
-    const T dw = knl_dw<T>(P.kernel_type, A, h, r);
-    T gx = dw * dx / r, gy = dw * dy / r, gz = dw * dz / r;
-    if (P.kgc > 0) kgc_apply(P, v.cm, n, i, gx, gy, gz);
-    const T mj = q.m, porj = q.por, rhoj = q.rho;
-    const T tmprho = mj * (rhoi / rhoj);
-    tx += use ? (uxi - (T)q.ux) * tmprho * gx : 0.0;
-    ty += use ? (uyi - (T)q.uy) * tmprho * gy : 0.0;
-    tz += use ? (uzi - (T)q.uz) * tmprho * gz : 0.0;
-    px += use ? uxi * mj / rhoj * (rhoi / pori - rhoj / porj) * gx : 0.0;
-    py += use ? uyi * mj / rhoj * (rhoi / pori - rhoj / porj) * gy : 0.0;
-    pz += use ? uzi * mj / rhoj * (rhoi / pori - rhoj / porj) * gz : 0.0;
+  const Kgc<T> K(P.kgc == 1, v.cm, n, i);
+  T wx = uxi, wy = uyi, wz = uzi;  // u_i . (Cm g) = (Cm u_i) . g
+  K.apply(wx, wy, wz);
+  // sums over V_j: (u_i - u_j) . grad~W, (rho_i/eps_i - rho_j/eps_j) u_i . grad~W
+  // and the delta-SPH term; the per-particle factors follow
+  T td = 0, pd = 0, tR = 0;
+  for_nbrs_cont<G>(v, i, [&](const NbC& q, bool use) {
+    const T dx = q.dx, dy = q.dy, dz = q.dz;
+    const T d2 = dx * dx + dy * dy + dz * dz, ir = pair_rinv(d2);
+    const T vs = q.vol * (knl_dw_ih<T>(P.kernel_type, A, h, ih, d2 * ir) * ir);
+    T cx = dx, cy = dy, cz = dz;
+    K.apply(cx, cy, cz);
+    td += use ? vs * ((uxi - q.ux) * cx + (uyi - q.uy) * cy + (uzi - q.uz) * cz) : 0.0;
+    pd += use ? vs * (rpi - q.rhopor) * (wx * dx + wy * dy + wz * dz) : 0.0;
     if (dsph) {
-      const T rrj = q.rref;
-      T phi = (gxi + (T)q.grx) * -dx;
-      phi += (gyi + (T)q.gry) * -dy;
-      phi += (gzi + (T)q.grz) * -dz;
-      phi = (-0.5 * phi) * (anto ? 1.0 : 0.0) + (rhoj / rrj - rhoi / rri);
-      T trr = -2 * P.delta_sph * h * rri * P.soundspeed * (mj / rhoj);
-      trr *= phi * dw / r;
-      tR += use ? trr : 0.0;
+      T phi = (gxi + q.grx) * -dx;
+      phi += (gyi + q.gry) * -dy;
+      phi += (gzi + q.grz) * -dz;
+      phi = (-0.5 * phi) * (anto ? 1.0 : 0.0) + (q.ratio - ratio_i);
+      tR += use ? vs * phi : 0.0;
     }
   });
-  tx = group_sum<G>(tx);
-  ty = group_sum<G>(ty);
-  tz = group_sum<G>(tz);
-  px = group_sum<G>(px);
-  py = group_sum<G>(py);
-  pz = group_sum<G>(pz);
+  td = group_sum<G>(td);
+  pd = group_sum<G>(pd);
   tR = group_sum<G>(tR);
   if (G > 1 && pair_sub<G>() != 0) return;
-  v.drho[i] = (R)((tx + ty + tz) + pori * (px + py + pz) * (1 - el) + tR * (dsph ? 1.0 : 0.0));
+  const T ds = -2 * P.delta_sph * h * rri * P.soundspeed;
+  v.drho[i] = (R)(rhoi * td + pori * pd * (1 - el) + (dsph ? ds * tR : 0.0));
 }
 
 // KERNEL_EOS (functions_PROP.cuh:7-28): p = B ((rho / rho_ref)^gamma - 1)
@@ -177,6 +222,9 @@ __global__ void k_eos(DevParams P, SphView<R> v) {
 // Eulerian advection term (interface, repulsive, surface-tension,
 // Boussinesq and concentration terms are off in this build).  Geometry and
 // the pressure term in FP64, as in the ISPH force kernels.
+// Neighbours from the packed records of the ISPH advection (NbP), with V_j in
+// place of m_j and rho_j, and the KGC inverse on the sums where they are linear
+// in the gradient.
 template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<R> v) {
   typedef R T;
@@ -185,84 +233,78 @@ __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<
   if (v.itype[i] != 1 || v.ptype[i] > 1000) return;
   const int pti = v.ptype[i];
   const int n = v.n;
-  const double hd = v.h[i];
+  const double hd = v.h[i], ihd = 1.0 / hd;
   const T h = (T)hd;
   const double Ad = knl_tmpA<double>(P.kernel_type, P.dim, hd);
-  const double xi = v.x[i], yi = v.y[i], zi = v.z[i];
   const T uxi = v.ux[i], uyi = v.uy[i], uzi = v.uz[i], tempi = v.temp[i];
   const double pid = v.pres[i], rhoid = v.rho[i], porid = v.por[i];
   const T mi = (T)v.m[i], rhoi = (T)rhoid, pori = (T)porid;
   const bool tab = P.prop_table != 0;
-  const T visi = tab ? v.visp[i] : (T)P.mu_fluid;
+  const T visi = tab ? v.visp[i] : (T)P.mu_fluid, visf = (T)P.mu_fluid;
+  const T vis_const = (visi * visf) / (visi + visf);
+  const T cv_i = 4 * pori / rhoi;
   const T eta = (T)(0.001 * hd);
   const T kci = tab ? v.condp[i] : (T)(pti > 1000 || pti < -1000 ? P.k_dem : P.k_fluid);
   const T cpi = (T)(pti > 1000 || pti < -1000 ? P.cp_dem : P.cp_fluid);
   const T el = P.eulerian ? (T)0 : (T)1;
   const bool euler = el < (T)1;
-  T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0;
-  double ptx = 0, pty = 0, ptz = 0, px = 0, py = 0, pz = 0;
-  for_nbrs4<false, G>(v, i, true, [&](const Nb<R>& q, bool on) {
+  const Kgc<double> K(P.kgc == 1, v.cm, n, i);
+  double wx = (double)uxi, wy = (double)uyi, wz = (double)uzi;  // u_i . (Cm g) = (Cm u_i) . g
+  K.apply(wx, wy, wz);
+  T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0, ax = 0, ay = 0, az = 0;
+  double px = 0, py = 0, pz = 0;  // sum_j V_j pp grad W
+  for_nbrs4_pk<true, G>(v, i, true, [&](const NbP<R>& q, bool on) {
     const bool use = on && q.pt <= 1000;
     const double dxd = q.dx, dyd = q.dy, dzd = q.dz;
-    const double rd = sqrt(dxd * dxd + dyd * dyd + dzd * dzd) + 1e-20;
-    const double dwd = knl_dw<double>(P.kernel_type, Ad, hd, rd);
-    double gxd = dwd * dxd / rd, gyd = dwd * dyd / rd, gzd = dwd * dzd / rd;
-    if (P.kgc > 0) kgc_apply(P, v.cm, n, i, gxd, gyd, gzd);
+    const double d2 = dxd * dxd + dyd * dyd + dzd * dzd;
+    const double ird = pair_rinv(d2), rd = d2 * ird;
+    const double dwd = knl_dw_ih<double>(P.kernel_type, Ad, hd, ihd, rd);
+    const double sd = dwd * ird;  // grad W = sd (x_i - x_j)
     if (P.fp_solve) {
       const double pp = P.pgrad_form ? q.pres - pid : pid + q.pres;
-      const double Cp = -porid * q.m * pp / (rhoid * q.rho);
-      ptx += use ? Cp * gxd : 0.0;
-      pty += use ? Cp * gyd : 0.0;
-      ptz += use ? Cp * gzd : 0.0;
-      px += use ? rhoid / porid * Cp * gxd : 0.0;
-      py += use ? rhoid / porid * Cp * gyd : 0.0;
-      pz += use ? rhoid / porid * Cp * gzd : 0.0;
+      const double c = use ? q.vol * pp * sd : 0.0;
+      px += c * dxd;
+      py += c * dyd;
+      pz += c * dzd;
     }
-    const T dx = (T)dxd, dy = (T)dyd, dz = (T)dzd, r = (T)rd, dw = (T)dwd;
-    const T gx = (T)gxd, gy = (T)gyd, gz = (T)gzd;
-    const T mj = (T)q.m, rhoj = (T)q.rho;
+    const T Vj = (T)q.vol, dw = (T)dwd;
     const T uxj = q.ux, uyj = q.uy, uzj = q.uz;
     if (P.fv_solve && pti > 0) {
-      T visj = tab ? v.visp[q.j] : (T)P.mu_fluid;
-      T Cv = dx * gx + dy * gy + dz * gz;
-      Cv *= (visi * visj) / (visi + visj);
-      Cv *= 4 * pori * (mj / (rhoi * rhoj));
-      Cv /= r;
-      Cv /= r;
+      const T visj = tab ? v.visp[q.j] : visf;
+      const T vm = tab ? (visi * visj) / (visi + visj) : vis_const;
+      // x . (Cm grad W) / r^2
+      const T Cv = (T)(sd * K.quad(dxd, dyd, dzd) * ird * ird) * (vm * cv_i * Vj);
       tx += use ? Cv * (uxi - uxj) : (T)0;
       ty += use ? Cv * (uyi - uyj) : (T)0;
       tz += use ? Cv * (uzi - uzj) : (T)0;
     }
     if (P.fva_solve) {
+      const T dx = (T)dxd, dy = (T)dyd, dz = (T)dzd, r = (T)rd;
       T uij_xij = (uxi - uxj) * dx + (uyi - uyj) * dy + (uzi - uzj) * dz;
       T hij = (h + (T)q.h) * (T)0.5;
       T phi = hij * uij_xij;
       phi /= (r * r + (T)0.01 * hij * hij);
       T Pij = mi * phi * ((T)(-0.1 * P.soundspeed) + (T)0.02 * phi);
-      Pij /= (rhoi + rhoj);
+      Pij /= (rhoi + (T)nb_rho(q));
       Pij *= (T)0.5;
-      const bool av = use && uij_xij < 0;
-      tx += av ? -Pij * gx : (T)0;
-      ty += av ? -Pij * gy : (T)0;
-      tz += av ? -Pij * gz : (T)0;
+      const T c = use && uij_xij < 0 ? -Pij * (T)sd : (T)0;
+      ax += c * dx;
+      ay += c * dy;
+      az += c * dz;
     }
     if (P.con_solve) {
       const int ptj = q.pt;
       T kcj = tab ? v.condp[q.j] : (T)(ptj > 1000 || ptj < -1000 ? P.k_dem : P.k_fluid);
-      T H = (T)4.0 * mj * kcj * kci * (tempi - (T)q.temp) * dw;
-      H /= cpi * (r + eta * eta) * rhoi * rhoj * (kci + kcj);
+      T H = (T)4.0 * Vj * kcj * kci * (tempi - (T)q.temp) * dw;
+      H /= cpi * ((T)rd + eta * eta) * rhoi * (kci + kcj);
       Rc += use ? H : (T)0;
     }
     if (euler) {
-      T c = mj / rhoj;
-      ex += use ? (uxi * (uxj - uxi) * gx + uyi * (uxj - uxi) * gy + uzi * (uxj - uxi) * gz) * c * (1 - el) : (T)0;
-      ey += use ? (uxi * (uyj - uyi) * gx + uyi * (uyj - uyi) * gy + uzi * (uyj - uyi) * gz) * c * (1 - el) : (T)0;
-      ez += use ? (uxi * (uzj - uzi) * gx + uyi * (uzj - uzi) * gy + uzi * (uzj - uzi) * gz) * c * (1 - el) : (T)0;
-      if (P.con_solve) {
-        T tj = q.temp;
-        et += use ? (uxi * (tj - tempi) * gx + uyi * (tj - tempi) * gy + uzi * (tj - tempi) * gz) * c * (1 - el)
-                  : (T)0;
-      }
+      const T ug = (T)(sd * (wx * dxd + wy * dyd + wz * dzd)) * Vj * (1 - el);
+      ex += use ? ug * (uxj - uxi) : (T)0;
+      ey += use ? ug * (uyj - uyi) : (T)0;
+      ez += use ? ug * (uzj - uzi) : (T)0;
+      if (P.con_solve) et += use ? ug * ((T)q.temp - tempi) : (T)0;
     }
   });
   tx = group_sum<G>(tx);
@@ -273,24 +315,28 @@ __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<
   ey = group_sum<G>(ey);
   ez = group_sum<G>(ez);
   et = group_sum<G>(et);
-  ptx = group_sum<G>(ptx);
-  pty = group_sum<G>(pty);
-  ptz = group_sum<G>(ptz);
   px = group_sum<G>(px);
   py = group_sum<G>(py);
   pz = group_sum<G>(pz);
+  if (P.fva_solve) {
+    ax = group_sum<G>(ax);
+    ay = group_sum<G>(ay);
+    az = group_sum<G>(az);
+    Kgc<T>(P.kgc == 1, v.cm, n, i).apply(ax, ay, az);
+  }
   if (G > 1 && pair_sub<G>() != 0) return;
-  // pressure first, then the other terms, in the reference's per-pair order
-  // of one accumulator; FP32 rounding of the sum of both is below the tests'
-  // tolerance
-  double fx = ptx + (double)tx, fy = pty + (double)ty, fz = ptz + (double)tz;
+  K.apply(px, py, pz);
+  // pressure -eps_i / rho_i V_j pp, then the other terms; FP32 rounding of the
+  // sum of both is below the tests' tolerance
+  const double ci = -porid / rhoid;
+  double fx = ci * px + (double)(tx + ax), fy = ci * py + (double)(ty + ay), fz = ci * pz + (double)(tz + az);
   if (P.fg_solve) fz += -P.gravity;
   v.fx[i] = (R)(fx - (double)ex);
   v.fy[i] = (R)(fy - (double)ey);
   v.fz[i] = (R)(fz - (double)ez);
-  v.pgx[i] = (R)px;
-  v.pgy[i] = (R)py;
-  v.pgz[i] = (R)pz;
+  v.pgx[i] = (R)-px;
+  v.pgy[i] = (R)-py;
+  v.pgz[i] = (R)-pz;
   v.fmag[i] = (R)sqrt(fx * fx + fy * fy + fz * fz);
   if (P.con_solve) v.dtemp[i] = Rc * (T)(pti != -3) - et;
 }
@@ -361,10 +407,13 @@ int wc_volume_mass(hipStream_t s, const DevParams& P, const SphView<R>& v, const
   return 0;
 }
 template <typename R> int wc_continuity(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  if (v.n <= 0) return 0;
+  if constexpr (std::is_same<R, float>::value) k_pack_cont<<<grid_for(v.n), kBlock, 0, s>>>(v);
   return pair_launch(v.n, [&](auto g, int grid) { k_continuity<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
 }
 template <typename R> int wc_eos(hipStream_t s, const DevParams& P, const SphView<R>& v) { WC_LAUNCH(k_eos, P, v); }
 template <typename R> int wc_interaction(hipStream_t s, const DevParams& P, const SphView<R>& v) {
+  TRY(sph_pack_velocity_records(s, v, false));
   return pair_launch(v.n,
                      [&](auto g, int grid) { k_wc_interaction<R, decltype(g)::value><<<grid, kBlock, 0, s>>>(P, v); });
 }

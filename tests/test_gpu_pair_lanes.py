@@ -76,3 +76,46 @@ def test_wcsph_step_at_every_lane_count(n):
     compare_fields(a1, b1, ["ux", "uy", "uz", "rho", "pres", "flt_s", "DEMpor", "temp"], 1e-9, "wcsph")
     compare_fields(a3, b3, ["drho", "ftotalx", "ftotaly", "ftotalz", "dtemp"], 1e-9, "wcsph/p3")
     g.close()
+
+
+OPTIONS = {
+    "artificial_viscosity": {"fva_solve": 1},
+    "no_kgc": {"kgc_solve": 0},
+    "no_kgc_artificial_viscosity": {"kgc_solve": 0, "fva_solve": 1},
+    "difference_form": {"pgrad_form": 1, "fva_solve": 1},
+    "no_pressure_no_viscosity": {"fp_solve": 0, "fv_solve": 0},
+    "gaussian": {"kernel_type": abi.KNL_GAUSSIAN},
+    "wendland6": {"kernel_type": abi.KNL_WENDLAND6},
+}
+
+
+@pytest.mark.parametrize("prec", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("solver", ["isph", "wcsph"])
+@pytest.mark.parametrize("name", OPTIONS)
+def test_pair_terms_under_every_option(name, solver, prec):
+    """The correction on the sums, u . (Cm g) = (Cm u) . g and the reciprocal
+    square root against the oracle's pair terms, option by option."""
+    from fluidized_bed_master_amd.sophia import Sophia
+    from oracle.oracle import Oracle
+    if name == "wendland6" and prec == abi.PREC_MIXED:
+        # porosity near zero under this kernel: the drag amplifies the FP32
+        # rounding of the porosity sum to 1e-4 of the force, whatever the order
+        pytest.skip("the sphere drag is ill-conditioned in FP32 porosities here")
+    if solver == "isph":
+        p, parts = configs.small_isph_dem(seed=6)
+        configs.heated(p, parts)
+    else:
+        p, parts = configs.wcsph_dem_column(9, 8, 14, con=1)
+    for k, val in OPTIONS[name].items():
+        setattr(p, k, val)
+    g, o = Sophia(p, parts, precision=prec), Oracle(p, parts)
+    opts = abi.ppe_opts(method=abi.PPE_JACOBI) if solver == "isph" else None
+    g.step(opts)
+    o.step(opts)
+    a1, _, a3 = g.get_particles(abi.SPH)
+    b1, _, b3 = o.get_particles(abi.SPH)
+    f1 = ["rho", "flt_s", "DEMpor", "grad_rhox", "grad_rhoz", "ux", "uy", "uz", "temp", "pgf_x", "pgf_y", "pgf_z"]
+    f3 = ["Cm", "ftotalx", "ftotaly", "ftotalz", "dtemp"] + (["fpx", "fpz"] if solver == "isph" else ["drho"])
+    compare_fields(a1, b1, f1, TOL[prec], f"{solver}/{name}", floor=1e-12)
+    compare_fields(a3, b3, f3, TOL[prec], f"{solver}/{name}/p3", floor=1e-12)
+    g.close()
