@@ -92,6 +92,23 @@ __device__ inline RowIter xcd_rows(int n) {
   return RowIter{lo + b * (int)blockDim.x + (int)threadIdx.x, hi, per * (int)blockDim.x};
 }
 
+// Lanes per row of the FP64 and u32-index operator passes: one lane walks a
+// row's ten pairs of quads in turn, which small systems cannot hide.  Time per
+// BiCGStab iteration with 1 / 4 / 8 lanes: 61.5 / 55.7 / 55.9 us for the periodic
+// box of 12,000 rows; 64.1 / 64.2 / 73.7 for a column of 55,000, where smaller
+// tiles stage more per row.
+inline int row_lanes(int n) { return n >= 30000 ? 1 : 4; }
+
+// f(i0, i1) for this block's tiles of kRedThreads / G rows; tiles as xcd_rows
+template <int G, class F>
+__device__ __forceinline__ void lane_rows(int n, F&& f) {
+  constexpr int TR = kRedThreads / G;
+  const int per = (int)gridDim.x >> 3;
+  const int chunk = ((((n + 7) >> 3) + 63) >> 6) << 6;
+  const int lo = (int)(blockIdx.x & 7) * chunk, hi = min(n, lo + chunk);
+  for (int i0 = lo + (int)(blockIdx.x >> 3) * TR; i0 < hi; i0 += per * TR) f(i0, min(i0 + TR, hi));
+}
+
 // Block sums of NV values into partials[q * G + block].  A one-block
 // finalize kernel adds the G partials in a fixed order (deterministic); a
 // "last block" reduction inside the producing kernel would need a
@@ -182,7 +199,9 @@ struct CoefQuad<2> {
 // STAGED (kFmtRun8 only): x is the block's LDS copy of the particles of its
 // nine run rows, and adj[r] maps a particle index of run row r to its LDS
 // slot (slot = index + adj[r]); the row's own particle lies in run row 4.
-template <int FMT, int CM, typename AT, typename XT, bool STAGED = false>
+// With G lanes per row each takes every G-th pair of quads, and the caller adds
+// the lanes (row_lanes).
+template <int FMT, int CM, typename AT, typename XT, bool STAGED = false, int G = 1>
 __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restrict__ x,
                                       const int* adj = nullptr) {
   const int cnt = o.ccnt[i];
@@ -191,6 +210,7 @@ __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restric
   const size_t n = (size_t)o.n;
   const int nq = (cnt + 3) >> 2;
   const int last = nq - 1;
+  const int q0 = G == 1 ? 0 : 2 * ((int)threadIdx.x & (G - 1));
   if (FMT == kFmtRun8) {
     const uint32_t key = o.keys[i];
     const int NI = o.NI, NJ = o.NJ;
@@ -212,12 +232,12 @@ __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restric
       if (r < 8) E[r] = acc;
     }
     const int self = STAGED ? i + adj[4] : i;
-    const size_t q1 = (size_t)min(1, last) * n + i;
-    uint32_t wn0 = o.idx[i], wn1 = o.idx[q1];
+    const size_t qs = (size_t)min(q0, last) * n + i, q1 = (size_t)min(q0 + 1, last) * n + i;
+    uint32_t wn0 = o.idx[qs], wn1 = o.idx[q1];
     CoefQuad<CM> cn0, cn1;
-    cn0.load(o, (size_t)i);
+    cn0.load(o, qs);
     cn1.load(o, q1);
-    for (int q = 0; q < nq; q += 2) {
+    for (int q = q0; q < nq; q += 2 * G) {
       const uint32_t w0 = wn0, w1 = wn1;
       const CoefQuad<CM> c0 = cn0, c1 = cn1;
       int j[8];
@@ -233,8 +253,8 @@ __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restric
       XT xv[8];
 #pragma unroll
       for (int u = 0; u < 8; u++) xv[u] = x[j[u]];
-      const size_t qa = (size_t)min(q + 2, last) * n + i;
-      const size_t qb = (size_t)min(q + 3, last) * n + i;
+      const size_t qa = (size_t)min(q + 2 * G, last) * n + i;
+      const size_t qb = (size_t)min(q + 2 * G + 1, last) * n + i;
       wn0 = o.idx[qa];
       wn1 = o.idx[qb];
       cn0.load(o, qa);
@@ -246,20 +266,20 @@ __device__ __forceinline__ AT row_sum(const PpeOp& o, int i, const XT* __restric
     }
   } else {
     const uint4* ix = reinterpret_cast<const uint4*>(o.idx);
-    const size_t q1 = (size_t)min(1, last) * n + i;
-    uint4 jn0 = ix[i], jn1 = ix[q1];
+    const size_t qs = (size_t)min(q0, last) * n + i, q1 = (size_t)min(q0 + 1, last) * n + i;
+    uint4 jn0 = ix[qs], jn1 = ix[q1];
     CoefQuad<CM> cn0, cn1;
-    cn0.load(o, (size_t)i);
+    cn0.load(o, qs);
     cn1.load(o, q1);
-    for (int q = 0; q < nq; q += 2) {
+    for (int q = q0; q < nq; q += 2 * G) {
       const uint4 j0 = jn0, j1 = jn1;
       const CoefQuad<CM> c0 = cn0, c1 = cn1;
       const int jj[8] = {(int)j0.x, (int)j0.y, (int)j0.z, (int)j0.w, (int)j1.x, (int)j1.y, (int)j1.z, (int)j1.w};
       XT xv[8];
 #pragma unroll
       for (int u = 0; u < 8; u++) xv[u] = x[4 * q + u < cnt ? jj[u] : i];
-      const size_t qa = (size_t)min(q + 2, last) * n + i;
-      const size_t qb = (size_t)min(q + 3, last) * n + i;
+      const size_t qa = (size_t)min(q + 2 * G, last) * n + i;
+      const size_t qb = (size_t)min(q + 2 * G + 1, last) * n + i;
       jn0 = ix[qa];
       jn1 = ix[qb];
       cn0.load(o, qa);
@@ -790,22 +810,24 @@ __global__ void k_jacobi(SphView<R> v, const int* row) {
 // ----- full-precision operator ----------------------------------------------
 // y = A x (FP64 or hi + lo); residual form y = rhs - A x; optional ||y||^2
 // partials (finished by k_fin with kFinNorm)
-template <int FMT, int CM>
+template <int FMT, int CM, int G>
 __global__ __launch_bounds__(kRedThreads) void k_apply_full(PpeOp o, const double* __restrict__ x,
                                                             double* __restrict__ y, int residual, int want_norm,
                                                             double* partials) {
   double d[1] = {0.0};
-  for (RowIter it = xcd_rows(o.n); it.i < it.end; it.i += it.stride) {
-    const int i = it.i;
-    double acc = 0;
-    if (o.row[i]) {
-      const double s = row_sum<FMT, CM, double>(o, i, x);
-      acc = o.diag[i] * x[i] - s;
-      if (residual) acc = o.rhs[i] - acc;
-    }
+  const int t = (int)threadIdx.x;
+  lane_rows<G>(o.n, [&](int i0, int i1) {
+    const int i = i0 + t / G;
+    if (i >= i1) return;
+    double s = 0;
+    const bool on = o.row[i] != 0;
+    if (on) s = group_sum<G>(row_sum<FMT, CM, double, double, false, G>(o, i, x));
+    if (G > 1 && (t & (G - 1)) != 0) return;
+    double acc = on ? o.diag[i] * x[i] - s : 0.0;
+    if (on && residual) acc = o.rhs[i] - acc;
     y[i] = acc;
     d[0] += acc * acc;
-  }
+  });
   if (want_norm) block_partials<1>(d, partials);
 }
 
@@ -870,25 +892,26 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_dir(int n, const double* __r
 }
 
 // y = A x with the inner operator; partials (w, y), (y, y)
-template <int FMT, int CM, typename V>
+template <int FMT, int CM, typename V, int G>
 __global__ __launch_bounds__(kRedThreads) void k_bi_mv(PpeOp o, const V* __restrict__ x, V* __restrict__ y,
                                                        const V* __restrict__ w, double* partials,
                                                        const BiState* st) {
   if (!iter_live(st)) return;
   typedef typename std::conditional<CM == 0, float, double>::type AT;
   double d[2] = {0.0, 0.0};
-  for (RowIter it = xcd_rows(o.n); it.i < it.end; it.i += it.stride) {
-    const int i = it.i;
-    AT acc = 0;
-    if (o.row[i]) {
-      const AT s = row_sum<FMT, CM, AT>(o, i, x);
-      acc = (CM == 0 ? (AT)o.dgi[i] : (AT)o.diag[i]) * (AT)x[i] - s;
-    }
-    const V yi = (V)acc;
+  const int t = (int)threadIdx.x;
+  lane_rows<G>(o.n, [&](int i0, int i1) {
+    const int i = i0 + t / G;
+    if (i >= i1) return;
+    AT s = 0;
+    const bool on = o.row[i] != 0;
+    if (on) s = group_sum<G>(row_sum<FMT, CM, AT, V, false, G>(o, i, x));
+    if (G > 1 && (t & (G - 1)) != 0) return;
+    const V yi = on ? (V)((CM == 0 ? (AT)o.dgi[i] : (AT)o.diag[i]) * (AT)x[i] - s) : (V)0;
     y[i] = yi;
     d[0] += (double)w[i] * (double)yi;
     d[1] += (double)yi * (double)yi;
-  }
+  });
   block_partials<2>(d, partials);
 }
 
@@ -956,32 +979,29 @@ __device__ bool stage_tile(const PpeOp& o, const XT* __restrict__ x, int i0, int
   return true;
 }
 
-template <typename V>
+template <typename V, int G>
 __global__ __launch_bounds__(kRedThreads, 8) void k_bi_mv_staged(PpeOp o, const V* __restrict__ x,
                                                               V* __restrict__ y, const V* __restrict__ w,
                                                               double* partials, const BiState* st) {
   if (!iter_live(st)) return;
   __shared__ Stage<V> S;
   double d[2] = {0.0, 0.0};
-  const RowIter it = xcd_rows(o.n);
   const int t = (int)threadIdx.x;
-  for (int i0 = it.i - t; i0 < it.end; i0 += it.stride) {
-    const int i1 = min(i0 + (int)blockDim.x, it.end);
+  lane_rows<G>(o.n, [&](int i0, int i1) {
     const bool staged = stage_tile(o, x, i0, i1, S);
-    const int i = i0 + t;
-    if (i < i1) {
-      double acc = 0;
-      if (o.row[i]) {
-        const double s = staged ? row_sum<kFmtRun8, 2, double, V, true>(o, i, S.x, S.adj)
-                                : row_sum<kFmtRun8, 2, double, V>(o, i, x);
-        acc = o.diag[i] * (double)x[i] - s;
-      }
-      const V yi = (V)acc;
-      y[i] = yi;
-      d[0] += (double)w[i] * (double)yi;
-      d[1] += (double)yi * (double)yi;
-    }
-  }
+    const int i = i0 + t / G;
+    if (i >= i1) return;
+    double s = 0;
+    const bool on = o.row[i] != 0;
+    if (on)
+      s = group_sum<G>(staged ? row_sum<kFmtRun8, 2, double, V, true, G>(o, i, S.x, S.adj)
+                              : row_sum<kFmtRun8, 2, double, V, false, G>(o, i, x));
+    if (G > 1 && (t & (G - 1)) != 0) return;
+    const V yi = on ? (V)(o.diag[i] * (double)x[i] - s) : (V)0;
+    y[i] = yi;
+    d[0] += (double)w[i] * (double)yi;
+    d[1] += (double)yi * (double)yi;
+  });
   block_partials<2>(d, partials);
 }
 
@@ -1097,35 +1117,33 @@ __global__ __launch_bounds__(kRedThreads) void k_win_true(PpeOp o, double* xa, d
 
 // The FP64 operator passes (y = A x or rhs - A x with an optional norm, and
 // the true residual after a fold) with x64 staged in LDS per tile like the
-// inner matvec (kFmtRun8).  Each thread sums the same rows in the same order
-// as the unstaged kernels, so the bits are the same.
+// inner matvec (kFmtRun8).
+template <int G>
 __global__ __launch_bounds__(kRedThreads) void k_apply_staged(PpeOp o, const double* __restrict__ x,
                                                               double* __restrict__ y, int residual, int want_norm,
                                                               double* partials) {
   __shared__ Stage<double> S;
   double d[1] = {0.0};
-  const RowIter it = xcd_rows(o.n);
   const int t = (int)threadIdx.x;
-  for (int i0 = it.i - t; i0 < it.end; i0 += it.stride) {
-    const int i1 = min(i0 + (int)blockDim.x, it.end);
+  lane_rows<G>(o.n, [&](int i0, int i1) {
     const bool staged = stage_tile(o, x, i0, i1, S);
-    const int i = i0 + t;
-    if (i < i1) {
-      double acc = 0;
-      if (o.row[i]) {
-        const double sm = staged ? row_sum<kFmtRun8, 2, double, double, true>(o, i, S.x, S.adj)
-                                 : row_sum<kFmtRun8, 2, double>(o, i, x);
-        acc = o.diag[i] * x[i] - sm;
-        if (residual) acc = o.rhs[i] - acc;
-      }
-      y[i] = acc;
-      d[0] += acc * acc;
-    }
-  }
+    const int i = i0 + t / G;
+    if (i >= i1) return;
+    double s = 0;
+    const bool on = o.row[i] != 0;
+    if (on)
+      s = group_sum<G>(staged ? row_sum<kFmtRun8, 2, double, double, true, G>(o, i, S.x, S.adj)
+                              : row_sum<kFmtRun8, 2, double, double, false, G>(o, i, x));
+    if (G > 1 && (t & (G - 1)) != 0) return;
+    double acc = on ? o.diag[i] * x[i] - s : 0.0;
+    if (on && residual) acc = o.rhs[i] - acc;
+    y[i] = acc;
+    d[0] += acc * acc;
+  });
   if (want_norm) block_partials<1>(d, partials);
 }
 
-template <typename V>
+template <typename V, int G>
 __global__ __launch_bounds__(kRedThreads) void k_bi_true_staged(PpeOp o, const double* __restrict__ x64,
                                                                 double* __restrict__ r64, V* __restrict__ r,
                                                                 const V* __restrict__ rh, double* partials,
@@ -1134,27 +1152,25 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_true_staged(PpeOp o, const d
   const double inv = 1.0 / st->xscale;
   __shared__ Stage<double> S;
   double d[3] = {0.0, 0.0, 0.0};
-  const RowIter it = xcd_rows(o.n);
   const int t = (int)threadIdx.x;
-  for (int i0 = it.i - t; i0 < it.end; i0 += it.stride) {
-    const int i1 = min(i0 + (int)blockDim.x, it.end);
+  lane_rows<G>(o.n, [&](int i0, int i1) {
     const bool staged = stage_tile(o, x64, i0, i1, S);
-    const int i = i0 + t;
-    if (i < i1) {
-      double acc = 0;
-      if (o.row[i]) {
-        const double sm = staged ? row_sum<kFmtRun8, 2, double, double, true>(o, i, S.x, S.adj)
-                                 : row_sum<kFmtRun8, 2, double>(o, i, x64);
-        acc = o.rhs[i] - (o.diag[i] * x64[i] - sm);
-      }
-      r64[i] = acc;
-      const V ri = (V)(acc * inv);
-      r[i] = ri;
-      d[0] += (double)ri * (double)ri;
-      d[1] += (double)rh[i] * (double)ri;
-      d[2] += acc * acc;
-    }
-  }
+    const int i = i0 + t / G;
+    if (i >= i1) return;
+    double s = 0;
+    const bool on = o.row[i] != 0;
+    if (on)
+      s = group_sum<G>(staged ? row_sum<kFmtRun8, 2, double, double, true, G>(o, i, S.x, S.adj)
+                              : row_sum<kFmtRun8, 2, double, double, false, G>(o, i, x64));
+    if (G > 1 && (t & (G - 1)) != 0) return;
+    const double acc = on ? o.rhs[i] - (o.diag[i] * x64[i] - s) : 0.0;
+    r64[i] = acc;
+    const V ri = (V)(acc * inv);
+    r[i] = ri;
+    d[0] += (double)ri * (double)ri;
+    d[1] += (double)rh[i] * (double)ri;
+    d[2] += acc * acc;
+  });
   block_partials<3>(d, partials);
 }
 
@@ -1209,7 +1225,7 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_fold(int n, const int* row, 
 
 // true residual after a fold: r64 = rhs - A x64 (full precision),
 // r = r64 / xscale; partials (r, r), (rh, r), (r64, r64)
-template <int FMT, int CMF, typename V>
+template <int FMT, int CMF, typename V, int G>
 __global__ __launch_bounds__(kRedThreads) void k_bi_true(PpeOp o, const double* __restrict__ x64,
                                                          double* __restrict__ r64, V* __restrict__ r,
                                                          const V* __restrict__ rh, double* partials,
@@ -1217,20 +1233,22 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_true(PpeOp o, const double* 
   if (st->done || !st->update) return;
   const double inv = 1.0 / st->xscale;
   double d[3] = {0.0, 0.0, 0.0};
-  for (RowIter it = xcd_rows(o.n); it.i < it.end; it.i += it.stride) {
-    const int i = it.i;
-    double acc = 0;
-    if (o.row[i]) {
-      const double s = row_sum<FMT, CMF, double>(o, i, x64);
-      acc = o.rhs[i] - (o.diag[i] * x64[i] - s);
-    }
+  const int t = (int)threadIdx.x;
+  lane_rows<G>(o.n, [&](int i0, int i1) {
+    const int i = i0 + t / G;
+    if (i >= i1) return;
+    double s = 0;
+    const bool on = o.row[i] != 0;
+    if (on) s = group_sum<G>(row_sum<FMT, CMF, double, double, false, G>(o, i, x64));
+    if (G > 1 && (t & (G - 1)) != 0) return;
+    const double acc = on ? o.rhs[i] - (o.diag[i] * x64[i] - s) : 0.0;
     r64[i] = acc;
     const V ri = (V)(acc * inv);
     r[i] = ri;
     d[0] += (double)ri * (double)ri;
     d[1] += (double)rh[i] * (double)ri;
     d[2] += acc * acc;
-  }
+  });
   block_partials<3>(d, partials);
 }
 
@@ -1386,6 +1404,16 @@ int win_grid(int n, int G) { return grid_rows((int)std::min<int64_t>((int64_t)n 
   } while (0)
 int win_blocks(int n) { return win_grid(n, win_group(n)); }
 
+// f(lanes as an integral constant) by row_lanes
+template <class F>
+void with_row_lanes(int n, F&& f) {
+  if (row_lanes(n) == 1) f(std::integral_constant<int, 1>{});
+  else f(std::integral_constant<int, 4>{});
+}
+
+// blocks (and reduction partials) of an operator pass
+int op_blocks(const PpeOp& o) { return o.fmt == kFmtWin ? win_blocks(o.n) : win_grid(o.n, row_lanes(o.n)); }
+
 void launch_win_mv(hipStream_t s, const PpeOp& o, const float* x, float* y, const float* wv, const WinCoarse& cz,
                    const PpeWork& w, const BiState* st) {
   const int G = win_group(o.n), g = win_grid(o.n, G);
@@ -1399,16 +1427,16 @@ void launch_win_mv(hipStream_t s, const PpeOp& o, const float* x, float* y, cons
 // y = A x in full precision by the operator's format
 void launch_apply_full(hipStream_t s, const PpeWork& w, const PpeOp& o, const double* x, double* y, bool residual,
                        bool norm) {
-  int G = w.nbg;
+  const int G = op_blocks(o);
   if (o.fmt == kFmtWin) {
     WIN_LAUNCH(k_win_apply, w.n, o, x, y, residual, norm, w.partials);
-    G = win_blocks(w.n);
-  } else if (o.fmt == kFmtRun8) {
-    k_apply_staged<<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
-  } else if (w.mixed) {
-    k_apply_full<kFmtIdx32, 1><<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
   } else {
-    k_apply_full<kFmtIdx32, 2><<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
+    with_row_lanes(w.n, [&](auto gl) {
+      constexpr int L = decltype(gl)::value;
+      if (o.fmt == kFmtRun8) k_apply_staged<L><<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
+      else if (w.mixed) k_apply_full<kFmtIdx32, 1, L><<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
+      else k_apply_full<kFmtIdx32, 2, L><<<G, kRedThreads, 0, s>>>(o, x, y, residual, norm, w.partials);
+    });
   }
   if (norm) launch_fin(s, w, kFinNorm, nullptr, G);
 }
@@ -1750,7 +1778,7 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
     tm->count(mv_all);
     return (w.mv_seq++ % kMvSample) == 0 ? tm : nullptr;
   };
-  const int Gm = FMT == kFmtWin ? win_blocks(n) : G;  // blocks of the operator passes
+  const int Gm = op_blocks(o);  // blocks of the operator passes
   // With the two-level preconditioner the window-staged matvec of a run that
   // launches bound adds the coarse correction to its operand and leaves the sum
   // in phc / shc: an iteration goes 85.0 -> 77 us at 4,200 rows and 123.7 -> 121.2
@@ -1762,8 +1790,13 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
   V* shc = fused ? (V*)w.vec[9] : sh;
   auto matvec = [&](const V* x, V* y, const V* ww, V* xc) {
     if constexpr (kWin) launch_win_mv(s, o, x, y, ww, fused ? WinCoarse{cw->y, xc, cw->AX, cw->AY} : WinCoarse{}, w, st);
-    else if constexpr (FMT == kFmtRun8) k_bi_mv_staged<V><<<G, kRedThreads, 0, s>>>(o, x, y, ww, w.partials, st);
-    else k_bi_mv<FMT, CM, V><<<G, kRedThreads, 0, s>>>(o, x, y, ww, w.partials, st);
+    else
+      with_row_lanes(n, [&](auto gl) {
+        constexpr int L = decltype(gl)::value;
+        if constexpr (FMT == kFmtRun8)
+          k_bi_mv_staged<V, L><<<Gm, kRedThreads, 0, s>>>(o, x, y, ww, w.partials, st);
+        else k_bi_mv<FMT, CM, V, L><<<Gm, kRedThreads, 0, s>>>(o, x, y, ww, w.partials, st);
+      });
   };
   int chunk = 8;
   BiState h{};
@@ -1796,9 +1829,13 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
       launch_fin(s, w, kFinRho);
       if constexpr (!kWin) k_bi_fold<V><<<G, kRedThreads, 0, s>>>(n, w.row, w.x64, xs, st);
       if constexpr (kWin) WIN_LAUNCH(k_win_true, n, o, w.x64, w.x64b, xs, w.r64, r, rh, w.partials, st);
-      else if constexpr (FMT == kFmtRun8)
-        k_bi_true_staged<V><<<G, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
-      else k_bi_true<FMT, CMF, V><<<G, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
+      else
+        with_row_lanes(n, [&](auto gl) {
+          constexpr int L = decltype(gl)::value;
+          if constexpr (FMT == kFmtRun8)
+            k_bi_true_staged<V, L><<<Gm, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
+          else k_bi_true<FMT, CMF, V, L><<<Gm, kRedThreads, 0, s>>>(o, w.x64, w.r64, r, rh, w.partials, st);
+        });
       launch_fin(s, w, kFinTrue, nullptr, Gm);
     }
     HIP_TRY(hipGetLastError());
