@@ -8,10 +8,10 @@
 // computed transposed so that the 16 MFMA columns are the 16 particles; the
 // per-particle sums then stay in registers (layout at the kernel).
 //
-// The backward kernel owns one particle per wave64 (grid-stride over
-// particles) and walks its neighbour list in tiles of 16 edges:
-//   layer 1  D[16 x 64] = E[16 x 32] W1^T[32 x 64]   4 x v_mfma_f32_16x16x32_bf16
-//            (the 6 edge inputs padded to K = 32 with zeros)
+// The backward kernel owns one particle per wave64, four waves per block, and
+// walks its neighbour list in tiles of 16 edges:
+//   layer 1  D[16 x 64] = E[16 x 16] W1^T[16 x 64]   4 x v_mfma_f32_16x16x16_bf16
+//            (the 6 edge inputs padded to K = 16 with zeros)
 //   layer 2  D[16 x 64] = H1[16 x 64] W2^T[64 x 64]  8 x v_mfma_f32_16x16x32_bf16
 // MFMA operand layout (16x16x32): lane l holds row (l mod 16) of A and
 // column (l mod 16) of B, K elements 8*(l/16) .. 8*(l/16)+7; the FP32
@@ -19,6 +19,18 @@
 // result is re-laid out into the layer-2 A operand through a 16 x 64 BF16
 // LDS tile.  The node MLP (64 x 64 per particle, 1/80 of the edge work)
 // runs on the VALU with the same BF16 weights.
+//
+// It is bound by the latency of each wave's chain of gathers, LDS tiles and
+// products, with as many waves as the FP32 accumulators leave room for:
+//   - a particle's edges are gathered 64 at a time, one per lane, into an LDS
+//     list that both passes read (by tiles of 16 lanes, in each pass: 1.58 ms
+//     for 64,000 rows; so, with W3 in padded LDS rows: 1.07 ms);
+//   - dW3 is shared by the four waves of a block, 16 rows each, and the W2
+//     operands lie in LDS, which brings the registers from over 400 to 256, two
+//     waves per SIMD (0.85 ms);
+//   - the XCDs take runs of particles by turns (0.79 ms).
+// Per-particle counts instead of sums for db2 and selects of a rounded dZ2 took
+// instructions out but no time.
 //
 // Backward recomputes the forward per particle (two passes over its edges)
 // and accumulates weight gradients with v_mfma_f32_16x16x16_bf16, whose A
@@ -38,18 +50,19 @@ typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-// Particles of this block: eight contiguous chunks, one per XCD (workgroups
-// are dealt to XCDs round robin), so the particles an XCD works on at one
-// time are consecutive and share their neighbour-list lines and neighbour
-// fields in that XCD's L2.  gridDim.x is a multiple of 8.
+// Particles of the backward kernel: one per wave, kBwdWaves per block, the
+// blocks of one XCD (workgroups are dealt to XCDs round robin) on consecutive
+// ones, so that they share neighbour fields in that XCD's L2.  The XCDs take such
+// runs by turns: with one eighth of the particles to each, those with more wall
+// particles, which have no row, stood idle for a quarter of the time.
+// gridDim.x is a multiple of 8; the trip count is the block's, not the wave's.
+constexpr int kBwdWaves = 4;
 struct PartIter {
-  int i, end, stride;
+  int i0, stride;
 };
-__device__ inline PartIter xcd_particles(int n) {
+__device__ inline PartIter xcd_particles() {
   const int x = blockIdx.x & 7, b = blockIdx.x >> 3, per = gridDim.x >> 3;
-  const int chunk = (n + 7) >> 3;
-  const int lo = x * chunk;
-  return PartIter{lo + b, min(n, lo + chunk), per};
+  return PartIter{(x * per + b) * kBwdWaves, (int)gridDim.x * kBwdWaves};
 }
 
 __device__ inline f4 mfma32(bf8 a, bf8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
@@ -60,145 +73,136 @@ struct Net {
   const float* master;  // biases are read in FP32
 };
 
-// B operands of layer 1 (B[k][n] = W1[n][k], k < 6) and layer 2
-// (B[k][n] = W2[n][k]) for this lane
-__device__ inline void load_fwd_operands(const Net& net, int lane, bf8 (&B1)[4], bf8 (&B2)[4][2]) {
-  const int kq = 8 * (lane >> 4), nl = lane & 15;
+// Operands of the backward kernel's W2 products, a lane's 16 bytes each, in LDS
+// and shared by the block's waves: fragments 2 nb, 2 nb + 1 of layer 2 (B[k][n] =
+// W2[n][k], n = nl + 16 nb) and 8 + 2 kb, 8 + 2 kb + 1 of dH1 = dZ2 W2 (B[k = n]
+// [col] = W2[n][col], col = nl + 16 kb)
+typedef bf8 W2Frags[16][64];
+
+__device__ inline void load_w2_frags(const Net& net, int frag, int lane, W2Frags& F) {
+  const int nl = lane & 15, c = nl + 16 * ((frag & 7) >> 1), k0 = 8 * (lane >> 4) + 32 * (frag & 1);
+  bf8 t;
 #pragma unroll
-  for (int nb = 0; nb < 4; nb++) {
-    const int nn = nl + 16 * nb;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int k = kq + j;
-      B1[nb][j] = k < kEin ? net.wbf[OFF_W1 + nn * kEin + k] : (__bf16)0.0f;
-      B2[nb][0][j] = net.wbf[OFF_W2 + nn * kH + k];
-      B2[nb][1][j] = net.wbf[OFF_W2 + nn * kH + 32 + k];
-    }
-  }
+  for (int j = 0; j < 8; j++) t[j] = net.wbf[OFF_W2 + (frag < 8 ? c * kH + k0 + j : (k0 + j) * kH + c)];
+  F[frag][lane] = t;
 }
 
-template <typename R>
-struct EdgeTile {
-  bf8 a1;            // layer-1 A operand (lanes 0-15 carry the 6 inputs)
-  uint32_t valid;    // bit e: edge e of the tile exists
+// Edge inputs of up to kEdgeBuf edges of one particle in LDS: row e holds the
+// six BF16 inputs of edge e and two zeros (one 16-byte read is a lane's part of
+// the layer-1 A operand).
+constexpr int kEdgeBuf = 128;
+struct EdgeList {
+  bf8 e[kEdgeBuf];
 };
 
-// inputs of edge (i, j): (x_i - x_j)/h_i, |x_i - x_j|/h_i, rho_j/rho_f, s_j
+// Gathers edges base .. base + kEdgeBuf - 1 of particle i, one edge per lane and
+// round; returns in valid[q] the edges 64 q + lane that exist.  Inputs of edge
+// (i, j): (x_i - x_j)/h_i, |x_i - x_j|/h_i, rho_j/rho_f, s_j.
 template <typename R>
-__device__ inline EdgeTile<R> edge_tile(const SphView<R>& v, const float2* nf, int i, int c, int cnt, int lane,
-                                        float ein[kEin]) {
-  EdgeTile<R> t;
-  for (int q = 0; q < 8; q++) t.a1[q] = (__bf16)0.0f;
-  for (int q = 0; q < kEin; q++) ein[q] = 0.f;
-  bool ok = false;
-  if (lane < 16) {
-    const int e = c * 16 + lane;
+__device__ inline void gather_edges(const SphView<R>& v, const float2* nf, int i, int base, int cnt, int lane,
+                                    EdgeList& E, uint64_t (&valid)[2]) {
+  const double ih = 1.0 / v.h[i];
+  const double xi = v.x[i], yi = v.y[i], zi = v.z[i];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    valid[q] = 0;
+    if (base + 64 * q >= cnt) continue;
+    const int e = base + 64 * q + lane;
+    bool ok = false;
+    bf8 t;
+    for (int k = 0; k < 8; k++) t[k] = (__bf16)0.0f;
     if (e < cnt) {
       const uint32_t ent = v.nbr[nbr_slot(e, i, v.n)];
       if (!(ent & kNbrFlag)) {
         const int j = (int)ent;
-        const double ih = 1.0 / v.h[i];
         double ex, ey, ez;
-        pdiff(v, v.x[i], v.y[i], v.z[i], j, ex, ey, ez);
+        pdiff(v, xi, yi, zi, j, ex, ey, ez);
         const double dx = ex * ih, dy = ey * ih, dz = ez * ih;
         const float2 f = nf[j];
-        ein[0] = (float)dx;
-        ein[1] = (float)dy;
-        ein[2] = (float)dz;
-        ein[3] = (float)sqrt(dx * dx + dy * dy + dz * dz);
-        ein[4] = f.x;
-        ein[5] = f.y;
+        t[0] = (__bf16)(float)dx;
+        t[1] = (__bf16)(float)dy;
+        t[2] = (__bf16)(float)dz;
+        t[3] = (__bf16)(float)sqrt(dx * dx + dy * dy + dz * dz);
+        t[4] = (__bf16)f.x;
+        t[5] = (__bf16)f.y;
         ok = true;
       }
     }
-    for (int q = 0; q < kEin; q++) t.a1[q] = (__bf16)ein[q];
+    E.e[64 * q + lane] = t;
+    valid[q] = __ballot(ok);
   }
-  t.valid = (uint32_t)(__ballot(ok) & 0xffffull);
-  return t;
+}
+
+// layer-1 A operand of tile c of the gathered edges (16x16x16 layout: row l mod
+// 16, inputs 4 (l / 16) .. +3, of which 8 .. 15 are zero) and its edge mask
+__device__ inline bf4 edge_operand(const EdgeList& E, int c, int lane) {
+  bf4 a;
+  for (int k = 0; k < 4; k++) a[k] = (__bf16)0.0f;
+  if (lane < 32) a = reinterpret_cast<const bf4*>(&E.e[16 * c + (lane & 15)])[lane >> 4];
+  return a;
+}
+__device__ inline uint32_t edge_mask(const uint64_t (&valid)[2], int c) {
+  return (uint32_t)((c < 4 ? valid[0] : valid[1]) >> (16 * (c & 3))) & 0xffffu;
 }
 
 // layer 1 + ReLU for one tile; z1 in result layout, H (LDS) gets BF16 h1
-__device__ inline void layer1(const Net& net, const bf8 (&B1)[4], bf8 a1, int lane, f4 (&h1)[4], __bf16 (*H)[kH + 8]) {
+__device__ inline void layer1(const float (&b1)[4], const bf4 (&B1)[4], bf4 a1, int lane, bf4 (&h1)[4],
+                              __bf16 (*H)[kH + 8]) {
   const int nl = lane & 15, er = 4 * (lane >> 4);
 #pragma unroll
   for (int nb = 0; nb < 4; nb++) {
     f4 z = {0.f, 0.f, 0.f, 0.f};
-    z = mfma32(a1, B1[nb], z);
-    const float b = net.master[OFF_B1 + nl + 16 * nb];
+    z = mfma16(a1, B1[nb], z);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      float hv = fmaxf(z[r] + b, 0.f);
+      float hv = fmaxf(z[r] + b1[nb], 0.f);
       __bf16 hb = (__bf16)hv;
-      h1[nb][r] = (float)hb;
+      h1[nb][r] = hb;
       H[er + r][nl + 16 * nb] = hb;
     }
   }
 }
 
 // layer 2 pre-activation for one tile (A operand read back from H)
-__device__ inline void layer2(const bf8 (&B2)[4][2], int lane, __bf16 (*H)[kH + 8], f4 (&z2)[4]) {
-  bf8 a0, a1;
+__device__ inline void layer2(const W2Frags& F, int lane, __bf16 (*H)[kH + 8], f4 (&z2)[4]) {
   const int e = lane & 15, kq = 8 * (lane >> 4);
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    a0[j] = H[e][kq + j];
-    a1[j] = H[e][32 + kq + j];
-  }
+  const bf8 a0 = *reinterpret_cast<const bf8*>(&H[e][kq]), a1 = *reinterpret_cast<const bf8*>(&H[e][32 + kq]);
 #pragma unroll
   for (int nb = 0; nb < 4; nb++) {
     f4 z = {0.f, 0.f, 0.f, 0.f};
-    z = mfma32(a0, B2[nb][0], z);
-    z = mfma32(a1, B2[nb][1], z);
+    z = mfma32(a0, F[2 * nb][lane], z);
+    z = mfma32(a1, F[2 * nb + 1][lane], z);
     z2[nb] = z;
   }
 }
 
-// node MLP forward: z3 = W3 m + b3 (lane l = output l), y = W4 relu(z3) + b4
-__device__ inline float node_forward(const Net& net, const float* Ms, const __bf16* W3s, int lane, float& z3) {
-  float z = net.master[OFF_B3 + lane];
-  for (int k = 0; k < kH; k++) z += (float)W3s[lane * kH + k] * Ms[k];
-  z3 = z;
-  float g = fmaxf(z, 0.f);
-  float y = (float)net.wbf[OFF_W4 + lane] * g;
-  for (int off = 32; off > 0; off >>= 1) y += __shfl_xor(y, off);
-  return y + net.master[OFF_B4];
+// Lanes of one wave exchange the edge inputs through LDS.  A wave's LDS
+// instructions execute in issue order, so ordering the compiler's code
+// motion with wavefront-scope fences is all the synchronisation needed.
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Forward over the edges of particle i: returns the aggregated message
-// (ready in Ms, LDS) -- shared by the forward and backward kernels.
-template <typename R>
-__device__ inline void aggregate(const Net& net, const SphView<R>& v, const float2* nf, int i, int lane,
-                                 const bf8 (&B1)[4], const bf8 (&B2)[4][2], __bf16 (*H)[kH + 8], float* Ms) {
-  const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
-  const int nl = lane & 15, er = 4 * (lane >> 4);
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  float ein[kEin];
-  for (int c = 0; c * 16 < cnt; c++) {
-    EdgeTile<R> t = edge_tile(v, nf, i, c, cnt, lane, ein);
-    f4 h1[4];
-    layer1(net, B1, t.a1, lane, h1, H);
-    __syncthreads();
-    f4 z2[4];
-    layer2(B2, lane, H, z2);
+// Rows of W3 and of its transpose in LDS: 144 bytes, so the 16-byte reads of
+// the 16 lanes of a quarter wave fall on different banks
+constexpr int kW3Row = kH + 8;
+
+// node MLP forward: z3 = W3 m + b3 (lane l = output l), y = W4 relu(z3) + b4
+__device__ inline float node_forward(const float* Ms, const __bf16 (*W3s)[kW3Row], int lane, float b3, float w4,
+                                     float b4, float& z3) {
+  float z = b3;
+#pragma unroll 2
+  for (int k8 = 0; k8 < kH; k8 += 8) {
+    const bf8 w = *reinterpret_cast<const bf8*>(&W3s[lane][k8]);
 #pragma unroll
-    for (int nb = 0; nb < 4; nb++) {
-      const float b = net.master[OFF_B2 + nl + 16 * nb];
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        if ((t.valid >> (er + r)) & 1u) acc[nb] += fmaxf(z2[nb][r] + b, 0.f);
-    }
-    __syncthreads();
+    for (int k = 0; k < 8; k++) z += (float)w[k] * Ms[k8 + k];
   }
-#pragma unroll
-  for (int nb = 0; nb < 4; nb++) {
-    acc[nb] += __shfl_xor(acc[nb], 16);
-    acc[nb] += __shfl_xor(acc[nb], 32);
-  }
-  if (lane < 16) {
-#pragma unroll
-    for (int nb = 0; nb < 4; nb++) Ms[lane + 16 * nb] = acc[nb] * (1.0f / 64.0f);
-  }
-  __syncthreads();
+  z3 = z;
+  float y = w4 * fmaxf(z, 0.f);
+  for (int off = 32; off > 0; off >>= 1) y += __shfl_xor(y, off);
+  return y + b4;
 }
 
 // Forward kernel, weights as the A operand.  Each layer is computed
@@ -260,15 +264,6 @@ __device__ inline uint32_t relu_pk_bf16(float a, float b) {
   const s2 v = __builtin_bit_cast(s2, __builtin_convertvector(f, bf2));
   const s2 z = {0, 0};
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(v, z));
-}
-
-// Lanes of one wave exchange the edge inputs through LDS.  A wave's LDS
-// instructions execute in issue order, so ordering the compiler's code
-// motion with wavefront-scope fences is all the synchronisation needed.
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 constexpr int kFwdWaves = 4;    // waves per block of the forward kernel
@@ -460,32 +455,51 @@ __global__ __launch_bounds__(64 * kFwdWaves, 4) void k_mlp_forward(Net net, SphV
 }
 
 template <typename R>
-__global__ __launch_bounds__(64) void k_mlp_backward(Net net, SphView<R> v, const float2* __restrict__ nf,
+__global__ __launch_bounds__(64 * kBwdWaves, 2) void k_mlp_backward(Net net, SphView<R> v, const float2* __restrict__ nf,
                                                       const int* __restrict__ row, const double* __restrict__ pprev,
                                                       const double* __restrict__ target, double inv_scale,
                                                       float inv_rows, float* __restrict__ partials) {
-  __shared__ __bf16 H[16][kH + 8];
-  __shared__ __bf16 DZ[16][kH + 8];
-  __shared__ __bf16 EIN[16][16];
-  __shared__ float Ms[kH];
-  __shared__ float DG[kH];
-  __shared__ float DM[kH];
-  __shared__ __bf16 W3s[kH * kH];
-  const int lane = threadIdx.x;
+  struct Work {
+    W2Frags F;
+    EdgeList E[kBwdWaves];
+    alignas(16) __bf16 H[kBwdWaves][16][kH + 8];
+    alignas(16) __bf16 DZ[kBwdWaves][16][kH + 8];
+    alignas(16) __bf16 W3s[kH][kW3Row];  // W3[l][k]
+    alignas(16) __bf16 W3t[kH][kW3Row];  // W3[l][k] at [k][l]
+    alignas(16) float DM[kBwdWaves][kH];
+    alignas(16) float Ms[2][kBwdWaves][kH];  // by turns, so that one barrier an iteration is enough
+    alignas(16) float DG[2][kBwdWaves][kH];
+  };
+  __shared__ union {
+    Work w;
+    float grad[kNParam + 1];  // the block's partial gradient, after the loop
+  } sh;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nl = lane & 15, er = 4 * (lane >> 4), kq = 8 * (lane >> 4);
-  for (int q = lane; q < kH * kH; q += 64) W3s[q] = net.wbf[OFF_W3 + q];
-  bf8 B1[4], B2[4][2];
-  load_fwd_operands(net, lane, B1, B2);
-  // B operand of dH1 = dZ2 W2: B[k = n][col = kout] = W2[n][kout]
-  bf8 Bt[4][2];
+  auto& W3s = sh.w.W3s;
+  auto& W3t = sh.w.W3t;
+  W2Frags& F = sh.w.F;
+  EdgeList& E = sh.w.E[wave];
+  auto& H = sh.w.H[wave];
+  auto& DZ = sh.w.DZ[wave];
+  auto& DM = sh.w.DM[wave];
+  for (int q = threadIdx.x; q < kH * kH; q += 64 * kBwdWaves) {
+    const __bf16 w = net.wbf[OFF_W3 + q];
+    W3s[q / kH][q % kH] = w;
+    W3t[q % kH][q / kH] = w;
+  }
+  for (int f = wave; f < 16; f += kBwdWaves) load_w2_frags(net, f, lane, F);
+  bf4 B1[4];  // B[k][n] = W1[n][k], k < 6
+  float b1[4], b2[4];
 #pragma unroll
-  for (int kb = 0; kb < 4; kb++)
+  for (int kb = 0; kb < 4; kb++) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      Bt[kb][0][j] = net.wbf[OFF_W2 + (kq + j) * kH + nl + 16 * kb];
-      Bt[kb][1][j] = net.wbf[OFF_W2 + (32 + kq + j) * kH + nl + 16 * kb];
-    }
-  const float w4 = (float)net.wbf[OFF_W4 + lane];
+    for (int j = 0; j < 4; j++)
+      B1[kb][j] = er + j < kEin ? net.wbf[OFF_W1 + (nl + 16 * kb) * kEin + er + j] : (__bf16)0.0f;
+    b1[kb] = net.master[OFF_B1 + nl + 16 * kb];
+    b2[kb] = net.master[OFF_B2 + nl + 16 * kb];
+  }
+  const float w4 = (float)net.wbf[OFF_W4 + lane], b3 = net.master[OFF_B3 + lane], b4 = net.master[OFF_B4];
   __syncthreads();
 
   f4 gW2[16], gW1[4];
@@ -494,18 +508,53 @@ __global__ __launch_bounds__(64) void k_mlp_backward(Net net, SphView<R> v, cons
 #pragma unroll
   for (int q = 0; q < 4; q++) gW1[q] = (f4){0.f, 0.f, 0.f, 0.f};
   float gb1[4] = {0, 0, 0, 0}, gb2[4] = {0, 0, 0, 0};
-  float gW3[kH];
+  // rows 16 wave .. + 15 of dW3, column = lane
+  float gW3[16];
 #pragma unroll
-  for (int k = 0; k < kH; k++) gW3[k] = 0.f;
+  for (int k = 0; k < 16; k++) gW3[k] = 0.f;
   float gb3 = 0.f, gW4 = 0.f, gb4 = 0.f, loss = 0.f;
 
-  for (PartIter it = xcd_particles(v.n); it.i < it.end; it.i += it.stride) {
-    const int i = it.i;
-    if (!row[i]) continue;
-    // pass 1: forward
-    aggregate(net, v, nf, i, lane, B1, B2, H, Ms);
+  int turn = 0;
+  for (PartIter it = xcd_particles(); it.i0 < v.n; it.i0 += it.stride, turn ^= 1) {
+    const int i = it.i0 + wave;
+    const bool live = i < v.n && row[i];
+    float* Ms = sh.w.Ms[turn][wave];
+    float* DG = sh.w.DG[turn][wave];
+    const int cnt = live ? min(v.nbr_cnt[i], v.nbr_cap) : 0;
+    uint64_t valid[2] = {0, 0};
+    // pass 1: forward, the message summed over the edges
+    if (live) {
+      float acc[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int base = 0; base < cnt; base += kEdgeBuf) {
+        gather_edges(v, nf, i, base, cnt, lane, E, valid);
+        wave_lds_sync();
+        for (int c = 0; c < kEdgeBuf / 16 && base + c * 16 < cnt; c++) {
+          const uint32_t on = edge_mask(valid, c);
+          bf4 h1[4];
+          f4 z2[4];
+          layer1(b1, B1, edge_operand(E, c, lane), lane, h1, H);
+          wave_lds_sync();
+          layer2(F, lane, H, z2);
+#pragma unroll
+          for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+              if ((on >> (er + r)) & 1u) acc[nb] += fmaxf(z2[nb][r] + b2[nb], 0.f);
+          wave_lds_sync();
+        }
+      }
+#pragma unroll
+      for (int nb = 0; nb < 4; nb++) {
+        acc[nb] += __shfl_xor(acc[nb], 16);
+        acc[nb] += __shfl_xor(acc[nb], 32);
+      }
+      if (lane < 16) {
+#pragma unroll
+        for (int nb = 0; nb < 4; nb++) Ms[lane + 16 * nb] = acc[nb] * (1.0f / 64.0f);
+      }
+      wave_lds_sync();
     float z3;
-    const float y = node_forward(net, Ms, W3s, lane, z3);
+    const float y = node_forward(Ms, W3s, lane, b3, w4, b4, z3);
     const float t = (float)((target[i] - pprev[i]) * inv_scale);
     const float err = y - t;
     const float dy = 2.f * err * inv_rows;
@@ -517,122 +566,164 @@ __global__ __launch_bounds__(64) void k_mlp_backward(Net net, SphView<R> v, cons
     gW4 += dy * g;
     const float dg = z3 > 0.f ? dy * w4 : 0.f;
     gb3 += dg;
-#pragma unroll
-    for (int k = 0; k < kH; k++) gW3[k] += dg * Ms[k];
     DG[lane] = dg;
+    } else {
+      Ms[lane] = 0.f;
+      DG[lane] = 0.f;
+    }
+    // dW3 += dG M^T of the block's particles, each wave its 16 rows
     __syncthreads();
+#pragma unroll
+    for (int p = 0; p < kBwdWaves; p++) {
+      const float mk = sh.w.Ms[turn][p][lane];
+#pragma unroll
+      for (int r4 = 0; r4 < 16; r4 += 4) {
+        const float4 d = *reinterpret_cast<const float4*>(&sh.w.DG[turn][p][16 * wave + r4]);
+        gW3[r4 + 0] += d.x * mk;
+        gW3[r4 + 1] += d.y * mk;
+        gW3[r4 + 2] += d.z * mk;
+        gW3[r4 + 3] += d.w * mk;
+      }
+    }
+    if (!live) continue;
     {
       float dm = 0.f;
-      for (int l = 0; l < kH; l++) dm += (float)W3s[l * kH + lane] * DG[l];
+#pragma unroll 2
+      for (int l8 = 0; l8 < kH; l8 += 8) {
+        const bf8 w = *reinterpret_cast<const bf8*>(&W3t[lane][l8]);
+#pragma unroll
+        for (int l = 0; l < 8; l++) dm += (float)w[l] * DG[l8 + l];
+      }
       DM[lane] = dm * (1.0f / 64.0f);
     }
-    __syncthreads();
-    // pass 2: edge backward
-    const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
-    float ein[kEin];
-    for (int c = 0; c * 16 < cnt; c++) {
-      EdgeTile<R> tt = edge_tile(v, nf, i, c, cnt, lane, ein);
-      if (lane < 16)
-        for (int q = 0; q < 16; q++) EIN[lane][q] = q < kEin ? (__bf16)ein[q] : (__bf16)0.0f;
-      f4 h1[4];
-      layer1(net, B1, tt.a1, lane, h1, H);
-      __syncthreads();
-      f4 z2[4];
-      layer2(B2, lane, H, z2);
-      // dZ2 in result layout; edges outside the list contribute nothing
-      f4 dz2[4];
+    wave_lds_sync();
+    float dmv[4];
 #pragma unroll
-      for (int nb = 0; nb < 4; nb++) {
-        const float b = net.master[OFF_B2 + nl + 16 * nb];
-        const float dmv = DM[nl + 16 * nb];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const bool on = ((tt.valid >> (er + r)) & 1u) && (z2[nb][r] + b > 0.f);
-          const float d = on ? dmv : 0.f;
-          dz2[nb][r] = d;
-          gb2[nb] += d;
-          DZ[er + r][nl + 16 * nb] = (__bf16)d;
-        }
+    for (int nb = 0; nb < 4; nb++) dmv[nb] = DM[nl + 16 * nb];
+    // pass 2: edge backward; a list of up to kEdgeBuf edges is still in E
+    for (int base = 0; base < cnt; base += kEdgeBuf) {
+      if (cnt > kEdgeBuf) {
+        gather_edges(v, nf, i, base, cnt, lane, E, valid);
+        wave_lds_sync();
       }
-      // dW2 tiles: A = dZ2 (rows n, K = edges), B = H1 (K = edges, cols k)
+      for (int c = 0; c < kEdgeBuf / 16 && base + c * 16 < cnt; c++) {
+        const uint32_t valid16 = edge_mask(valid, c);
+        bf4 h1[4];
+        layer1(b1, B1, edge_operand(E, c, lane), lane, h1, H);
+        wave_lds_sync();
+        f4 z2[4];
+        layer2(F, lane, H, z2);
+        // dZ2 in result layout; edges outside the list contribute nothing
+        f4 dz2[4];
 #pragma unroll
-      for (int nb = 0; nb < 4; nb++) {
-        bf4 a;
-        for (int r = 0; r < 4; r++) a[r] = (__bf16)dz2[nb][r];
+        for (int nb = 0; nb < 4; nb++) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const bool on = ((valid16 >> (er + r)) & 1u) && (z2[nb][r] + b2[nb] > 0.f);
+            const float d = on ? dmv[nb] : 0.f;
+            dz2[nb][r] = d;
+            gb2[nb] += d;
+            DZ[er + r][nl + 16 * nb] = (__bf16)d;
+          }
+        }
+        // dW2 tiles: A = dZ2 (rows n, K = edges), B = H1 (K = edges, cols k)
+#pragma unroll
+        for (int nb = 0; nb < 4; nb++) {
+          bf4 a;
+          for (int r = 0; r < 4; r++) a[r] = (__bf16)dz2[nb][r];
+#pragma unroll
+          for (int kb = 0; kb < 4; kb++) gW2[nb * 4 + kb] = mfma16(a, h1[kb], gW2[nb * 4 + kb]);
+        }
+        wave_lds_sync();
+        // dH1 = dZ2 W2 (A from the DZ tile), then dZ1 through the ReLU
+        const bf8 ad0 = *reinterpret_cast<const bf8*>(&DZ[nl][kq]);
+        const bf8 ad1 = *reinterpret_cast<const bf8*>(&DZ[nl][32 + kq]);
+        bf4 be;
+        for (int r = 0; r < 4; r++)
+          be[r] = nl < 8 ? reinterpret_cast<const __bf16*>(&E.e[16 * c + er + r])[nl & 7] : (__bf16)0.0f;
 #pragma unroll
         for (int kb = 0; kb < 4; kb++) {
-          bf4 b;
-          for (int r = 0; r < 4; r++) b[r] = (__bf16)h1[kb][r];
-          gW2[nb * 4 + kb] = mfma16(a, b, gW2[nb * 4 + kb]);
+          f4 dh = {0.f, 0.f, 0.f, 0.f};
+          dh = mfma32(ad0, F[8 + 2 * kb][lane], dh);
+          dh = mfma32(ad1, F[8 + 2 * kb + 1][lane], dh);
+          bf4 a;
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const bool on = ((valid16 >> (er + r)) & 1u) && (float)h1[kb][r] > 0.f;
+            const float d = on ? dh[r] : 0.f;
+            gb1[kb] += d;
+            a[r] = (__bf16)d;
+          }
+          gW1[kb] = mfma16(a, be, gW1[kb]);
         }
+        wave_lds_sync();
       }
-      __syncthreads();
-      // dH1 = dZ2 W2 (A from the DZ tile), then dZ1 through the ReLU
-      bf8 ad0, ad1;
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        ad0[j] = DZ[nl][kq + j];
-        ad1[j] = DZ[nl][32 + kq + j];
-      }
-      bf4 be;
-      for (int r = 0; r < 4; r++) be[r] = EIN[er + r][nl];
-#pragma unroll
-      for (int kb = 0; kb < 4; kb++) {
-        f4 dh = {0.f, 0.f, 0.f, 0.f};
-        dh = mfma32(ad0, Bt[kb][0], dh);
-        dh = mfma32(ad1, Bt[kb][1], dh);
-        bf4 a;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const bool on = ((tt.valid >> (er + r)) & 1u) && h1[kb][r] > 0.f;
-          const float d = on ? dh[r] : 0.f;
-          gb1[kb] += d;
-          a[r] = (__bf16)d;
-        }
-        gW1[kb] = mfma16(a, be, gW1[kb]);
-      }
-      __syncthreads();
     }
   }
-  // partial gradients of this block
+  // the block's partial gradient: the waves add theirs in turn
+  __syncthreads();
+  for (int q = threadIdx.x; q <= kNParam; q += 64 * kBwdWaves) sh.grad[q] = 0.f;
+  for (int w = 0; w < kBwdWaves; w++) {
+    __syncthreads();
+    if (wave == w) {
+      float* P = sh.grad;
+      auto put = [&](int q, float a) { P[q] += a; };
+#pragma unroll
+      for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) {
+          const int n = 16 * nb + er + jj;
+          if (nl < kEin) put(OFF_W1 + n * kEin + nl, gW1[nb][jj]);
+#pragma unroll
+          for (int kb = 0; kb < 4; kb++) put(OFF_W2 + n * kH + 16 * kb + nl, gW2[nb * 4 + kb][jj]);
+        }
+#pragma unroll
+      for (int nb = 0; nb < 4; nb++) {
+        float a = gb1[nb], b = gb2[nb];
+        a += __shfl_xor(a, 16);
+        a += __shfl_xor(a, 32);
+        b += __shfl_xor(b, 16);
+        b += __shfl_xor(b, 32);
+        if (lane < 16) {
+          put(OFF_B1 + lane + 16 * nb, a);
+          put(OFF_B2 + lane + 16 * nb, b);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; r++) P[OFF_W3 + (16 * w + r) * kH + lane] = gW3[r];
+      put(OFF_B3 + lane, gb3);
+      put(OFF_W4 + lane, gW4);
+      if (lane == 0) {
+        put(OFF_B4, gb4);
+        put(kNParam, loss);
+      }
+    }
+  }
+  __syncthreads();
   float* P = partials + (size_t)blockIdx.x * (kNParam + 1);
-#pragma unroll
-  for (int nb = 0; nb < 4; nb++)
-#pragma unroll
-    for (int jj = 0; jj < 4; jj++) {
-      const int n = 16 * nb + er + jj;
-      if (nl < kEin) P[OFF_W1 + n * kEin + nl] = gW1[nb][jj];
-#pragma unroll
-      for (int kb = 0; kb < 4; kb++) P[OFF_W2 + n * kH + 16 * kb + nl] = gW2[nb * 4 + kb][jj];
-    }
-#pragma unroll
-  for (int nb = 0; nb < 4; nb++) {
-    float a = gb1[nb], b = gb2[nb];
-    a += __shfl_xor(a, 16);
-    a += __shfl_xor(a, 32);
-    b += __shfl_xor(b, 16);
-    b += __shfl_xor(b, 32);
-    if (lane < 16) {
-      P[OFF_B1 + lane + 16 * nb] = a;
-      P[OFF_B2 + lane + 16 * nb] = b;
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < kH; k++) P[OFF_W3 + lane * kH + k] = gW3[k];
-  P[OFF_B3 + lane] = gb3;
-  P[OFF_W4 + lane] = gW4;
-  if (lane == 0) {
-    P[OFF_B4] = gb4;
-    P[kNParam] = loss;
-  }
+  for (int q = threadIdx.x; q <= kNParam; q += 64 * kBwdWaves) P[q] = sh.grad[q];
 }
 
-__global__ void k_reduce_partials(const float* __restrict__ partials, int nblocks, float* __restrict__ grad,
-                                  double* __restrict__ loss) {
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > kNParam) return;
+// Sum of the blocks' partial gradients in FP64, in a fixed order: 64 parameters
+// per block by 16 slices of the partials, so that they are read by 139
+// blocks of 16 waves (one thread per parameter walking 1024 partials of 35 KB took
+// 260 us, 139 waves with one load in flight each; now 6 us for 512).
+constexpr int kRedSlices = 16;
+__global__ __launch_bounds__(64 * kRedSlices) void k_reduce_partials(const float* __restrict__ partials, int nblocks,
+                                                                     float* __restrict__ grad,
+                                                                     double* __restrict__ loss) {
+  __shared__ double part[kRedSlices][64];
+  const int l = threadIdx.x & 63, sl = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + l;
   double s = 0;
-  for (int b = 0; b < nblocks; b++) s += partials[(size_t)b * (kNParam + 1) + p];
+  if (p <= kNParam) {
+#pragma unroll 8
+    for (int b = sl; b < nblocks; b += kRedSlices) s += partials[(size_t)b * (kNParam + 1) + p];
+  }
+  part[sl][l] = s;
+  __syncthreads();
+  if (sl != 0 || p > kNParam) return;
+  for (int q = 1; q < kRedSlices; q++) s += part[q][l];
   if (p < kNParam) grad[p] = (float)s;
   else *loss = s;
 }
@@ -841,9 +932,9 @@ int mlp_backward(hipStream_t s, const DevParams& P, const SphView<R>& v, Mlp& m,
   Net net{m.wbf, m.master};
   const int g = kMlpBwdBlocks;
   const double inv_scale = scale != 0 ? 1.0 / scale : 0.0;
-  k_mlp_backward<R><<<g, 64, 0, s>>>(net, v, m.nf, row, pprev, target, inv_scale, 1.0f / (float)n_rows,
+  k_mlp_backward<R><<<g, 64 * kBwdWaves, 0, s>>>(net, v, m.nf, row, pprev, target, inv_scale, 1.0f / (float)n_rows,
                                      m.partials);
-  k_reduce_partials<<<grid_for(kNParam + 1), kBlock, 0, s>>>(m.partials, g, m.grad, m.scal + 4);
+  k_reduce_partials<<<(kNParam + 1 + 63) / 64, 64 * kRedSlices, 0, s>>>(m.partials, g, m.grad, m.scal + 4);
   HIP_TRY(hipGetLastError());
   if (step) {
     m.adam_t += 1;

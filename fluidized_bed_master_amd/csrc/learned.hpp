@@ -18,7 +18,7 @@ constexpr int OFF_B3 = OFF_W3 + kH * kH;     // 64
 constexpr int OFF_W4 = OFF_B3 + kH;          // 64
 constexpr int OFF_B4 = OFF_W4 + kH;          // 1
 constexpr int kNParam = OFF_B4 + 1;          // 8833
-constexpr int kMlpBwdBlocks = 1024;          // persistent blocks of the backward pass
+constexpr int kMlpBwdBlocks = 512;            // persistent blocks of the backward pass, two per CU
 
 struct Mlp {
   bool ready = false;      // parameters set
