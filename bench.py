@@ -39,13 +39,13 @@ def _matvec_bytes(layout: dict, n_sph: int, fp32: bool) -> float:
     """Compulsory HBM bytes of one inner PPE matvec y = A x over the compact
     operator: every stored entry's coefficient and column index once (on the
     mixed path one 4-byte word holds both), and per particle the entry count
-    (4), run lengths (8), cell key (4), row flag (4), diagonal (4 FP32 inner
-    diagonal, 8 FP64), own x, y and the fused dot operand (3 vector words);
-    the neighbour gathers of x hit the cache and count once through the
-    own-x read."""
+    (4), cell key (4), row flag (4), diagonal (4 FP32 inner diagonal, 8 FP64),
+    own x, y and the fused dot operand (3 vector words), on the FP64 path the
+    run lengths (8) too; the neighbours' x are staged from the same streams and
+    count once through the own-x read."""
     vec = 4 if fp32 else 8
     coef = layout["coef_bytes"] if fp32 else 8
-    return layout["nnz"] * (coef + layout["index_bytes"]) + n_sph * ((24.0 if fp32 else 28.0) + 3 * vec)
+    return layout["nnz"] * (coef + layout["index_bytes"]) + n_sph * ((16.0 if fp32 else 28.0) + 3 * vec)
 
 
 def run_gpu(params, parts, precision, ppe_opts, steps, warmup, timers=False, mlp_weights=None, keep_pressure=False,
@@ -263,7 +263,7 @@ def main(argv=None) -> int:
             ab = _matvec_bytes(layout, n_sph, fp32=True)
             avg_s = tot_all / real / 1e3
             ach = ab / avg_s / 1e9
-            roofline = {"bound": "hbm", "kernel": "k_bi_mv_staged (inner FP32 matvec)", "achieved": round(ach, 1),
+            roofline = {"bound": "hbm", "kernel": "k_win_mv (inner FP32 matvec)", "achieved": round(ach, 1),
                         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                         "traffic": _pmc_traffic() if a.config == "c5_1m" else None,
                         "traffic_source": str(PMC_FILE.relative_to(ROOT)) if a.config == "c5_1m" else None,

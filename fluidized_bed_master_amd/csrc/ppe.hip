@@ -30,7 +30,7 @@
 // last fold ("reliable updates", Sleijpen & van der Vorst 1996), so the
 // Krylov space is never restarted.  All scalars stay on the device; every
 // reduction is two-stage and deterministic (per-block partials summed in a
-// fixed order by the last block to finish).  The host checks convergence
+// fixed order by a one-block kernel).  The host checks convergence
 // once per chunk of iterations.
 #include "ppe.hpp"
 #include "nbr.hpp"
@@ -522,7 +522,7 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
   }
   const Kgc<double> K(P.kgc == 1, v.cm, n, i);
   double bd = 0, Aij = 0, AP = 0, lag = 0;  // bd: -div of eps u
-  double dcomp = 0;  // sum over stored columns of a - hi16(a) (mixed)
+  double dcomp = 0;  // sum over stored columns of a - hi (mixed)
   int kc = 0, run = 0;
   uint64_t rcw = 0;
   uint32_t word = 0;

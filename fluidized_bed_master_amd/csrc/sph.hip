@@ -1,11 +1,10 @@
 // SPH stage kernels of the ISPH step on gfx950.
 //
-// One thread per particle.  Pair loops walk the neighbour list built at
-// NNPS (slot-major, so the k-th neighbour of 64 consecutive particles is one
-// coalesced 256 B read); the list keeps the reference's cell visiting order,
-// so sums are accumulated in the same order as the reference kernels.
-// Neighbour fields are gathered from SoA streams of cell-sorted particles;
-// spatial locality of the sort keeps those gathers in L2.
+// Pair loops walk the neighbour list built at NNPS (chunks of 8 slots per
+// particle), one to eight lanes per particle by its count (pair_lanes); the list
+// keeps the reference's cell visiting order, and a lane adds its share of the
+// slots in that order.  Neighbour fields are gathered from SoA streams or packed
+// records of cell-sorted particles; the sort keeps those gathers in L2.
 //
 // Each kernel cites the reference kernel it computes.
 #include "common.hpp"

@@ -469,13 +469,13 @@ int sophia_ppe_apply(sophia_ctx* ctx, const double* x, double* y, int32_t n);
  * the neighbour list and the position records.  y = A x (FP32 arithmetic,
  * sorted order, SPH count) and the mean device time of `reps` launches after
  * one untimed one.  Needs a mixed-precision context with an assembled
- * operator in run-offset format (row-major cell keys). */
+ * operator in the compact format (row-major cell keys). */
 int sophia_ppe_matvec_probe(sophia_ctx* ctx, int32_t variant, int32_t reps, const double* x, double* y,
                             int32_t n, double* us_per_launch);
 /* storage of the assembled operator: stored entries, bytes per column index
- * (1: u8 offset inside a cell run, 4: u32 index, 0: the u8 offset rides in
- * the low byte of the FP32 inner coefficient, whose significand is rounded
- * to 16 bits) and per coefficient as read by the inner iterations (4: FP32,
+ * (1: u8 offset inside a cell run, 4: u32 index, 0: an 11-bit slot in the
+ * row's 27-cell window rides in the word of the inner coefficient, whose
+ * significand is rounded to 16 bits) and per coefficient as read by the inner iterations (4: FP32,
  * 8: FP64).  Any may be NULL. */
 int sophia_ppe_layout(const sophia_ctx* ctx, int64_t* nnz, int32_t* index_bytes, int32_t* coef_bytes);
 /* Coarse operator of the last two-level solve (no reference counterpart;
