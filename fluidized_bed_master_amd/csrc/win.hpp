@@ -12,7 +12,7 @@
 // x-runs) this takes the eight compares and selects per entry that find the
 // run out of the inner loop, and it works across a periodic wrap.
 //
-// Bound: the operator stream from HBM (4 B per entry) plus 36 B per row; the
+// Bound: the operator stream from HBM (4 B per entry) plus 28 B per row; the
 // staging reads about 11 values per row from L2.
 #pragma once
 
