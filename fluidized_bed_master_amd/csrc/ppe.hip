@@ -47,7 +47,7 @@ namespace {
 
 constexpr int kRedThreads = 256;
 constexpr int kMaxGrid = 2048;  // 8 XCDs x 256 blocks
-enum { kFlagOffset = 1u, kFlagRunCount = 2u, kFlagOrder = 4u };
+enum { kFlagOffset = 1u, kFlagRunCount = 2u, kFlagOrder = 4u, kFlagRange = 8u };
 
 int grid_rows(int n) {
   int g = grid_for(n > 0 ? n : 1, kRedThreads);
@@ -349,8 +349,10 @@ __device__ inline int pick9(const int (&a)[9], int r) {
 }
 
 // The row mask and the Dirichlet pressures.  peak (mixed path): per block the
-// largest |eps rho| and |m / rho| of its particles, from which the assembly
-// bounds a row's coefficients.
+// largest |eps rho| and |m / rho| of its rows, from which the assembly bounds a
+// row's coefficients.  Rows alone: only they are columns, and walls beside a
+// sphere and without fluid (eps = -1e18) or dummies without a density would lift
+// every row's bound out of its coefficients' range.
 __global__ __launch_bounds__(kBlock) void k_rowmask(DevParams P, int n, const int* ptype, const int* btype,
                                                     const int* itype, const int* surf, const double* m,
                                                     const double* rho, const double* por, double* pres, int* row,
@@ -364,7 +366,7 @@ __global__ __launch_bounds__(kBlock) void k_rowmask(DevParams P, int n, const in
     // a free-surface particle is a known value p_ref, not an unknown
     if (dirichlet) pres[i] = P.p_ref;
     row[i] = fluid && !dirichlet ? 1 : 0;
-    if (peak) {
+    if (peak && fluid && !dirichlet) {
       pr = fmaxf(pr, (float)fabs(por[i] * rho[i]));
       vol = fmaxf(vol, (float)fabs(m[i] / rho[i]));
     }
@@ -449,17 +451,32 @@ __global__ void k_pack_asm(SphView<float> v, const int* __restrict__ row, const 
   v.ra[i] = r;
 }
 
+// The anchor that puts the binade `top` (a biased exponent) one below the last.
+__device__ inline int anchor_of(int top) { return min(max(top + 1 - 31, 1), 223); }
+// How many binades a row's largest coefficient may lie below its bound.  The
+// window words then still hold 18 binades below the largest one, so that what is
+// lost of the smaller ones is under the rounding of the largest (2^-17).
+constexpr int kAnchorSlack = 12;
+
+// A row whose coefficients lie outside the range that its bound gives (a lone pair
+// near the end of the kernel's support, one row of a very different density
+// somewhere) is marked with this bit of its count and the anchor of its own largest
+// coefficient, and kFlagRange has the host launch the marked rows again (OWN): the
+// second pass inside the kernel takes it from 230 to over 256 registers.
+constexpr int kRowRedo = 1 << 30;
+
 // One row by G lanes.  With one lane the quads of stored columns collect in
 // registers and leave whole; with more, the lanes of a round rank their columns
 // by a scan over the group, so the stored order is the list's either way, and
 // store them one by one.
-template <typename R, int FMT, int MIXED, int G>
+template <typename R, int FMT, int MIXED, int G, bool OWN = false>
 __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R>& v, const AsmOut& o, int i,
                                              const WinSlots& ww) {
   const int n = v.n;
   const size_t nn = (size_t)n;
   const int cnt = min(v.nbr_cnt[i], v.nbr_cap);
   const int sub = pair_sub<G>();
+  if (OWN && !(o.ccnt[i] & kRowRedo)) return;
   if (!o.row[i]) {
     if (sub != 0) return;
     o.ccnt[i] = 0;
@@ -500,9 +517,11 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
   const double uxi = v.ux[i], uyi = v.uy[i], uzi = v.uz[i];
   const double rhoi = v.rho[i], pori = v.por[i], irhoi = 1.0 / rhoi;
   int anchor = 0;
-  if (FMT == kFmtWin) {
+  if (OWN) {
+    anchor = (o.ccnt[i] >> 16) & 255;
+  } else if (FMT == kFmtWin) {
     // a bound of the row's coefficients: the largest eps_j rho_j and V_j of any
-    // particle, and |Cm| |W'(r) / r| at r -> 0
+    // row, and |Cm| |W'(r) / r| at r -> 0
     const double r0 = 0.01 * hd;
     double cmn = 1.0;
     if (P.kgc > 0) {
@@ -517,9 +536,9 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
     const double bound = (fabs(pori * rhoi) + (double)__uint_as_float(o.flags[2])) *
                          (double)__uint_as_float(o.flags[3]) * fabs(irhoi) * cmn *
                          fabs(knl_dw_ih<double>(P.kernel_type, A, hd, ihd, r0)) / r0;
-    const int top = (int)((__float_as_uint((float)bound) >> 23) & 255u);
-    anchor = min(max(top + 1 - 31, 1), 223);
+    anchor = anchor_of((int)((__float_as_uint((float)bound) >> 23) & 255u));
   }
+  float amax = 0.f;  // kFmtWin: the largest |a| stored
   const Kgc<double> K(P.kgc == 1, v.cm, n, i);
   double bd = 0, Aij = 0, AP = 0, lag = 0;  // bd: -div of eps u
   double dcomp = 0;  // sum over stored columns of a - hi (mixed)
@@ -663,6 +682,7 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
     if (MIXED) {
       double hv;
       if (FMT == kFmtWin) {
+        if (!OWN) amax = fmaxf(amax, fabsf((float)a));
         hw = win_word(a, anchor, (uint32_t)nq.slot & (uint32_t)kWinMax);
         hv = (double)win_val(hw, anchor << 23);
       } else {
@@ -741,9 +761,19 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
       if (FMT == kFmtRun8 && !MIXED) o.idx[(size_t)q * nn + i] = word;
     }
   }
+  int meta = FMT == kFmtWin ? kc | (anchor << 16) : kc;
+  if (FMT == kFmtWin && !OWN) {
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    const int top = (int)((__float_as_uint(amax) >> 23) & 255u), e = top - anchor;
+    if (amax > 0.f && (e > 30 || e < 30 - kAnchorSlack) && anchor_of(top) != anchor) {
+      meta = kc | (anchor_of(top) << 16) | kRowRedo;
+      bad |= kFlagRange;
+    }
+  }
   if (bad) atomicOr(o.flags, bad);
   if (G > 1 && sub != 0) return;
-  o.ccnt[i] = FMT == kFmtWin ? kc | (anchor << 16) : kc;
+  o.ccnt[i] = meta;
   o.runc[i] = rcw;
   const double tdt = P.dt_sph;
   const double bi = P.rho_fluid * (bd + 2 * (double)v.dpor[i] - (double)v.dpor_prev[i]) / tdt;
@@ -761,7 +791,7 @@ __device__ __forceinline__ void assemble_row(const DevParams& P, const SphView<R
 // takes each neighbour's window slot from the plan.  (A walk over the row's 27
 // cells through the cell table in place of the plan took 3.3 ms at 1.16 M
 // particles, nearly three times the rest of the assembly.)
-template <typename R, int FMT, int MIXED, int G>
+template <typename R, int FMT, int MIXED, int G, bool OWN = false>
 __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, AsmOut o) {
   if constexpr (FMT != kFmtWin) {
     const int i = pair_particle<G>();
@@ -794,7 +824,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
         atomicOr(o.flags, (unsigned)kFlagOffset);
         continue;
       }
-      assemble_row<R, FMT, MIXED, G>(P, v, o, i, w);
+      assemble_row<R, FMT, MIXED, G, OWN>(P, v, o, i, w);
     }
   }
 }
@@ -1594,6 +1624,11 @@ int ppe_assemble(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork
       k_zero_u32<<<1, 64, 0, s>>>(w.flags, 2);
       fmt = kFmtIdx32;  // an overfull run or window: plain indices
       continue;
+    }
+    if (fmt == kFmtWin && (f & kFlagRange)) {
+      TRY(pair_launch(v.n, asm_lanes(v.n), [&](auto gl, int grid) {
+        k_assemble<R, kFmtWin, 1, decltype(gl)::value, true><<<grid, kBlock, 0, s>>>(P, v, o);
+      }));
     }
     if (f & kFlagOrder) {
       set_error("PPE assembly: neighbour list not in cell-run order");

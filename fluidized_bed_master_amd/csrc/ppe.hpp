@@ -39,13 +39,14 @@ constexpr int kWinMax = (1 << kWinBits) - 1;
 //   sign (1) | exponent (5) | fraction (15) | window slot (11),
 // the exponent counted from the row's anchor (the upper 16 bits of ccnt), so
 // that hi = win_val(word, anchor << 23) takes three integer operations.  The
-// anchor puts a bound of the row's coefficients in the top binade but one;
-// below the 31 binades hi is the nearest value of the range.
+// anchor puts the row's largest coefficient in one of the 13 binades below the
+// top one; below the 31 binades hi is the nearest value of the range.
 // The inner diagonal takes up the rounding of its row,
 // dgi_i = d_i - sum_j (a_ij - hi_ij): the inner operator then maps a
 // constant vector exactly as the FP64 one does, and differs from it by
 // sum_j (a_ij - hi_ij) (x_i - x_j) only (relative 2^-16 of a difference).
-// hi + lo keeps a to about 2^-40 for the FP64 residual.
+// hi + lo keeps a to about 2^-40 for the FP64 residual (kFmtWin: what lies below
+// the range, to 2^-43 of the row's largest).
 __device__ inline uint32_t hi16_bits(double a) { return (__float_as_uint((float)a) + 0x80u) & 0xFFFFFF00u; }
 __device__ inline float hi_val(uint32_t e) { return __uint_as_float(e & 0xFFFFFF00u); }
 __device__ inline float win_val(uint32_t w, int anchor23) {
