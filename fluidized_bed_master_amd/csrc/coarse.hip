@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, double
     const int m = win_stage(
         o, s0, i1, S, &e0, [](int x, int y, int z, int) { return (int)agg_parity(x, y, z); },
         [](int par, int, int) { return (uint8_t)par; });
-    const int i = s0 + (int)threadIdx.x;
+    const int i = s0 + (int)threadIdx.x, first = s0;
     s0 = m;
     if (i >= m) continue;
     double acc[8];
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, double
       int cx, cy, cz;
       cell_xyz(key, o.NI, o.NJ, cx, cy, cz);
       const uint8_t own = agg_parity(cx, cy, cz);
-      const uint8_t* win = S.x + S.p.pre[9 * (win_ekey(o, key) - e0)];
+      const uint8_t* win = S.x + S.p.pre[win_first(o, S.p, e0, first, i, key)];
       acc[0] = o.diag[i];
       const int meta = o.ccnt[i];
       const int nq = ((meta & 0xFFFF) + 3) >> 2, anc = (meta >> 16) << 23;

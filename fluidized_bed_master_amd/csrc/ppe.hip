@@ -805,13 +805,13 @@ __global__ __launch_bounds__(kBlock) void k_assemble(DevParams P, SphView<R> v, 
       const int m = win_plan(o, s0, i1, S, &e0, &cells, [](int, int, int, int first) { return first; });
       if ((int)threadIdx.x < cells) S.start[threadIdx.x] = S.pre[threadIdx.x] - S.start[threadIdx.x];
       __syncthreads();
-      const int i = s0 + (int)threadIdx.x / G;
+      const int i = s0 + (int)threadIdx.x / G, first = s0;
       s0 = m;
       if (i >= m) continue;
       WinSlots w{};
-      if (cells > 0) {
+      if (cells > 0 && o.row[i]) {
         const uint32_t key = o.keys[i], cb = cell_bits_of(o, key);
-        const int c = 9 * (win_ekey(o, key) - e0);
+        const int c = win_first(o, S, e0, first, i, key);
         w.D = S.start + c;
         w.base = S.pre[c];
         w.total = S.pre[c + 27] - S.pre[c];

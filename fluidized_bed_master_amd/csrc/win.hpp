@@ -21,19 +21,25 @@
 namespace sophia {
 
 constexpr int kWinThreads = 256;
-constexpr int kWinCells = 256;  // staged cells per tile: 28 planes
+constexpr int kWinCells = 256;  // staged cells per tile
+constexpr int kWinPlanes = kWinCells / 9;
 // staged values per tile: a 256-row tile of the 1 mm columns takes about 2800;
 // with the tables it is 19.5 KB in FP32, eight blocks per CU
 constexpr int kWinCap = 4096;  // the coarse correction's table leaves no room for more
 static_assert(kWinMax < kWinCap, "a single row's window always fits");
 
-// Where the cells of a tile's planes go: cell c = 9 (e - ea + 1) + r holds the
-// slots [pre[c], pre[c + 1]) of the staged copy.
+// Where the cells of a tile's planes go: cell c = 9 p + r, cell r of the p-th
+// planned plane, holds the slots [pre[c], pre[c + 1]) of the staged copy.
 struct WinPlan {
   int pre[kWinCells + 1];
   int start[kWinCells];  // cellval of the cell
   int wsum[kWinThreads / 64];
+  // a tile with gaps (kWinGaps): its planes, and each row's first
+  int plane[kWinPlanes];
+  int cut;
+  uint8_t first[kWinThreads];
 };
+constexpr int kWinGaps = INT32_MIN;
 template <typename XT>
 struct WinStage {
   XT x[kWinCap];
@@ -46,47 +52,116 @@ __device__ inline int win_ekey(const O& o, uint32_t key) {
   return (int)(key - (uint32_t)t * (uint32_t)o.NI) + 1 + (o.NI + 2) * t;
 }
 
-// The block plans the longest of the row ranges [i0, i1), its first half,
-// quarter, ... whose planes fit and returns its end m (all threads alike); *e0
-// is the extended key of row i0 and *cells the planned cells, 0 when there is
-// nothing to stage: rows past the last cell, or a single particle whose window
-// does not fit (no row of an assembled operator).  `cellval(x, y, z, first)` is
-// kept per cell in S.start; first is -1 for places outside the grid.
+// inclusive sum or maximum over the block's threads; w takes one word per wave
+template <bool MAX>
+__device__ inline int win_scan(int v, int* w) {
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(v, off);
+    if (lane >= off) v = MAX ? max(v, u) : v + u;
+  }
+  if (lane == 63) w[wave] = v;
+  __syncthreads();
+  for (int k = 0; k < kWinThreads / 64 - 1; k++) {
+    const int u = w[k];
+    if (k < wave) v = MAX ? max(v, u) : v + u;
+  }
+  __syncthreads();  // w may be written again
+  return v;
+}
+
+// The particles of planned cell c, the r-th of the plane around extended key e, and
+// S.start[c] from `cellval`.
+template <class O, class CV>
+__device__ inline int win_cell_len(const O& o, int e, int r, int c, WinPlan& S, CV&& cellval) {
+  const int row = e / (o.NI + 2);
+  int x = e - (o.NI + 2) * row - 1, z = row / o.NJ;
+  int y = row - o.NJ * z;
+  y += r % 3 - 1;
+  z += r / 3 - 1;
+  int first = -1, len = 0;  // outside the grid: no particles
+  if (cell_in(o.pmask, 2, z, o.NK) && cell_in(o.pmask, 1, y, o.NJ) && cell_in(o.pmask, 0, x, o.NI)) {
+    const int k = x + o.NI * (y + o.NJ * z);
+    first = (int)o.cell_off[k];
+    len = (int)o.cell_off[k + 1] - first;
+  }
+  S.start[c] = cellval(x, y, z, first);
+  return len;
+}
+
+// A plan for a range whose cells lie too far apart, or hold too much, for one run
+// of planes: the planes around its rows' cells alone, side by side, each once
+// (walls and other particles that are not rows need none: a range without rows is
+// done at once).  Returns the end of the rows that fit.  (Halving the range until
+// its run of planes fits, walls and empty cells included, took 85 us a pass for a
+// film of two layers on sparse walls, 278 k particles, in place of 17.2; 37.5 / 21.6
+// for a column of 144 k rows under walls three times its height; 29.0 / 11.7 for one
+// of 64 k rows in a domain sixteen times as wide.)
+template <class O, class CV>
+__device__ int win_plan_gaps(const O& o, int i0, int i1, WinPlan& S, int* ncells, CV&& cellval) {
+  const int t = (int)threadIdx.x, i = i0 + t;
+  int e = -1;
+  if (i < i1 && o.row[i] != 0) {
+    const uint32_t key = o.keys[i];
+    if (key < (uint32_t)o.ncell) e = win_ekey(o, key);
+  }
+  // keys ascend: the row before this one has the largest key so far
+  const int emax = win_scan<true>(e, S.wsum);
+  const int up = __shfl_up(emax, 1);
+  if ((t & 63) == 63) S.wsum[t >> 6] = emax;
+  if (t == 0) S.cut = i1;
+  __syncthreads();
+  const int prev = t == 0 ? -1 : ((t & 63) == 0 ? S.wsum[(t >> 6) - 1] : up);
+  __syncthreads();
+  const int add = e < 0 ? 0 : (prev < 0 ? 3 : min(e - prev, 3));
+  const int p = win_scan<false>(add, S.wsum);  // planes up to this row's e + 1
+  if (e >= 0 && p > kWinPlanes) atomicMin(&S.cut, i);
+  if (e >= 0 && p <= kWinPlanes) {
+    if (add > 0) S.plane[p - 1] = e + 1;
+    if (add > 1) S.plane[p - 2] = e;
+    if (add > 2) S.plane[p - 3] = e - 1;
+    S.first[t] = (uint8_t)(p - 3);
+  } else {
+    S.first[t] = 0;
+  }
+  // planes in use: those of the last row that fits
+  int np = win_scan<true>(e >= 0 && p <= kWinPlanes ? p : 0, S.wsum);
+  if (t == kWinThreads - 1) S.wsum[0] = np;
+  __syncthreads();
+  np = S.wsum[0];
+  __syncthreads();
+  if (np == 0) return i1;  // no rows
+  const int len = t < 9 * np ? win_cell_len(o, S.plane[t / 9], t % 9, t, S, static_cast<CV&&>(cellval)) : 0;
+  const int pre = win_scan<false>(len, S.wsum);
+  S.pre[t + 1] = pre;
+  if (t == 0) S.pre[0] = 0;
+  __syncthreads();
+  while (np >= 3 && S.pre[9 * np] > kWinCap) np--;
+  // np < 3: a particle whose window does not fit (no row of an assembled operator)
+  *ncells = np >= 3 ? 9 * np : 0;
+  if (e >= 0 && p > max(np, 3)) atomicMin(&S.cut, i);
+  __syncthreads();
+  return S.cut;
+}
+
+// The block plans the row range [i0, i1), or as much of it from i0 on as fits, and
+// returns the planned end m (all threads alike); *e0 is the extended key of row i0,
+// or kWinGaps (win_first), and *cells the planned cells, 0 when there is nothing to
+// stage: no rows, or a row whose window does not fit (no row of an assembled
+// operator).  `cellval(x, y, z, first)` is kept per cell in S.start; first is -1 for
+// places outside the grid.
 template <class O, class CV>
 __device__ int win_plan(const O& o, int i0, int i1, WinPlan& S, int* e0, int* ncells, CV&& cellval) {
   const int t = (int)threadIdx.x, lane = t & 63;
-  const uint32_t ka = o.keys[i0];
-  const int NI2 = o.NI + 2;
-  *e0 = 0;
+  const uint32_t ka = o.keys[i0], kb = o.keys[i1 - 1];
+  *e0 = kWinGaps;
   *ncells = 0;
-  if (ka >= (uint32_t)o.ncell) return i1;
+  __syncthreads();  // the previous tile is done with S
+  if (ka >= (uint32_t)o.ncell) return i1;  // past the last cell
   const int ea = win_ekey(o, ka);
-  *e0 = ea;
-  for (int m = i1;; m = i0 + (m - i0) / 2) {
-    __syncthreads();  // the previous tile is done with S
-    const uint32_t kb = o.keys[m - 1];
-    const int cells = kb < (uint32_t)o.ncell ? 9 * (win_ekey(o, kb) - ea + 3) : kWinCells + 1;
-    if (cells > kWinCells) {
-      if (m - i0 == 1) return m;
-      continue;
-    }
-    int len = 0;
-    if (t < cells) {
-      const int p = t / 9, r = t - 9 * p;
-      const int e = ea - 1 + p;
-      const int row = e / NI2;
-      int x = e - NI2 * row - 1, z = row / o.NJ;
-      int y = row - o.NJ * z;
-      y += r % 3 - 1;
-      z += r / 3 - 1;
-      int first = -1;  // outside the grid: no particles
-      if (cell_in(o.pmask, 2, z, o.NK) && cell_in(o.pmask, 1, y, o.NJ) && cell_in(o.pmask, 0, x, o.NI)) {
-        const int k = x + o.NI * (y + o.NJ * z);
-        first = (int)o.cell_off[k];
-        len = (int)o.cell_off[k + 1] - first;
-      }
-      S.start[t] = cellval(x, y, z, first);
-    }
+  const int cells = kb < (uint32_t)o.ncell ? 9 * (win_ekey(o, kb) - ea + 3) : kWinCells + 1;
+  if (cells <= kWinCells) {
+    const int len = t < cells ? win_cell_len(o, ea - 1 + t / 9, t % 9, t, S, cellval) : 0;
     int inc = len;
     for (int off = 1; off < 64; off <<= 1) {
       const int v = __shfl_up(inc, off);
@@ -101,16 +176,24 @@ __device__ int win_plan(const O& o, int i0, int i1, WinPlan& S, int* e0, int* nc
       add += w < (t >> 6) ? v : 0;
       total += v;
     }
-    if (total > kWinCap) {
-      if (m - i0 == 1) return m;
-      continue;
+    if (total <= kWinCap) {
+      S.pre[t + 1] = inc + add;
+      if (t == 0) S.pre[0] = 0;
+      __syncthreads();
+      *e0 = ea;
+      *ncells = cells;
+      return i1;
     }
-    S.pre[t + 1] = inc + add;
-    if (t == 0) S.pre[0] = 0;
-    __syncthreads();
-    *ncells = cells;
-    return m;
+    __syncthreads();  // S.wsum is read
   }
+  return win_plan_gaps(o, i0, i1, S, ncells, static_cast<CV&&>(cellval));
+}
+
+// first planned cell of the window of row i, whose cell key is `key`, of the tile
+// planned from row s0 on
+template <class O>
+__device__ inline int win_first(const O& o, const WinPlan& S, int e0, int s0, int i, uint32_t key) {
+  return e0 == kWinGaps ? 9 * S.first[i - s0] : 9 * (win_ekey(o, key) - e0);
 }
 
 // win_plan, then the values: `val(cellval, l, c)` is that of the l-th particle of
@@ -201,7 +284,7 @@ __device__ __forceinline__ void win_rows(const PpeOp& o, WinStage<XT>& S, H&& he
       if (i < m) {
         // particles that no cell or plan holds are not rows: any slot will do
         const uint32_t key = o.keys[i];
-        const int c = key < (uint32_t)o.ncell ? 9 * (win_ekey(o, key) - e0) : 0;
+        const int c = key < (uint32_t)o.ncell ? win_first(o, S.p, e0, s0, i, key) : 0;
         const int cw = min(max(c, 0), kWinCells - 27);
         f(i, S.p.pre[cw], (t & (G - 1)) == 0, hd, cw + 13);
       }

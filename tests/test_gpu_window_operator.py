@@ -167,3 +167,86 @@ def test_row_far_below_the_others_keeps_its_precision():
     assert abs(a.ppe_apply(e)[i] + d[i]) <= 2.0 ** -39 * d[i]
     assert abs(a.matvec_probe(0, e, reps=1)[0][i] + d[i]) <= 2.0 ** -16 * d[i]
     a.close()
+
+
+def _film():
+    # two layers of fluid in a tray with sparse walls: in the upper cells of the
+    # walls a run of planes holds a handful of particles
+    p, parts = configs.isph_dem_column(300, 300, 2, 1.0e-3, jitter=0.02, seed=3, tank_extra=10)
+    keep = (parts["p_type"] == abi.PT_FLUID) | (configs.uniform(9, len(parts)) < 0.3)
+    return p, parts[keep]
+
+
+def _wide(nx=40, ny=40, nz=40):
+    # a column in one corner of a domain sixteen times as wide: the cells of one
+    # x-row end and those of the next begin 200 apart
+    p, parts = configs.isph_dem_column(nx, ny, nz, 1.0e-3, jitter=0.02, seed=3)
+    far = parts[:200].copy()
+    far["x"] += 0.6
+    return p, np.concatenate([far, parts])
+
+
+def _spray(n=60, fill=0.02):
+    # drops: single particles and small groups, most cells empty
+    p, parts = configs.isph_dem_column(n, n, n, 1.0e-3, jitter=0.4, seed=3, wall_layers=1, u_noise=0.01)
+    fluid = parts["p_type"] == abi.PT_FLUID
+    u = configs.uniform(12, len(parts))
+    drop = configs.uniform(13, (n // 4 + 1) ** 3) < fill  # groups of up to 4^3
+    g = [np.minimum((parts[c] / 4e-3).astype(int), n // 4) for c in "xyz"]
+    in_drop = drop[np.clip(g[0] + (n // 4 + 1) * (g[1] + (n // 4 + 1) * g[2]), 0, len(drop) - 1)]
+    return p, parts[~fluid | (u < fill) | (fluid & in_drop & (u < 0.5))]
+
+
+def _dense():
+    # 1,000 particles and more around a cell: a tile's planes hold more than it stages
+    p, parts = configs.taylor_green(22, jitter=0.05)
+    more = np.concatenate([parts] * 2)
+    for k, c in enumerate("xyz"):
+        more[c] = np.mod(more[c] + configs.uniform(20 + k, len(more), 0.0, 0.1), 2 * np.pi)
+    p.sph_max_neighbors = 240
+    return p, more
+
+
+@pytest.mark.parametrize("make", [_film, _wide, lambda: _wide(60, 62, 70), _spray, lambda: _spray(40, 0.3), _dense],
+                         ids=["film", "wide", "wide_2_lanes", "spray", "spray_of_groups", "dense"])
+def test_tiles_with_gaps_match_fp64_formats(make):
+    """Tiles planned around their rows' cells alone: the product, the inner product
+    and (two-level) the coarse operator beside the FP64 path's formats."""
+    p, parts = make()
+    a, b = _assembled(p, parts, abi.PREC_MIXED), _assembled(p, parts, abi.PREC_FP64)
+    assert a.ppe_layout()["index_bytes"] == 0
+    assert a.ppe_layout()["nnz"] == b.ppe_layout()["nnz"]
+    d, _, rows = b.get_ppe_system()
+    r = rows == 1
+    assert np.array_equal(a.get_ppe_system()[2], rows) and r.sum() > 0
+    x = np.random.default_rng(5).uniform(-1, 1, len(rows)) * r
+    ref = b.ppe_apply(x)
+    scale = np.maximum(2 * np.abs(d[r]), 1e-3 * np.abs(d[r]).max())
+    assert (np.abs(a.ppe_apply(x) - ref)[r] / scale).max() <= 2.0 ** -18
+    assert (np.abs(a.matvec_probe(0, x, reps=1)[0] - ref)[r] / scale).max() <= 2.0 ** -16 + 2.0 ** -18
+    if not p.periodic_mask:
+        E = []
+        for g, mixed in ((a, True), (b, False)):
+            st = g.ppe(abi.ppe_opts(method=abi.PPE_BICGSTAB, rtol=1e-3, precond=abi.PRECOND_TWO_LEVEL, max_iter=200,
+                                    guess=abi.GUESS_ZERO, precision=abi.PPE_MIXED_IR if mixed else abi.PPE_FP64))
+            if st["precond_used"] == abi.PRECOND_TWO_LEVEL:
+                E.append(g.ppe_coarse()[1].astype(float))
+        assert len(E) == (0 if make is _spray else 2)  # lone drops: a singular coarse operator
+        # FP32 entries of sums of coefficients with relative errors of 2^-18
+        if E:
+            assert np.abs(E[0] - E[1]).max() <= 2.0 ** -17 * np.abs(E[1]).max()
+    a.close()
+    b.close()
+
+
+def test_wall_cells_and_gaps_cost_no_tiles():
+    """A pass over the film takes no longer than one over a full column of as many
+    particles, which has four times its entries (0.8 of it; 3.9 times where every
+    wall cell and gap has a tile of its own)."""
+    us = []
+    for p, parts in (_film(), configs.c4_train()):
+        g = _assembled(p, parts, abi.PREC_MIXED)
+        x = np.ones(len(g.get_ppe_system()[2]))
+        us.append(min(g.matvec_probe(0, x, reps=50)[1] for _ in range(5)))
+        g.close()
+    assert us[0] <= 2 * us[1], us
