@@ -348,69 +348,75 @@ __device__ inline int pick9(const int (&a)[9], int r) {
   return v;
 }
 
-// The row mask and the Dirichlet pressures.  peak (mixed path): per block the
+// What the assembly asks of all rows: bounds of their coefficients, and how densely
+// they lie: the planes around the cells of the rows of each 64 consecutive
+// particles (as a tile would plan them, win_plan_gaps), summed.
+struct RowStat {
+  float pr, vol, planes;
+  __device__ void add(const RowStat& b) {
+    pr = fmaxf(pr, b.pr);
+    vol = fmaxf(vol, b.vol);
+    planes += b.planes;
+  }
+};
+// over the block; the sum is thread 0's
+__device__ inline void block_stat(RowStat& s) {
+  __shared__ RowStat red[kBlock / 64];
+  for (int off = 32; off > 0; off >>= 1)
+    s.add(RowStat{__shfl_xor(s.pr, off), __shfl_xor(s.vol, off), __shfl_xor(s.planes, off)});
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int w = 1; w < kBlock / 64; w++) s.add(red[w]);
+}
+
+// The row mask and the Dirichlet pressures.  stat (mixed path): per block the
 // largest |eps rho| and |m / rho| of its rows, from which the assembly bounds a
-// row's coefficients.  Rows alone: only they are columns, and walls beside a
-// sphere and without fluid (eps = -1e18) or dummies without a density would lift
-// every row's bound out of its coefficients' range.
+// row's coefficients, and their planes.  Rows alone: only they are columns, and
+// walls beside a sphere and without fluid (eps = -1e18) or dummies without a density
+// would lift every row's bound out of its coefficients' range.
 __global__ __launch_bounds__(kBlock) void k_rowmask(DevParams P, int n, const int* ptype, const int* btype,
                                                     const int* itype, const int* surf, const double* m,
                                                     const double* rho, const double* por, double* pres, int* row,
-                                                    float2* peak) {
-  __shared__ float2 red[kBlock / 64];
-  float pr = 0.f, vol = 0.f;
+                                                    const uint32_t* keys, RowStat* stat) {
+  RowStat s{};
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
     const int t = ptype[i];
     const bool fluid = itype[i] <= 2 && !(P.open_boundary > 0 && btype[i] > 0) && t < 1000 && t > 0;
     const bool dirichlet = fluid && P.free_surface > 0 && surf[i] != 0;
     // a free-surface particle is a known value p_ref, not an unknown
     if (dirichlet) pres[i] = P.p_ref;
-    row[i] = fluid && !dirichlet ? 1 : 0;
-    if (peak && fluid && !dirichlet) {
-      pr = fmaxf(pr, (float)fabs(por[i] * rho[i]));
-      vol = fmaxf(vol, (float)fabs(m[i] / rho[i]));
+    const bool on = fluid && !dirichlet;
+    row[i] = on ? 1 : 0;
+    if (!stat) continue;
+    if (on) {
+      s.pr = fmaxf(s.pr, (float)fabs(por[i] * rho[i]));
+      s.vol = fmaxf(s.vol, (float)fabs(m[i] / rho[i]));
     }
+    const int lane = threadIdx.x & 63;
+    const uint32_t key = keys[i];
+    const int e = (int)key + 2 * (int)(key / (uint32_t)P.NI);  // win_ekey but for a constant
+    const uint64_t below = __ballot(on) & ((1ull << lane) - 1);
+    const int prev = __shfl(e, below ? 63 - __clzll(below) : lane);
+    if (on) s.planes += below ? (float)min(e - prev, 3) : 3.f;
   }
-  if (!peak) return;
-  for (int off = 32; off > 0; off >>= 1) {
-    pr = fmaxf(pr, __shfl_xor(pr, off));
-    vol = fmaxf(vol, __shfl_xor(vol, off));
-  }
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(pr, vol);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kBlock / 64; w++) {
-      pr = fmaxf(pr, red[w].x);
-      vol = fmaxf(vol, red[w].y);
-    }
-    peak[blockIdx.x] = make_float2(pr, vol);
-  }
+  if (!stat) return;
+  block_stat(s);
+  if (threadIdx.x == 0) stat[blockIdx.x] = s;
 }
 
-// one block: clears the assembly's flags and leaves the two peaks (FP32 bits)
+// one block: clears the assembly's flags and leaves the sums of RowStat (FP32 bits)
 // behind them.  (An atomic maximum from each wave of k_rowmask in place of the
 // partials took 141 us at 1.16 M particles.)
-__global__ __launch_bounds__(kBlock) void k_asm_begin(const float2* peak, int G, unsigned* flags) {
-  __shared__ float2 red[kBlock / 64];
-  float pr = 0.f, vol = 0.f;
-  for (int b = threadIdx.x; b < G; b += kBlock) {
-    pr = fmaxf(pr, peak[b].x);
-    vol = fmaxf(vol, peak[b].y);
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    pr = fmaxf(pr, __shfl_xor(pr, off));
-    vol = fmaxf(vol, __shfl_xor(vol, off));
-  }
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(pr, vol);
-  __syncthreads();
+__global__ __launch_bounds__(kBlock) void k_asm_begin(const RowStat* stat, int G, unsigned* flags) {
+  RowStat s{};
+  for (int b = threadIdx.x; b < G; b += kBlock) s.add(stat[b]);
+  block_stat(s);
   if (threadIdx.x == 0) {
-    for (int w = 1; w < kBlock / 64; w++) {
-      pr = fmaxf(pr, red[w].x);
-      vol = fmaxf(vol, red[w].y);
-    }
     flags[0] = flags[1] = 0u;
-    flags[2] = __float_as_uint(pr);
-    flags[3] = __float_as_uint(vol);
+    flags[2] = __float_as_uint(s.pr);
+    flags[3] = __float_as_uint(s.vol);
+    flags[4] = __float_as_uint(s.planes);
   }
 }
 
@@ -1424,15 +1430,14 @@ void launch_fin(hipStream_t s, const PpeWork& w, int op, unsigned* count_out = n
 
 // blocks of a window-staged pass over n rows with G lanes each
 int win_grid(int n, int G) { return grid_rows((int)std::min<int64_t>((int64_t)n * G, INT32_MAX)); }
-#define WIN_LAUNCH(kern, n, ...)                                                      \
+#define WIN_LAUNCH(kern, o, ...)                                                      \
   do {                                                                                \
-    switch (win_group(n)) {                                                           \
-      case 1: kern<1><<<win_grid(n, 1), kRedThreads, 0, s>>>(__VA_ARGS__); break;     \
-      case 2: kern<2><<<win_grid(n, 2), kRedThreads, 0, s>>>(__VA_ARGS__); break;     \
-      default: kern<4><<<win_grid(n, 4), kRedThreads, 0, s>>>(__VA_ARGS__); break;    \
+    switch (win_group((o).n, (o).nnz)) {                                              \
+      case 1: kern<1><<<win_grid((o).n, 1), kRedThreads, 0, s>>>(o, __VA_ARGS__); break;  \
+      case 2: kern<2><<<win_grid((o).n, 2), kRedThreads, 0, s>>>(o, __VA_ARGS__); break;  \
+      default: kern<4><<<win_grid((o).n, 4), kRedThreads, 0, s>>>(o, __VA_ARGS__); break; \
     }                                                                                 \
   } while (0)
-int win_blocks(int n) { return win_grid(n, win_group(n)); }
 
 // f(lanes as an integral constant) by row_lanes
 template <class F>
@@ -1442,11 +1447,11 @@ void with_row_lanes(int n, F&& f) {
 }
 
 // blocks (and reduction partials) of an operator pass
-int op_blocks(const PpeOp& o) { return o.fmt == kFmtWin ? win_blocks(o.n) : win_grid(o.n, row_lanes(o.n)); }
+int op_blocks(const PpeOp& o) { return win_grid(o.n, o.fmt == kFmtWin ? win_group(o.n, o.nnz) : row_lanes(o.n)); }
 
 void launch_win_mv(hipStream_t s, const PpeOp& o, const float* x, float* y, const float* wv, const WinCoarse& cz,
                    const PpeWork& w, const BiState* st) {
-  const int G = win_group(o.n), g = win_grid(o.n, G);
+  const int G = win_group(o.n, o.nnz), g = win_grid(o.n, G);
   if (cz.y && G == 2) k_win_mv<2, true><<<g, kRedThreads, 0, s>>>(o, x, y, wv, cz, w.partials, st);
   else if (cz.y) k_win_mv<4, true><<<g, kRedThreads, 0, s>>>(o, x, y, wv, cz, w.partials, st);
   else if (G == 1) k_win_mv<1, false><<<g, kRedThreads, 0, s>>>(o, x, y, wv, cz, w.partials, st);
@@ -1459,7 +1464,7 @@ void launch_apply_full(hipStream_t s, const PpeWork& w, const PpeOp& o, const do
                        bool norm) {
   const int G = op_blocks(o);
   if (o.fmt == kFmtWin) {
-    WIN_LAUNCH(k_win_apply, w.n, o, x, y, residual, norm, w.partials);
+    WIN_LAUNCH(k_win_apply, o, x, y, residual, norm, w.partials);
   } else {
     with_row_lanes(w.n, [&](auto gl) {
       constexpr int L = decltype(gl)::value;
@@ -1501,8 +1506,8 @@ int ppe_workspace_alloc(PpeWork& w, int n, int cap, bool mixed) {
   HIP_TRY(A(&w.state, sizeof(BiState)));
   HIP_TRY(hipMemset(w.state, 0, sizeof(BiState)));
   HIP_TRY(hipHostMalloc(&w.host_state, sizeof(BiState), hipHostMallocDefault));
-  HIP_TRY(A((void**)&w.flags, 16));
-  HIP_TRY(hipHostMalloc((void**)&w.host_flags, 16, hipHostMallocDefault));
+  HIP_TRY(A((void**)&w.flags, 32));
+  HIP_TRY(hipHostMalloc((void**)&w.host_flags, 32, hipHostMallocDefault));
   w.vec_bytes = mixed ? 4 : 8;
   for (int k = 0; k < (mixed ? 10 : 8); k++) HIP_TRY(A(&w.vec[k], N * w.vec_bytes));
   if (mixed) HIP_TRY(A((void**)&w.x64b, N * 8));
@@ -1542,6 +1547,7 @@ PpeOp ppe_op(const PpeWork& w) {
   o.n = w.n;
   o.nq = w.cap4 / 4;
   o.fmt = w.fmt;
+  o.nnz = w.nnz;
   o.NI = w.NI;
   o.NJ = w.NJ;
   o.NK = w.NK;
@@ -1575,6 +1581,23 @@ int cell_offsets(hipStream_t s, int n, const uint32_t* keys, int num_cells, uint
 // 330 / 294 / 329 / 392 at 281,000, 1220 / 1298 / 1433 / 1751 at 1.16 M).
 inline int asm_lanes(int n) { return n >= 500000 ? 1 : pair_lanes(n); }
 
+// Whether a system's rows lie too thinly for the window format: where the tiles of
+// its passes plan many planes for few entries, u32 columns are read faster than the
+// planes are staged, unless their words, twice as long, no longer fit the caches.
+// Entries per plane (RowStat), and us per BiCGStab iteration with windows / with u32
+// columns, two lanes per row: full columns at h = 1.3 dx 820 (276 k particles,
+// 70 / 91), at 1.2 dx 520 (68 / 77), at 1.1 dx 290 (65.0 / 64.5), at 1.0 dx 185
+// (69 / 59; 616 k, 14.4 M entries, 100 / 84; 1.16 M, 28 M entries, 138 / 154); layers
+// of four particles 550 (70 / 80), of two 370 (82 / 55; 834 k 189 / 115), of one 115
+// (53 / 45; 669 k 99 / 71); half-empty groups 240 (17.7 M entries, 98 / 98) and 140
+// (93 / 75); sprays 14 and less (127 / 47, 140 / 41).  Four lanes, where a launch takes
+// as long as either: 125 (37 / 38), 6 (69 / 36).
+inline bool rows_thin(int n, const unsigned* flags) {
+  float planes;
+  std::memcpy(&planes, flags + 4, 4);
+  return flags[1] <= 16000000u && (float)flags[1] < (n >= kWinTwo ? 430.f : 50.f) * planes;
+}
+
 template <typename R>
 int ppe_assemble(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork& w, const uint32_t* keys,
                  const uint32_t* cell_off) {
@@ -1595,17 +1618,19 @@ int ppe_assemble(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork
   w.rowmajor = P.z_index == 0;
   AsmOut o{v.n, P.NI, P.NJ, P.NK, P.pmask, P.NI * P.NJ * P.NK, keys, cell_off, w.row, w.ccnt, w.runc, w.idx, w.hi, w.lo, w.c64,
            w.diag, w.dinv, w.rhs, w.dgi, w.flags};
-  // flags: overflow bits, stored entries, then the two peaks
+  // flags: overflow bits, stored entries, then the rows' statistics
   const int gm = std::min(grid_for(v.n), kMaxGrid);
-  float2* peak = reinterpret_cast<float2*>(w.partials);
-  k_rowmask<<<gm, kBlock, 0, s>>>(P, v.n, v.ptype, v.btype, v.itype, v.surf, v.m, v.rho, v.por, v.pres, w.row,
-                                  w.mixed ? peak : nullptr);
-  k_asm_begin<<<1, kBlock, 0, s>>>(peak, w.mixed ? gm : 0, w.flags);
+  RowStat* stat = reinterpret_cast<RowStat*>(w.partials);
+  k_rowmask<<<gm, kBlock, 0, s>>>(P, v.n, v.ptype, v.btype, v.itype, v.surf, v.m, v.rho, v.por, v.pres, w.row, keys,
+                                  w.mixed ? stat : nullptr);
+  k_asm_begin<<<1, kBlock, 0, s>>>(stat, w.mixed ? gm : 0, w.flags);
   if constexpr (std::is_same<R, float>::value) k_pack_asm<<<grid_for(v.n), kBlock, 0, s>>>(v, w.row, keys, P.NI, P.NJ);
   // window slots (mixed) need row-major keys; the x-runs of the FP64 format
   // are contiguous only in row-major keys without periodic wrap
   const int long_axis = std::max({P.NI, P.NJ, P.NK});  // images need whole coordinates in ten bits (win_step)
-  int fmt = P.z_index || (P.pmask && long_axis > 1000) ? kFmtIdx32 : (w.mixed ? kFmtWin : (P.pmask ? kFmtIdx32 : kFmtRun8));
+  const bool win = w.mixed && !P.z_index && !(P.pmask && long_axis > 1000);
+  int fmt = win ? (w.thin ? kFmtIdx32 : kFmtWin) : (w.mixed || P.z_index || P.pmask ? kFmtIdx32 : kFmtRun8);
+  bool overfull = false;
   for (;;) {
     TRY(pair_launch(v.n, asm_lanes(v.n), [&](auto gl, int grid) {
       constexpr int G = decltype(gl)::value;
@@ -1617,13 +1642,23 @@ int ppe_assemble(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork
     k_count_nnz<<<w.nbg, kRedThreads, 0, s>>>(v.n, w.ccnt, fmt == kFmtWin ? 0xFFFF : -1, w.partials);
     launch_fin(s, w, kFinCount, w.flags + 1);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(w.host_flags, w.flags, 8, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(w.host_flags, w.flags, 20, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     const unsigned f = w.host_flags[0];
     if (fmt != kFmtIdx32 && (f & (kFlagOffset | kFlagRunCount))) {
       k_zero_u32<<<1, 64, 0, s>>>(w.flags, 2);
       fmt = kFmtIdx32;  // an overfull run or window: plain indices
+      overfull = true;
       continue;
+    }
+    if (win && !overfull) {
+      // the format goes by this system alone; the last one's is tried first
+      w.thin = rows_thin(v.n, w.host_flags);
+      if (w.thin != (fmt == kFmtIdx32)) {
+        k_zero_u32<<<1, 64, 0, s>>>(w.flags, 2);
+        fmt = w.thin ? kFmtIdx32 : kFmtWin;
+        continue;
+      }
     }
     if (fmt == kFmtWin && (f & kFlagRange)) {
       TRY(pair_launch(v.n, asm_lanes(v.n), [&](auto gl, int grid) {
@@ -1820,7 +1855,7 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
   // at 276,000.  At 1.16 M rows the prolongation pass (6 us) is cheaper than
   // the gather of the correction in every tile (345 -> 356 us per iteration).
   constexpr bool kWin = FMT == kFmtWin;
-  const bool fused = kWin && cw && win_group(n) > 1;
+  const bool fused = kWin && cw && n < 500000 && win_group(n, o.nnz) > 1;
   V* phc = fused ? (V*)w.vec[8] : ph;
   V* shc = fused ? (V*)w.vec[9] : sh;
   auto matvec = [&](const V* x, V* y, const V* ww, V* xc) {
@@ -1863,7 +1898,7 @@ int bicgstab_run(hipStream_t s, PpeWork& w, const CoarseWork* cw, double rn, dou
       k_bi_xr<V><<<G, kRedThreads, 0, s>>>(n, xs, phc, shc, r, t, rh, w.partials, st);
       launch_fin(s, w, kFinRho);
       if constexpr (!kWin) k_bi_fold<V><<<G, kRedThreads, 0, s>>>(n, w.row, w.x64, xs, st);
-      if constexpr (kWin) WIN_LAUNCH(k_win_true, n, o, w.x64, w.x64b, xs, w.r64, r, rh, w.partials, st);
+      if constexpr (kWin) WIN_LAUNCH(k_win_true, o, w.x64, w.x64b, xs, w.r64, r, rh, w.partials, st);
       else
         with_row_lanes(n, [&](auto gl) {
           constexpr int L = decltype(gl)::value;
@@ -2029,7 +2064,7 @@ __global__ void k_to_f64(int n, const float* __restrict__ a, double* __restrict_
 template <typename R>
 int ppe_matvec_probe(hipStream_t s, const DevParams& P, const SphView<R>& v, PpeWork& w, int variant, int reps,
                      const double* x64, double* y64, float2* pk, float* ms) {
-  if (!w.mixed || w.fmt != kFmtWin) {
+  if (!w.mixed || (w.fmt != kFmtWin && !w.thin)) {
     set_error("matvec probe: needs the mixed-precision operator with window slots");
     return SOPHIA_E_STATE;
   }
@@ -2055,7 +2090,12 @@ int ppe_matvec_probe(hipStream_t s, const DevParams& P, const SphView<R>& v, Ppe
   for (int k = 0; k <= reps; k++) {
     if (k == 1) HIP_TRY(hipEventRecord(e0, s));  // the first launch warms the caches, untimed
     if (variant == 1) k_mf_matvec<R><<<grid_xcd(n), kBlock, 0, s>>>(P, v, w.row, w.diag, pk, x, y);
-    else launch_win_mv(s, o, x, y, rh, WinCoarse{}, w, st);
+    else if (w.fmt == kFmtWin) launch_win_mv(s, o, x, y, rh, WinCoarse{}, w, st);
+    else
+      with_row_lanes(n, [&](auto gl) {
+        constexpr int L = decltype(gl)::value;
+        k_bi_mv<kFmtIdx32, 0, float, L><<<op_blocks(o), kRedThreads, 0, s>>>(o, x, y, rh, w.partials, st);
+      });
   }
   HIP_TRY(hipEventRecord(e1, s));
   HIP_TRY(hipEventSynchronize(e1));

@@ -21,8 +21,9 @@ namespace sophia {
 //              column is stored as a u8 offset from its run's first particle,
 //              and a u64 per row holds the 9 run lengths (7 bits each).  Needs
 //              every run <= 256 particles.
-//   kFmtIdx32: plain u32 column indices (Morton keys, overfull cells, and the
-//              FP64 path of periodic boxes).
+//   kFmtIdx32: plain u32 column indices (Morton keys, overfull cells, the FP64
+//              path of periodic boxes, and on the mixed path rows that lie
+//              thinly, rows_thin).
 enum { kFmtRun8 = 0, kFmtIdx32 = 1, kFmtWin = 2 };
 constexpr int kRunBits = 7;  // kFmtRun8: bits per run length in the row's u64
 constexpr int kRunMax = (1 << kRunBits) - 1;
@@ -71,6 +72,7 @@ __device__ inline uint32_t win_word(double a, int anchor, uint32_t off) {
 
 struct PpeOp {
   int n = 0, nq = 0, fmt = kFmtRun8;
+  int64_t nnz = 0;                     // stored entries
   int NI = 1, NJ = 1, NK = 1, ncell = 1, pmask = 0;
   const uint32_t* keys = nullptr;      // sorted cell key per particle
   const uint32_t* cell_off = nullptr;  // first particle of each cell (dense, num_cells + 1)
@@ -93,6 +95,7 @@ struct PpeWork {
   bool mixed = false;
   int fmt = kFmtRun8;
   int NI = 1, NJ = 1, NK = 1, ncell = 1, pmask = 0;
+  bool thin = false;     // mixed: the last system's rows lay too thinly for kFmtWin
   bool rowmajor = true;  // cell keys are row-major (not Morton)
   const uint32_t* keys = nullptr;
   const uint32_t* cell_off = nullptr;

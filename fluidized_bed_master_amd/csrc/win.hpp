@@ -234,11 +234,10 @@ __device__ __forceinline__ u32x4 ldq(const u32x4* p) {
 }
 
 // What a lane has in hand of its row before the tile is staged: the row's
-// first two quads travel while the block stages.  G = 1 (large operators,
-// streamed from HBM once per pass) loads past the caches, so that x stays in
-// L2: 83.3 -> 78.5 us at 1.16 M rows, 69.4 -> 64.4 us for the 10^6-row box;
-// an operator that fits the last-level cache is better left to it.  Two quads
-// in flight: one 92, three 90, four 96 us (registers spill at eight waves).
+// first two quads travel while the block stages.  G = 1 (operators streamed from
+// HBM, win_group) loads past the caches, so that x stays in L2: 83.3 -> 78.5 us at
+// 1.16 M rows, 69.4 -> 64.4 us for the 10^6-row box.  Two quads in flight: one 92,
+// three 90, four 96 us (registers spill at eight waves).
 constexpr int kWinQ = 2;
 template <int G>
 struct WinHead {
@@ -362,7 +361,16 @@ __device__ __forceinline__ double win_row_sum_full(const PpeOp& o, int i, const 
 // turn, which hides behind other waves only when there are many: at 4,200 /
 // 92,000 / 276,000 / 1,160,000 rows the inner product takes 14.7 / 15.3 / 27.2 /
 // 78.5 us with one lane, 8.2 / 10.5 / 22.7 / 86 with two and 7.1 / 11.2 / 26 / 110
-// with four (a tile has 256 / G rows, so more lanes stage more per row).
-inline int win_group(int n) { return n >= 500000 ? 1 : (n >= 40000 ? 2 : 4); }
+// with four (a tile has 256 / G rows, so more lanes stage more per row).  One lane
+// pays where the words come from HBM, past the 256 MB last-level cache (us per
+// BiCGStab iteration, one lane past the caches / two through them):
+//   columns, 494 k / 616 k / 806 k / 1.16 M particles  125 / 158 / 211 / 311 MB
+//                                      106 / 87, 127 / 102, 148 / 128, 196 / 203
+//   h = 1.0 dx, 616 k particles                58 MB   140 / 100
+//   h = 1.6 dx, 616 k and 1.16 M         277, 546 MB   199 / 174, 335 / 311
+//   boxes, 512 k / 729 k / 1 M      164 / 233 / 320 MB  96 / 94, 149 / 127, 161 / 189
+constexpr int64_t kWinStream = 290000000;  // bytes of words
+constexpr int kWinTwo = 40000;
+inline int win_group(int n, int64_t nnz) { return 4 * nnz > kWinStream ? 1 : (n >= kWinTwo ? 2 : 4); }
 
 }  // namespace sophia

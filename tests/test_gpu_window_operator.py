@@ -207,14 +207,39 @@ def _dense():
     return p, more
 
 
-@pytest.mark.parametrize("make", [_film, _wide, lambda: _wide(60, 62, 70), _spray, lambda: _spray(40, 0.3), _dense],
-                         ids=["film", "wide", "wide_2_lanes", "spray", "spray_of_groups", "dense"])
-def test_tiles_with_gaps_match_fp64_formats(make):
-    """Tiles planned around their rows' cells alone: the product, the inner product
-    and (two-level) the coarse operator beside the FP64 path's formats."""
+def _freeboard():
+    # walls three times the column's height: tiles of thin wall rings
+    return configs.isph_dem_column(40, 42, 30, 1.0e-3, jitter=0.02, seed=3, tank_extra=90)
+
+
+def _surface():
+    # the top layer half in one cell layer and half in the next: a third of its rows
+    # lie by ones and twos
+    return configs.isph_dem_column(120, 120, 5, 1.0e-3, jitter=0.45, seed=3, tank_extra=6)
+
+
+# (system, bytes per column index: 0 window slots, 4 where the rows lie thinly)
+GAPS = {
+    "film": (_film, 4),
+    "wide": (_wide, 0),
+    "wide_2_lanes": (lambda: _wide(60, 62, 70), 0),
+    "freeboard": (_freeboard, 0),
+    "surface": (_surface, 0),
+    "spray": (_spray, 4),
+    "spray_of_groups": (lambda: _spray(40, 0.3), 0),
+    "dense": (_dense, 0),
+}
+
+
+@pytest.mark.parametrize("name", GAPS)
+def test_tiles_with_gaps_match_fp64_formats(name):
+    """Tiles planned around their rows' cells alone, and the u32 columns of thin
+    systems: the product, the inner product and (two-level) the coarse operator
+    beside the FP64 path's formats; a second assembly gives the same bits."""
+    make, index_bytes = GAPS[name]
     p, parts = make()
     a, b = _assembled(p, parts, abi.PREC_MIXED), _assembled(p, parts, abi.PREC_FP64)
-    assert a.ppe_layout()["index_bytes"] == 0
+    assert a.ppe_layout()["index_bytes"] == index_bytes
     assert a.ppe_layout()["nnz"] == b.ppe_layout()["nnz"]
     d, _, rows = b.get_ppe_system()
     r = rows == 1
@@ -223,7 +248,13 @@ def test_tiles_with_gaps_match_fp64_formats(make):
     ref = b.ppe_apply(x)
     scale = np.maximum(2 * np.abs(d[r]), 1e-3 * np.abs(d[r]).max())
     assert (np.abs(a.ppe_apply(x) - ref)[r] / scale).max() <= 2.0 ** -18
-    assert (np.abs(a.matvec_probe(0, x, reps=1)[0] - ref)[r] / scale).max() <= 2.0 ** -16 + 2.0 ** -18
+    inner = a.matvec_probe(0, x, reps=1)[0]
+    assert (np.abs(inner - ref)[r] / scale).max() <= 2.0 ** -16 + 2.0 ** -18
+    full = a.ppe_apply(x)
+    a.ppe(abi.ppe_opts(method=abi.PPE_BICGSTAB, precision=abi.PPE_MIXED_IR, max_iter=1,
+                       zero_mean=1 if p.periodic_mask else 0))
+    assert a.ppe_layout()["index_bytes"] == index_bytes
+    assert np.array_equal(a.ppe_apply(x), full) and np.array_equal(a.matvec_probe(0, x, reps=1)[0], inner)
     if not p.periodic_mask:
         E = []
         for g, mixed in ((a, True), (b, False)):
@@ -231,7 +262,7 @@ def test_tiles_with_gaps_match_fp64_formats(make):
                                     guess=abi.GUESS_ZERO, precision=abi.PPE_MIXED_IR if mixed else abi.PPE_FP64))
             if st["precond_used"] == abi.PRECOND_TWO_LEVEL:
                 E.append(g.ppe_coarse()[1].astype(float))
-        assert len(E) == (0 if make is _spray else 2)  # lone drops: a singular coarse operator
+        assert len(E) == (0 if name == "spray" else 2)  # lone drops: a singular coarse operator
         # FP32 entries of sums of coefficients with relative errors of 2^-18
         if E:
             assert np.abs(E[0] - E[1]).max() <= 2.0 ** -17 * np.abs(E[1]).max()
