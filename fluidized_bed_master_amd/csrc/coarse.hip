@@ -143,14 +143,19 @@ __global__ __launch_bounds__(256) void k_coarse_rows(PpeOp o, AggGrid g, double*
 }
 
 // Pass 1 of the window format (kFmtWin): the tile's cells are staged in LDS as
-// in the matvec, each slot holding the parities of its cell's aggregate
-// coordinates.  Aggregates that couple differ by at most one per axis, so the
-// exclusive or with the row's own parities is the slot sum's index: one byte
-// from LDS per entry in place of a key gather and three divisions.
-__device__ inline uint8_t agg_parity(int x, int y, int z) {
-  return (uint8_t)(((x / kAgg) & 1) | (((y / kAgg) & 1) << 1) | (((z / kAgg) & 1) << 2));
+// in the matvec, each slot holding two bits per axis of its cell's aggregate
+// coordinates, which differ wherever two aggregates couple: one byte from LDS per
+// entry in place of a key gather and three divisions.  The bits are the parity and,
+// for the last of an odd number of aggregates, a mark in its place: across a
+// periodic wrap it meets the first, whose parity it shares.
+__device__ inline uint32_t agg_bits(int c, int n) {
+  const int a = c / kAgg;
+  return (n & 1) && n > 1 && a == n - 1 ? 8u : (uint32_t)(a & 1);
 }
-__global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, double* __restrict__ slots) {
+__device__ inline uint8_t agg_mark(int x, int y, int z, const AggGrid& g) {
+  return (uint8_t)(agg_bits(x, g.AX) | agg_bits(y, g.AY) << 1 | agg_bits(z, g.AZ) << 2);
+}
+__global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, AggGrid g, double* __restrict__ slots) {
   __shared__ WinStage<uint8_t> S;
   const int n = o.n;
   const int b = (gridDim.x & 7) ? (int)blockIdx.x : (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3));
@@ -158,8 +163,8 @@ __global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, double
   for (int s0 = i0; s0 < i1;) {
     int e0;
     const int m = win_stage(
-        o, s0, i1, S, &e0, [](int x, int y, int z, int) { return (int)agg_parity(x, y, z); },
-        [](int par, int, int) { return (uint8_t)par; });
+        o, s0, i1, S, &e0, [&](int x, int y, int z, int) { return (int)agg_mark(x, y, z, g); },
+        [](int mark, int, int) { return (uint8_t)mark; });
     const int i = s0 + (int)threadIdx.x, first = s0;
     s0 = m;
     if (i >= m) continue;
@@ -170,7 +175,7 @@ __global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, double
       const uint32_t key = o.keys[i];
       int cx, cy, cz;
       cell_xyz(key, o.NI, o.NJ, cx, cy, cz);
-      const uint8_t own = agg_parity(cx, cy, cz);
+      const uint8_t own = agg_mark(cx, cy, cz, g);
       const uint8_t* win = S.x + S.p.pre[win_first(o, S.p, e0, first, i, key)];
       acc[0] = o.diag[i];
       const int meta = o.ccnt[i];
@@ -187,7 +192,7 @@ __global__ __launch_bounds__(kWinThreads) void k_coarse_rows_win(PpeOp o, double
         l = lp[qn];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-          const int sl = (int)(win[c[u] & (uint32_t)kWinMax] ^ own);
+          const int d = (int)(win[c[u] & (uint32_t)kWinMax] ^ own), sl = (d | d >> 3) & 7;
           const double a = (double)win_val(c[u], anc) + (double)lv[u];  // 0 for padding entries
 #pragma unroll
           for (int t = 0; t < 8; t++) acc[t] -= sl == t ? a : 0.0;
@@ -501,7 +506,7 @@ static int coarse_rows(hipStream_t s, CoarseWork& c, const PpeWork& w) {
   const AggGrid g = agg_grid(c);
   const int gr = grid_xcd(w.n);
   if (w.fmt == kFmtWin) {
-    k_coarse_rows_win<<<gr, kWinThreads, 0, s>>>(o, c.slots);
+    k_coarse_rows_win<<<gr, kWinThreads, 0, s>>>(o, g, c.slots);
   } else if (w.fmt == kFmtRun8) {
     k_coarse_rows<kFmtRun8, 2><<<gr, 256, 0, s>>>(o, g, c.slots);
   } else {
