@@ -250,9 +250,5 @@ __device__ inline double nb_vol(const Nb<R>& q) { return q.m / q.rho; }
 template <typename R>
 __device__ inline double nb_vol(const NbP<R>& q) { return q.vol; }
 __device__ inline float nb_vol(const NbR& q) { return q.vol; }
-template <typename R>
-__device__ inline double nb_rho(const Nb<R>& q) { return q.rho; }
-template <typename R>
-__device__ inline double nb_rho(const NbP<R>& q) { return q.m / q.vol; }
 
 }  // namespace sophia

@@ -458,7 +458,7 @@ __global__ __launch_bounds__(kBlock) void k_advection(DevParams P, SphView<R> v)
   // u_i . (Cm g) = (Cm u_i) . g
   double wx = (double)uxi, wy = (double)uyi, wz = (double)uzi;
   K.apply(wx, wy, wz);
-  T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0, ax = 0, ay = 0, az = 0;
+  T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0;
   double px = 0, py = 0, pz = 0, fl = 0;
   auto term = [&](const auto& q, bool on) {
     const bool use = on && q.pt < 1000;
@@ -505,12 +505,14 @@ __global__ __launch_bounds__(kBlock) void k_advection(DevParams P, SphView<R> v)
       T phi = hij * uij_xij;
       phi /= (r * r + (T)0.01 * hij * hij);
       T Pij = mi * phi * ((T)(-0.1 * P.soundspeed) + (T)0.02 * phi);
-      Pij /= (rhoi + (T)nb_rho(q));
+      Pij /= (rhoi + (T)v.rho[q.j]);  // not m / V: there may be no mass
       Pij *= (T)0.5;
-      const T c = use && uij_xij < 0 ? -Pij * (T)sd : (T)0;
-      ax += c * dx;
-      ay += c * dy;
-      az += c * dz;
+      double gx = dxd, gy = dyd, gz = dzd;  // Cm x
+      K.apply(gx, gy, gz);
+      const T c = use && uij_xij < 0 ? -Pij : (T)0;
+      tx += c * (T)(sd * gx);
+      ty += c * (T)(sd * gy);
+      tz += c * (T)(sd * gz);
     }
     if (euler) {
       const T ug = (T)(sd * (wx * dxd + wy * dyd + wz * dzd)) * Vj * (1 - eli);
@@ -548,19 +550,8 @@ __global__ __launch_bounds__(kBlock) void k_advection(DevParams P, SphView<R> v)
   py = group_sum<G>(py);
   pz = group_sum<G>(pz);
   fl = group_sum<G>(fl);
-  if (P.fva_solve) {
-    ax = group_sum<G>(ax);
-    ay = group_sum<G>(ay);
-    az = group_sum<G>(az);
-  }
   if (G > 1 && pair_sub<G>() != 0) return;
   K.apply(px, py, pz);
-  if (P.fva_solve) {
-    Kgc<T>(P.kgc == 1, v.cm, n, i).apply(ax, ay, az);
-    tx += ax;
-    ty += ay;
-    tz += az;
-  }
   if (P.fg_solve) tz += -(T)P.gravity;
   v.fx[i] = tx - ex;
   v.fy[i] = ty - ey;

@@ -251,7 +251,7 @@ __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<
   const Kgc<double> K(P.kgc == 1, v.cm, n, i);
   double wx = (double)uxi, wy = (double)uyi, wz = (double)uzi;  // u_i . (Cm g) = (Cm u_i) . g
   K.apply(wx, wy, wz);
-  T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0, ax = 0, ay = 0, az = 0;
+  T tx = 0, ty = 0, tz = 0, Rc = 0, ex = 0, ey = 0, ez = 0, et = 0;
   double px = 0, py = 0, pz = 0;  // sum_j V_j pp grad W
   for_nbrs4_pk<true, G>(v, i, true, [&](const NbP<R>& q, bool on) {
     const bool use = on && q.pt <= 1000;
@@ -285,12 +285,14 @@ __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<
       T phi = hij * uij_xij;
       phi /= (r * r + (T)0.01 * hij * hij);
       T Pij = mi * phi * ((T)(-0.1 * P.soundspeed) + (T)0.02 * phi);
-      Pij /= (rhoi + (T)nb_rho(q));
+      Pij /= (rhoi + (T)v.rho[q.j]);  // not m / V: there may be no mass
       Pij *= (T)0.5;
-      const T c = use && uij_xij < 0 ? -Pij * (T)sd : (T)0;
-      ax += c * dx;
-      ay += c * dy;
-      az += c * dz;
+      double gx = dxd, gy = dyd, gz = dzd;  // Cm x
+      K.apply(gx, gy, gz);
+      const T c = use && uij_xij < 0 ? -Pij : (T)0;
+      tx += c * (T)(sd * gx);
+      ty += c * (T)(sd * gy);
+      tz += c * (T)(sd * gz);
     }
     if (P.con_solve) {
       const int ptj = q.pt;
@@ -318,18 +320,12 @@ __global__ __launch_bounds__(kBlock) void k_wc_interaction(DevParams P, SphView<
   px = group_sum<G>(px);
   py = group_sum<G>(py);
   pz = group_sum<G>(pz);
-  if (P.fva_solve) {
-    ax = group_sum<G>(ax);
-    ay = group_sum<G>(ay);
-    az = group_sum<G>(az);
-    Kgc<T>(P.kgc == 1, v.cm, n, i).apply(ax, ay, az);
-  }
   if (G > 1 && pair_sub<G>() != 0) return;
   K.apply(px, py, pz);
   // pressure -eps_i / rho_i V_j pp, then the other terms; FP32 rounding of the
   // sum of both is below the tests' tolerance
   const double ci = -porid / rhoid;
-  double fx = ci * px + (double)(tx + ax), fy = ci * py + (double)(ty + ay), fz = ci * pz + (double)(tz + az);
+  double fx = ci * px + (double)tx, fy = ci * py + (double)ty, fz = ci * pz + (double)tz;
   if (P.fg_solve) fz += -P.gravity;
   v.fx[i] = (R)(fx - (double)ex);
   v.fy[i] = (R)(fy - (double)ey);
