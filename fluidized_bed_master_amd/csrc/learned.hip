@@ -36,9 +36,9 @@
 // and accumulates weight gradients with v_mfma_f32_16x16x16_bf16, whose A
 // and B operands are exactly the FP32 result layout above (K = the 16 edges
 // of a tile), so dW2 += dZ2^T H1 and dW1 += dZ1^T E need no re-layout.
-// dH1 = dZ2 W2 goes through a second LDS tile.  Each persistent block
-// writes its partial gradient; a second kernel sums the partials in a fixed
-// order (deterministic), then Adam updates the FP32 master copy and the
+// dH1 = dZ2 W2 goes through a second LDS tile.  Each block adds its waves'
+// FP32 accumulators in FP64 and writes that partial gradient; a second kernel sums
+// the partials in a fixed order (deterministic), then Adam updates the FP32 master copy and the
 // BF16 copy is refreshed.
 #include "learned.hpp"
 
@@ -452,7 +452,7 @@ template <typename R>
 __global__ __launch_bounds__(64 * kBwdWaves, 2) void k_mlp_backward(Net net, SphView<R> v, const float2* __restrict__ nf,
                                                       const int* __restrict__ row, const double* __restrict__ pprev,
                                                       const double* __restrict__ target, double inv_scale,
-                                                      float inv_rows, float* __restrict__ partials) {
+                                                      float inv_rows, double* __restrict__ partials) {
   struct Work {
     W2Frags F;
     EdgeList E[kBwdWaves];
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(64 * kBwdWaves, 2) void k_mlp_backward(Net net, Sph
   };
   __shared__ union {
     Work w;
-    float grad[kNParam + 1];  // the block's partial gradient, after the loop
+    double grad[kNParam + 1];  // the block's partial gradient, after the loop
   } sh;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nl = lane & 15, er = 4 * (lane >> 4), kq = 8 * (lane >> 4);
@@ -654,14 +654,14 @@ __global__ __launch_bounds__(64 * kBwdWaves, 2) void k_mlp_backward(Net net, Sph
       }
     }
   }
-  // the block's partial gradient: the waves add theirs in turn
+  // the block's partial gradient: the waves add theirs in turn, in FP64
   __syncthreads();
-  for (int q = threadIdx.x; q <= kNParam; q += 64 * kBwdWaves) sh.grad[q] = 0.f;
+  for (int q = threadIdx.x; q <= kNParam; q += 64 * kBwdWaves) sh.grad[q] = 0.0;
   for (int w = 0; w < kBwdWaves; w++) {
     __syncthreads();
     if (wave == w) {
-      float* P = sh.grad;
-      auto put = [&](int q, float a) { P[q] += a; };
+      double* P = sh.grad;
+      auto put = [&](int q, double a) { P[q] += a; };
 #pragma unroll
       for (int nb = 0; nb < 4; nb++)
 #pragma unroll
@@ -673,7 +673,7 @@ __global__ __launch_bounds__(64 * kBwdWaves, 2) void k_mlp_backward(Net net, Sph
         }
 #pragma unroll
       for (int nb = 0; nb < 4; nb++) {
-        float a = gb1[nb], b = gb2[nb];
+        double a = gb1[nb], b = gb2[nb];
         a += __shfl_xor(a, 16);
         a += __shfl_xor(a, 32);
         b += __shfl_xor(b, 16);
@@ -694,16 +694,16 @@ __global__ __launch_bounds__(64 * kBwdWaves, 2) void k_mlp_backward(Net net, Sph
     }
   }
   __syncthreads();
-  float* P = partials + (size_t)blockIdx.x * (kNParam + 1);
+  double* P = partials + (size_t)blockIdx.x * (kNParam + 1);
   for (int q = threadIdx.x; q <= kNParam; q += 64 * kBwdWaves) P[q] = sh.grad[q];
 }
 
 // Sum of the blocks' partial gradients in FP64, in a fixed order: 64 parameters
 // per block by 16 slices of the partials, so that they are read by 139
 // blocks of 16 waves (one thread per parameter walking 1024 partials of 35 KB took
-// 260 us, 139 waves with one load in flight each; now 6 us for 512).
+// 260 us, 139 waves with one load in flight each; now 15 us for 1024 of 71 KB).
 constexpr int kRedSlices = 16;
-__global__ __launch_bounds__(64 * kRedSlices) void k_reduce_partials(const float* __restrict__ partials, int nblocks,
+__global__ __launch_bounds__(64 * kRedSlices) void k_reduce_partials(const double* __restrict__ partials, int nblocks,
                                                                      float* __restrict__ grad,
                                                                      double* __restrict__ loss) {
   __shared__ double part[kRedSlices][64];
@@ -808,7 +808,7 @@ int mlp_alloc(Mlp& m, int n, int cap) {
     HIP_TRY(hipMalloc(&m.adam_m, kNParam * 4));
     HIP_TRY(hipMalloc(&m.adam_v, kNParam * 4));
     HIP_TRY(hipMalloc(&m.wbf, kNParam * 2));
-    HIP_TRY(hipMalloc(&m.partials, (size_t)kMlpBwdBlocks * (kNParam + 1) * 4));
+    HIP_TRY(hipMalloc(&m.partials, (size_t)kMlpBwdBlocks * (kNParam + 1) * 8));
     HIP_TRY(hipMalloc(&m.scal, 8 * 8));
     HIP_TRY(hipMalloc(&m.fpart, kFeatBlocks * 3 * 8));
     HIP_TRY(hipHostMalloc((void**)&m.host_scal, 8 * 8, hipHostMallocDefault));
@@ -924,7 +924,8 @@ int mlp_backward(hipStream_t s, const DevParams& P, const SphView<R>& v, Mlp& m,
   }
   if (v.n <= 0 || n_rows <= 0) return 0;
   Net net{m.wbf, m.master};
-  const int g = kMlpBwdBlocks;
+  // no more blocks than have particles; a multiple of 8, for the XCDs
+  const int g = std::min(kMlpBwdBlocks, ((v.n + kBwdWaves - 1) / kBwdWaves + 7) / 8 * 8);
   const double inv_scale = scale != 0 ? 1.0 / scale : 0.0;
   k_mlp_backward<R><<<g, 64 * kBwdWaves, 0, s>>>(net, v, m.nf, row, pprev, target, inv_scale, 1.0f / (float)n_rows,
                                      m.partials);

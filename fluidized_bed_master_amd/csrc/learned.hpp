@@ -18,7 +18,9 @@ constexpr int OFF_B3 = OFF_W3 + kH * kH;     // 64
 constexpr int OFF_W4 = OFF_B3 + kH;          // 64
 constexpr int OFF_B4 = OFF_W4 + kH;          // 1
 constexpr int kNParam = OFF_B4 + 1;          // 8833
-constexpr int kMlpBwdBlocks = 512;            // persistent blocks of the backward pass, two per CU
+// Blocks of the backward pass, two per CU at a time: as many again, so that an FP32
+// accumulator takes up at most n / 1024 particles (dW3; the others a quarter).
+constexpr int kMlpBwdBlocks = 1024;
 
 struct Mlp {
   bool ready = false;      // parameters set
@@ -34,7 +36,7 @@ struct Mlp {
   double* guess = nullptr;   // predicted pressure (FP64, sorted order)
   double* target = nullptr;  // training target (FP64, sorted order)
   double* pprev = nullptr;   // pressure before the solve (FP64, sorted order)
-  float* partials = nullptr; // per-block gradient partials (kMlpBwdBlocks x (kNParam + 1))
+  double* partials = nullptr;  // per-block gradient partials (kMlpBwdBlocks x (kNParam + 1))
   double* scal = nullptr;    // device scalars: sum r^2, sum diag, rows, scale, loss
   double* fpart = nullptr;   // per-block partials of the feature sums
   double* host_scal = nullptr;
