@@ -30,7 +30,8 @@
 //     waves per SIMD (0.85 ms);
 //   - the XCDs take runs of particles by turns (0.79 ms).
 // Per-particle counts instead of sums for db2 and selects of a rounded dZ2 took
-// instructions out but no time.
+// instructions out but no time.  Half as many blocks, with dW3 written out halfway
+// through in place of shorter sums, spilled: 0.87 ms.
 //
 // Backward recomputes the forward per particle (two passes over its edges)
 // and accumulates weight gradients with v_mfma_f32_16x16x16_bf16, whose A
@@ -350,9 +351,8 @@ __global__ __launch_bounds__(64 * kFwdWaves, 4) void k_mlp_forward(Net net, SphV
       const uint32_t ent = nxt;
       const int kn = k0 + 4 + g4;
       if (k0 + 4 < maxc) nxt = kn < cnt ? v.nbr[nbr_slot(kn, i, v.n)] : kNbrFlag;
-      // an edge outside the list gets all-zero inputs, bias inputs
-      // included, so its layer-1 and layer-2 sums are exactly 0 and it adds
-      // nothing to the message
+      // an edge outside the list gets all-zero inputs, bias inputs included, so
+      // its h1 is exactly 0 and it adds ReLU(b2), taken off after the last slot
       bf8 e8;
 #pragma unroll
       for (int q = 0; q < 8; q++) e8[q] = (__bf16)0.0f;

@@ -54,12 +54,14 @@ __device__ inline int pair_particle() { return particle_index() / G; }
 template <int G>
 __device__ inline int pair_sub() { return (int)threadIdx.x & (G - 1); }
 
-// Measured with 1 / 2 / 4 / 8 lanes (us): advection 72 / 41 / 27 / 17 at 4,200
-// particles, 116 / 121 / 124 / 119 at 56,000 (FP64), 112 / 112 / 111 / 115 at 118,000,
-// 292 / 265 / 278 / 304 at 281,000, 1139 / 1112 / 1209 / 1362 at 1.16 M; prep 52 / 29 /
-// 18 / 11, 84 / 62 / 61 / 62, 64 / 48 / 52 / 50, 128 / 112 / 118 / 121 and 605 / 506 / 499 /
-// 523: past 90,000 particles two lanes are the better half of the gathers in
-// flight per wave, below there are too few waves and more lanes win.
+// One rule for all of them, by the whole step (us, with 1 / 2 / 4 / 8 lanes), since
+// the kernels of a step differ by a few per cent either way: ISPH with one Jacobi
+// sweep, mixed, 627 / 478 / 432 / 410 at 5,200 particles, 718 / 619 / 590 / 587 at 37,000,
+// 782 / 643 / 642 / 636 at 51,000, 833 / 704 / 697 / 716 at 70,000, 860 / 778 / 780 / 791 at
+// 92,000, 1492 / 1342 / 1412 / 1566 at 276,000, 4937 / 4647 / 4562 / 4767 at 1.16 M; FP64
+// 871 / 766 / 734 / 731 at 51,000, 1115 / 852 / 814 / 834 at 70,000, 1179 / 989 / 938 / 949
+// at 92,000, 2179 / 1890 / 1930 / 2109 at 276,000.  WCSPH and the 2D step lie the same
+// way; the rule is within 2 % of the best but at 92,000 in FP64 (5 %).
 inline int pair_lanes(int n) { return n >= 90000 ? 2 : (n >= 40000 ? 4 : 8); }
 
 // f(lanes as an integral constant, grid) for n particles
@@ -159,7 +161,7 @@ __device__ inline void for_nbrs4_pk(const SphView<R>& v, int i, bool eps_rule, F
       q[u].dz = pi.z - a.z;
       q[u].m = a.w;
       if constexpr (VEL && std::is_same<R, float>::value) {
-        // mixed path: two more records, {rho, p, u, T} and {S, h, p_type}
+        // mixed path: two more records, {V, p, u, T} and {S, h, p_type}
         const PkB b = v.pkb[j];
         const PkC c = v.pkc[j];
         q[u].vol = b.vol; q[u].pres = b.p;

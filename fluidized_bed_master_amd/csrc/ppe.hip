@@ -959,7 +959,7 @@ __global__ __launch_bounds__(kRedThreads) void k_bi_mv(PpeOp o, const V* __restr
 // those ranges of x into LDS with coalesced loads (about 11 values per row on
 // a 1 mm column, against ~65 gathered entries per row) and its rows gather
 // from LDS.  A tile whose ranges do not fit takes the global gathers.
-constexpr int kStageCap = 4864;  // values: 19 KB (FP32) / 38 KB (FP64) per block
+constexpr int kStageCap = 4864;  // values: 38 KB per block
 
 template <typename XT>
 struct Stage {
@@ -2015,7 +2015,7 @@ int ppe_solve(hipStream_t s, PpeWork& w, double* pres, const sophia_ppe_opts& o,
 // / rho_i), c_ij = -(x_ij . Cm_i grad W_ij) / r_ij^2, recomputed per launch
 // in FP32 from the neighbour list, the position records and one float2 per
 // column (V_j, m_j eps_j; zero for non-row columns).  Probe only: it reads
-// the 4-byte neighbour list where the stored operator reads 5 bytes per
+// the 4-byte neighbour list where the stored operator reads a 4-byte word per
 // entry, and adds the kernel gradient per pair.
 template <typename R>
 __global__ void k_mf_pack(int n, const SphView<R> v, const int* row, float2* pk) {
