@@ -274,17 +274,21 @@ def test_tiles_with_gaps_match_fp64_formats(name):
     b.close()
 
 
-def test_wall_cells_and_gaps_cost_no_tiles():
-    """A pass over the film takes no longer than one over a full column of as many
-    particles, which has four times its entries (0.8 of it; 3.9 times where every
-    wall cell and gap has a tile of its own)."""
+@pytest.mark.parametrize("gaps,full,index_bytes,most", [
+    (_wide, lambda: configs.isph_dem_column(40, 40, 40, 1.0e-3, jitter=0.02, seed=3), 0, 1.7),
+    (_film, configs.c4_train, 4, 2.0)], ids=["wide", "film"])
+def test_wall_cells_and_gaps_cost_no_tiles(gaps, full, index_bytes, most):
+    """A pass over the wide domain takes little longer than one over its column alone
+    (1.1 of it; 2.7 where every gap halves its tile until the planes fit), and one over
+    the film no longer than over a full column of as many particles (0.8; 3.9)."""
     us = []
-    for p, parts in (_film(), configs.c4_train()):
+    for k, (p, parts) in enumerate((gaps(), full())):
         g = _assembled(p, parts, abi.PREC_MIXED)
+        assert g.ppe_layout()["index_bytes"] == (index_bytes if k == 0 else 0)
         x = np.ones(len(g.get_ppe_system()[2]))
         us.append(min(g.matvec_probe(0, x, reps=50)[1] for _ in range(5)))
         g.close()
-    assert us[0] <= 2 * us[1], us
+    assert us[0] <= most * us[1], us
 
 
 @pytest.mark.parametrize("n", [17, 26, 40], ids=["even", "odd", "odd_drifted"])
