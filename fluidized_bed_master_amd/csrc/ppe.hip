@@ -1578,7 +1578,9 @@ int cell_offsets(hipStream_t s, int n, const uint32_t* keys, int num_cells, uint
 // Lanes per row of the assembly: as the pair kernels, but one for large
 // operators, whose whole-quad stores beat the lanes' single ones (1 / 2 / 4 / 8
 // lanes: 99 / 59 / 34 / 23 us at 4,200 particles, 147 / 134 / 142 / 161 at 118,000,
-// 330 / 294 / 329 / 392 at 281,000, 1220 / 1298 / 1433 / 1751 at 1.16 M).
+// 330 / 294 / 329 / 392 at 281,000, 1220 / 1298 / 1433 / 1751 at 1.16 M; whole steps
+// with 1 / 2: 1370 / 1338 at 276,000, 2070 / 2048 at 458,000, 2314 / 2367 at 533,000,
+// 2999 / 3044 at 707,000).
 inline int asm_lanes(int n) { return n >= 500000 ? 1 : pair_lanes(n); }
 
 // Whether a system's rows lie too thinly for the window format: where the tiles of

@@ -1037,7 +1037,8 @@ int sph_kgc_porosity(hipStream_t s, const DevParams& P, const SphView<R>& v, con
     if (v.n <= 0) return 0;
     TRY(pack_r32(s, v, false, false));
     // one lane for large runs: the spheres around a particle are few, and lanes
-    // that share them idle (914 us with one, 1010 with two at 1.16 M)
+    // that share them idle (914 us with one, 1010 with two at 1.16 M; whole steps
+    // 1352 / 1333 at 276,000, 2040 / 2046 at 458,000, 2645 / 2653 at 616,000)
     return pair_launch(v.n, v.n >= 500000 ? 1 : pair_lanes(v.n), [&](auto g, int grid) {
       constexpr int G = decltype(g)::value;
       if (kgc) k_kgc_porosity<true, G><<<grid, kBlock, 0, s>>>(P, v, d, dc);
