@@ -633,10 +633,11 @@ __host__ __device__ inline T knl_dw_ih(int kt, T tA, T tH, T ih, T rr) {
 // rounding), 6 and 10 operations in place of the correctly rounded square root
 // and division (about 20 and 45); within an ulp or two of them.  With V from
 // the records and the correction on the sums the stages' errors are no larger for
-// it: against 80-bit sums (columns, box; Wendland C2) Shepard sum 4.4e-16 -> 1.5e-16,
-// PPE diagonal 2.9e-16 -> 1.7e-16, pressure force 4.7e-16 -> 3.8e-16, KGC inverse
-// 3.2e-16 -> 3.3e-16 in FP64; 1.67e-7 -> 0.99e-7 and 1.55e-7 -> 0.95e-7 (KGC) in FP32,
-// where r rounded once more changes nothing (0.99e-7, 0.96e-7).  The offset,
+// it (the porosity's would be: knl_w_por): against 80-bit sums (columns, box;
+// Wendland C2) Shepard sum 4.4e-16 -> 1.5e-16, PPE diagonal 2.9e-16 -> 1.7e-16,
+// pressure force 4.7e-16 -> 3.8e-16, KGC inverse 3.2e-16 -> 3.3e-16 in FP64;
+// 1.67e-7 -> 0.99e-7 and 1.55e-7 -> 0.95e-7 (KGC) in FP32, where r rounded once more
+// changes nothing in these (0.99e-7, 0.96e-7).  The offset,
 // far below any pair's d2, keeps the self pair (d2 = 0) finite: its r is 0 and
 // its 1 / r at most 1e15 (FP32) or 1e20.
 __device__ inline float pair_rinv(float d2) {
@@ -649,6 +650,24 @@ __device__ inline double pair_rinv(double d2) {
   const double y = __builtin_amdgcn_rsq(d2);
   const double e = fma(-d2 * y, y, 1.0);
   return fma(fma(0.375, e, 0.5), y * e, y);
+}
+
+// The kernel of the porosity sums from d2 and 1 / r: r and r / h rounded once each (a
+// Newton step), where the products d2 / r and r (1 / h) are one and a half ulp off.
+// 1 - eps is small and the drag and the density take differences of it, so that two
+// ulps of q = r / 2h, magnified by 4 / (1 - q), show: with the products the density
+// of a WCSPH step with spheres is 1.35e-7 from FP64, the ISPH pressure force
+// 2.39e-7; so 1.07e-7 and 2.01e-7 (a correctly rounded root and division: 1.14e-7 and
+// 2.54e-7).  The other sums do not move with it, nor does the time: 4650 -> 4632 us
+// an ISPH step at 1.16 M particles, 2511 -> 2514 a WCSPH step at 859,000.
+template <typename T>
+__device__ inline T knl_w_por(int kt, T tA, T tH, T ih, T d2, T ir) {
+  T r = d2 * ir;
+  r = fma(fma(-r, r, d2), (T)0.5 * ir, r);
+  if (kt != SOPHIA_KNL_WENDLAND2) return knl_w<T>(kt, tA, tH, r);
+  const T q = r * ih, tR = fma(fma(-q, tH, r), ih, q) * (T)0.5;
+  const T o = 1 - tR;
+  return tR < 1 ? tA * o * o * o * o * (1 + 4 * tR) : (T)0;
 }
 
 // The symmetric KGC inverse of one particle (identity without the correction).

@@ -146,7 +146,7 @@ __global__ __launch_bounds__(kBlock) void k_porosity_sph(DevParams P, SphView<R>
   auto term = [&](const auto& q, bool on) {
     T dx = (T)q.dx, dy = (T)q.dy, dz = (T)q.dz;
     const T d2 = dx * dx + dy * dy + dz * dz;
-    const T w = knl_w_ih<T>(P.kernel_type, A, h, ih, d2 * pair_rinv(d2));
+    const T w = knl_w_por<T>(P.kernel_type, A, h, ih, d2, pair_rinv(d2));
     const bool use = on && pti <= 1000 && q.pt == 1;
     flt += use ? (T)nb_vol(q) * w : (T)0;
   };
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kBlock) void k_kgc_porosity(DevParams P, SphView<fl
       yz += ky * dz;
       zz += k * dz * dz;
     }
-    const T w = knl_w_ih<T>(P.kernel_type, A, h, ih, r);
+    const T w = knl_w_por<T>(P.kernel_type, A, h, ih, d2, ir);
     const bool usep = on && !q.flag && pti <= 1000 && q.pt == 1;
     flt += usep ? q.vol * w : (T)0;
   });

@@ -181,3 +181,30 @@ def test_neighbours_without_mass_keep_their_density(prec):
     compare_fields(a1, b1, ["ux", "uy", "uz"], TOL[prec], "massless walls", mask=f)
     compare_fields(a3, b3, ["ftotalx", "ftotaly", "ftotalz"], TOL[prec], "massless walls/p3", mask=f)
     g.close()
+
+
+@pytest.mark.parametrize("solver,field,most", [("wcsph", "rho", 1.2e-7), ("isph", "fpx", 2.2e-7)])
+def test_porosity_sums_round_their_distances_once(solver, field, most):
+    """Mixed path, mean over eight inputs of the 2-norm distance from the oracle: what
+    the FP32 porosity sums leave in the density of a WCSPH step with spheres and in the
+    ISPH pressure force.  1.07e-7 and 2.0e-7 with r and r / h rounded once, 1.35e-7 and
+    2.4e-7 with both as products (1.5 ulp each); the bounds lie between."""
+    from fluidized_bed_master_amd.sophia import Sophia
+    from oracle.oracle import Oracle
+    err = []
+    for seed in range(8):
+        if solver == "wcsph":
+            p, parts = configs.wcsph_dem_column(14, 13, 18, con=1, seed=seed + 2, jitter=0.05)
+        else:
+            p, parts = configs.isph_dem_column(16, 17, 15, 1.0e-3, d_dem=2.0e-3, dem_height=6e-3, phi=0.6, jitter=0.05,
+                                               seed=seed + 8, u_noise=0.05, dem_u_noise=0.05)
+            configs.heated(p, parts)
+        g, o = Sophia(p, parts, precision=abi.PREC_MIXED), Oracle(p, parts)
+        opts = abi.ppe_opts(method=abi.PPE_JACOBI) if solver == "isph" else None
+        g.step(opts)
+        o.step(opts)
+        k = 0 if field == "rho" else 2
+        a, b = g.get_particles(abi.SPH)[k][field], o.get_particles(abi.SPH)[k][field]
+        err.append(np.linalg.norm(a - b) / np.linalg.norm(b))
+        g.close()
+    assert np.mean(err) <= most, err
